@@ -103,47 +103,63 @@ int solve_plan(const DeviceBatch& d, const gpsat_solve_opts& o, int32_t n_jobs, 
     a.o.deadline_ticks = o.deadline_ms > 0 ? (int64_t)(o.deadline_ms * clock_khz) : 0;
     a.o.inst_conflicts = o.inst_conflicts;
     a.o.telemetry = o.telemetry ? 1 : 0;
-    a.max_n = d.max_n;
     a.all3 = d.all3 ? 1 : 0;
-    a.wo_cap = max_L;
-    a.wl_cap = 2 * d.max_n * a.o.watch_slack;
-    a.wpair_cap = 2 * (d.max_m + o.learnt_cap);
-    a.lmeta_cap = 5 * o.learnt_cap;   // 4 metadata ints + 1 remap slot per clause
-    const int64_t clause_ints = (int64_t)a.wo_cap + a.wl_cap + a.wpair_cap + a.lmeta_cap + a.o.larena_cap;
-    const size_t state_b = solve_state_lds_bytes(d.max_n);
-    const size_t lds_all = state_b + 4 * (size_t)((clause_ints + 63) & ~(int64_t)63);
-
     hipDeviceProp_t prop;
     hipError_t e = device_props(d.device, prop);
     if (e != hipSuccess) return hip_fail("hipGetDeviceProperties", e);
     p.cus = prop.multiProcessorCount;
     const size_t lds_cu = prop.maxSharedMemoryPerMultiProcessor ? prop.maxSharedMemoryPerMultiProcessor : 65536;
     const size_t lds_block_max = prop.sharedMemPerBlock ? prop.sharedMemPerBlock : 65536;
-    const size_t lds_hyb = state_b + 4 * (size_t)(a.wo_cap + a.wpair_cap - 2 * o.learnt_cap);
+    const bool ids16 = o.clause_mem != 4 && solve_ids16(d.max_n, d.max_m, max_L, a.o);
+    a.lay = solve_layout(d.max_n, d.max_m, max_L, d.all3 && ids16, ids16 ? 2 : 4, a.o);
+    const size_t state_b = (size_t)a.lay.state_bytes;
+    const size_t lds_hyb = state_b + (size_t)a.lay.watch_bytes, lds_all = lds_hyb + (size_t)a.lay.arena_bytes;
     int mode;
-    if (state_b > lds_block_max) mode = 4;   // per-var state alone exceeds the LDS: all in HBM
+    if (state_b > lds_block_max || o.clause_mem == 4) mode = 4;   // all in HBM
+    else if (!ids16) mode = 2;
     else if (o.clause_mem == 1) mode = lds_all <= lds_block_max ? 1 : 2;
     else if (o.clause_mem == 2) mode = 2;
     else if (o.clause_mem == 3) mode = lds_hyb <= lds_block_max ? 3 : 2;
-    else if (o.clause_mem == 4) mode = 4;
     else {
-        // automatic: with few jobs the grid cannot fill the GPU and each job's latency is
-        // what counts, so the clause part goes to LDS as far as it fits; with many, LDS only
-        // while it leaves room for enough resident wavefronts
-        const bool few_jobs = n_jobs <= 4 * prop.multiProcessorCount;
-        if (lds_all <= (few_jobs ? lds_block_max : std::min<size_t>(48 * 1024, lds_block_max))) mode = 1;
+        // automatic: the placement with the least estimated run time, in units of a mean job on an
+        // otherwise idle GPU: a wavefront's share of the jobs at the speed of that placement, plus
+        // the longest jobs the run ends on (3-4 mean jobs on random 3-SAT).  The clause part in LDS
+        // is fastest per job but leaves few wavefronts room; the split placement is 7% slower per
+        // job; with the clause part in HBM a job takes 1.2 times as long alone and twice as long
+        // with 32 wavefronts on the CU.  Measured against all three (random 3-SAT at 4.26, ms for
+        // LDS / split / HBM): 20,000 x n=50 12.3 / 6.6 / 6.6, 8,000 x n=64 14.6 / 7.7 / 8.5,
+        // 12,000 x n=75 39 / 19 / 16, 6,000 x n=100 68 / 43 / 44, 3,000 x n=120 130 / 102 / 114.
+        const auto estimate = [&](int md, size_t lds, double pace, double crowd, double tail) {
+            const size_t most = 4 * (size_t)solve_waves_per_eu(md);
+            const double per_cu = (double)std::max<size_t>(1, std::min<size_t>(most, lds_cu / std::max<size_t>(lds, 1)));
+            const double w = std::min(per_cu * p.cus, (double)std::max(n_jobs, 1));
+            return (pace + crowd * w / (most * (double)p.cus)) * std::max(n_jobs, 1) / w + tail;
+        };
+        double best = estimate(2, state_b, 1.2, 0.85, 4.2);
+        mode = 2;
+        // with few jobs the longest one decides: the fastest placement that fits (580 colourings
+        // and pigeonhole formulas: 402 ms in LDS, 465 in HBM)
+        const bool few_jobs = n_jobs <= 4 * p.cus;
+        if (few_jobs && lds_all <= lds_block_max) mode = 1;
         else if (few_jobs && lds_hyb <= lds_block_max) mode = 3;
-        else mode = 2;
+        else if (lds_hyb <= lds_block_max && estimate(3, lds_hyb, 1.07, 0.0, 3.4) < best) {
+            best = estimate(3, lds_hyb, 1.07, 0.0, 3.4);
+            mode = 3;
+        }
+        if (!few_jobs && lds_all <= lds_block_max && estimate(1, lds_all, 1.0, 0.0, 3.2) < best) mode = 1;
     }
-    const int64_t slice_ints = clause_ints + (mode == 4 ? (int64_t)state_b / 4 : 0);
-    a.ws_ints_per_wave = (slice_ints + 63) & ~(int64_t)63;
+    if (mode == 4) a.lay = solve_layout(d.max_n, d.max_m, max_L, false, 4, a.o);
+    const int64_t slice = a.lay.arena_bytes + (mode == 2 || mode == 4 ? a.lay.watch_bytes : 0) +
+                          (mode == 4 ? a.lay.state_bytes : 0);
+    a.ws_ints_per_wave = (slice / 4 + 63) & ~(int64_t)63;
     p.mode = mode;
     p.lds_bytes = mode == 1 ? lds_all : mode == 3 ? lds_hyb : mode == 4 ? 0 : state_b;
     a.lds_per_wave = (int64_t)p.lds_bytes;
     int waves = o.waves;
     if (waves <= 0) {
-        const size_t per_cu_lds = p.lds_bytes ? lds_cu / p.lds_bytes : (size_t)4 * kSolveWavesPerEu;
-        const int per_cu = (int)std::max<size_t>(1, std::min<size_t>(4 * kSolveWavesPerEu, per_cu_lds));
+        const size_t most = 4 * (size_t)solve_waves_per_eu(mode);
+        const size_t per_cu_lds = p.lds_bytes ? lds_cu / p.lds_bytes : most;
+        const int per_cu = (int)std::max<size_t>(1, std::min<size_t>(most, per_cu_lds));
         waves = prop.multiProcessorCount * per_cu;
     }
     p.wpb = solve_waves_per_block(p.lds_bytes);

@@ -127,7 +127,8 @@ __device__ __forceinline__ uint32_t shfl_xor32(uint32_t x)
     return (uint32_t)__builtin_amdgcn_ds_bpermute(((l ^ 32) << 2), (int)x);
 }
 
-__device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
+// (the builtin itself: HIP's __ballot goes through a 0/1 integer, two vector operations more)
+__device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 
 __device__ __forceinline__ int readlane(int x, int l) { return __builtin_amdgcn_readlane(x, l); }
 __device__ __forceinline__ int readfirst(int x) { return __builtin_amdgcn_readfirstlane(x); }

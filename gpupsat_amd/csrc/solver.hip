@@ -25,10 +25,6 @@ namespace gpsat {
 
 namespace {
 
-constexpr int32_t F_DELETED = 1;
-constexpr int32_t F_USED = 2;
-constexpr int32_t F_LOCKED = 4;
-
 __device__ __forceinline__ int32_t prefix_count(uint64_t m)
 {
     return (int32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
@@ -47,976 +43,1336 @@ __device__ __forceinline__ int32_t wave_inclusive_scan(int32_t x)
     return x;
 }
 
-// Max over the wave of a 64-bit key.
-__device__ __forceinline__ uint64_t wave_max_u64(uint64_t k)
+// Max over the 64 lanes in every lane, by DPP and the permlane swaps as wave_or32 (a shuffle
+// tree of 64-bit keys is 12 LDS round trips; this is none).
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t x)
 {
-#pragma unroll
-    for (int s = 1; s < 64; s <<= 1) {
-        uint32_t lo = __shfl_xor((uint32_t)k, s);
-        uint32_t hi = __shfl_xor((uint32_t)(k >> 32), s);
-        uint64_t o = ((uint64_t)hi << 32) | lo;
-        k = o > k ? o : k;
-    }
-    return k;
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0u, x, 0xB1, 0xF, 0xF, true));
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0u, x, 0x4E, 0xF, 0xF, true));
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0u, x, 0x124, 0xF, 0xF, true));
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0u, x, 0x128, 0xF, 0xF, true));
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    x = max(r[0], r[1]);
+    const auto q = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return max(q[0], q[1]);
 }
 
 __device__ __forceinline__ int32_t uni(int32_t x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ uint32_t uniu(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
 
-// Orders this wavefront's memory accesses across its lanes (per-wave LDS state and, in HBM
-// mode, its slice of the global workspace): waits for its outstanding memory operations,
-// then keeps the compiler from moving accesses across.  The wavefronts of a workgroup are
-// independent, so no workgroup barrier is involved.
-__device__ __forceinline__ void wave_mem_sync()
+// A 64-bit value of lane 0 in every lane.  Values that steer the search must reach it through
+// readfirstlane: a shuffle's result counts as divergent, and one divergent exit of the search
+// loop turns all of its scalar state and branches into vector registers and exec masks.
+__device__ __forceinline__ uint64_t lane0_u64(uint64_t x)
 {
-    __builtin_amdgcn_s_waitcnt(0);
-    wave_sync();
-}
-
-struct Ctx {
-    // instance (uniform)
-    int32_t n, m, inst;
-    bool all3;           // original clause c is lits[3c .. 3c+3)
-    const int32_t* lits;
-    const int32_t* coff;
-    // per-var / per-literal state (LDS)
-    int8_t* lv;          // [2n] literal value: 1 true, -1 false, 0 unassigned
-    int8_t* phase;       // [n]
-    int32_t* seen;       // [n]
-    int32_t* level;      // [n]
-    int32_t* reason;     // [n]  clause id, -1 for decisions and level-0 facts
-    int32_t* trail;      // [n]
-    int32_t* tlim;       // [n+2] trail index where each level starts
-    float* act;          // [n]
-    int32_t* wstart;     // [2n+1] start of each original-clause watch list in Wo
-    int32_t* wcnt_o;     // [2n]
-    int32_t* wcnt_l;     // [2n]
-    int32_t* lbuf;       // [n+1] clause being learned
-    int32_t* lstamp;     // [n+2] level stamps for LBD
-    int32_t* bumps;      // [n]
-    // clause part (LDS or HBM)
-    int32_t* Wo;         // original-clause watch lists (capacity = occurrences)
-    int32_t* Wl;         // learned-clause watch lists, slack slots per literal
-    int32_t* wpair;      // [2*m] the two watched literals of every original clause
-    int32_t* wpl;        // [2*learnt_cap] the same for the learned clauses (clause m + i at 2i)
-    int32_t* lmeta;      // [4*learnt_cap] start, len, flags, lbd; then [learnt_cap] remap slots
-    int32_t* larena;     // learned literals
-    int32_t slack, learnt_cap, larena_cap;
-    // search state (uniform)
-    int32_t dl, tsize, qhead;
-    int32_t nlearnt, larena_used;
-    float inc;
-    int32_t stamp;
-    int32_t base_trail;      // trail entries of the formula's unit clauses
-    int32_t setup_inst;      // instance whose watch lists are built (-1: none)
-    bool setup_ok;
-    bool ran;            // the current job set up its instance (its per-var state is valid)
-    int64_t conf_reported;  // conflicts of the current job already added to its instance pool
-    uint64_t ph_t;           // telemetry: tick at which the current phase began
-    int32_t ph_cur;          // telemetry: the current phase (Phase)
-    unsigned long long* ph_out;  // telemetry: this job's JS_PH_* counters (null: off)
-    int64_t conflicts, decisions, props, learned, restarts;
-    int32_t levelmax;
-};
-
-__device__ __forceinline__ void clause_span(const Ctx& J, int32_t c, const int32_t*& cl, int32_t& len)
-{
-    if (c < J.m && J.all3) {
-        cl = J.lits + 3 * c;
-        len = 3;
-    } else if (c < J.m) {
-        const int32_t b = J.coff[c];
-        len = J.coff[c + 1] - b;
-        cl = J.lits + b;
-    } else {
-        const int32_t* mt = J.lmeta + 4 * (c - J.m);
-        cl = J.larena + mt[0];
-        len = mt[1];
-    }
-}
-
-// Uniform assignment: every lane stores the same values.
-__device__ __forceinline__ void assign(Ctx& J, int32_t u, int32_t r)
-{
-    const int32_t v = u >> 1;
-    J.lv[u] = 1;
-    J.lv[u ^ 1] = -1;
-    J.level[v] = J.dl;
-    J.reason[v] = r;
-    J.trail[J.tsize] = u;
-    J.tsize++;
-}
-
-// Walk the watch list of the false literal fl, 64 entries per step.  Moves watches,
-// compacts the list in place, assigns units in lane order and reports the first
-// conflict.  Returns the new list length.
-template <bool LEARNT>
-__device__ int32_t walk_list(Ctx& J, int32_t fl, int32_t* W, int32_t base, int32_t cnt, int32_t& confl)
-{
-    const int lane = lane_id();
-    int32_t keep = 0;
-    for (int32_t i0 = 0; i0 < cnt; i0 += kWave) {
-        const int32_t i = i0 + lane;
-        const bool active = i < cnt;
-        const int32_t c = active ? W[base + i] : 0;
-        bool kept = active;
-        int32_t unit = -1;
-        bool conf = false;
-        if (active && confl < 0) {
-            bool dead = false;
-            if (LEARNT) dead = (J.lmeta[4 * (c - J.m) + 2] & F_DELETED) != 0;
-            if (dead) {
-                kept = false;
-            } else {
-                int32_t* wp = LEARNT ? J.wpl + 2 * (c - J.m) : J.wpair + 2 * c;
-                const int32_t w0 = wp[0], w1 = wp[1];
-                const int32_t other = (w0 == fl) ? w1 : w0;
-                if (w0 != fl && w1 != fl) {
-                    kept = false;   // stale entry: the clause moved its watch away from fl
-                } else if (J.lv[other] != 1) {
-                    int32_t rep = -1;
-                    if (!LEARNT && J.all3) {
-                        // three literals, two of them the watches: the candidate is the third
-                        // (no offset reads, no search loop)
-                        const int32_t* cl = J.lits + 3 * c;
-                        const int32_t q = (int32_t)((uint32_t)cl[0] + (uint32_t)cl[1] + (uint32_t)cl[2] -
-                                                    (uint32_t)w0 - (uint32_t)w1);
-                        if (q != w0 && q != w1 && J.lv[q] != -1) rep = q;
-                    } else {
-                        const int32_t* cl;
-                        int32_t len;
-                        clause_span(J, c, cl, len);
-                        for (int32_t k = 0; k < len; k++) {
-                            const int32_t q = cl[k];
-                            if (q != w0 && q != w1 && J.lv[q] != -1) {
-                                rep = q;
-                                break;
-                            }
-                        }
-                    }
-                    if (rep >= 0) {
-                        kept = false;
-                        if (!LEARNT) {
-                            const int32_t pos = atomicAdd(&J.wcnt_o[rep], 1);
-                            J.Wo[J.wstart[rep] + pos] = c;
-                            wp[0] = other;
-                            wp[1] = rep;
-                        } else {
-                            const int32_t pos = atomicAdd(&J.wcnt_l[rep], 1);
-                            if (pos < J.slack) {
-                                J.Wl[rep * J.slack + pos] = c;
-                                wp[0] = other;
-                                wp[1] = rep;
-                            } else {
-                                // no room: the learned clause stops propagating (it may still
-                                // be a reason; its literals stay in the arena)
-                                atomicSub(&J.wcnt_l[rep], 1);
-                                atomicOr(&J.lmeta[4 * (c - J.m) + 2], F_DELETED);
-                            }
-                        }
-                    } else if (J.lv[other] == -1) {
-                        conf = true;
-                    } else {
-                        unit = other;
-                    }
-                }
-            }
-        }
-        const uint64_t km = ballot(kept);
-        if (kept) W[base + keep + prefix_count(km)] = c;
-        keep += popc64(km);
-        const uint64_t cm = ballot(conf);
-        if (cm && confl < 0) confl = uni(readlane(c, ctz64(cm)));
-        uint64_t um = ballot(unit >= 0);
-        while (um && confl < 0) {
-            const int j = ctz64(um);
-            um &= um - 1;
-            const int32_t u = uni(readlane(unit, j));
-            const int32_t rc = uni(readlane(c, j));
-            const int8_t val = J.lv[u];
-            if (val == -1) confl = rc;
-            else if (val == 0) assign(J, u, rc);
-        }
-    }
-    return keep;
-}
-
-// walk_list for the original clauses of a batch whose clauses all have three literals, with
-// one divergent region (the watch moves) instead of a branch per test: every lane reads its
-// entry's clause, watch pair, the other watch's value and the third literal's value, and the
-// outcome (keep, move, unit, conflict) is computed from them.  A clause's third literal is the
-// sum of its literals minus its two watches, so no search loop either.
-__device__ int32_t walk_list3(Ctx& J, int32_t fl, int32_t base, int32_t cnt, int32_t& confl)
-{
-    const int lane = lane_id();
-    int32_t* W = J.Wo;
-    int32_t keep = 0;
-    for (int32_t i0 = 0; i0 < cnt; i0 += kWave) {
-        const int32_t i = i0 + lane;
-        const bool in_list = i < cnt;
-        const bool active = in_list && confl < 0;
-        // lanes past the end re-read the last entry (in bounds) and take no action
-        const int32_t c = W[base + min(i, cnt - 1)];
-        const int32_t w0 = J.wpair[2 * c], w1 = J.wpair[2 * c + 1];
-        const int32_t* cl = J.lits + 3 * c;
-        const uint32_t lsum = (uint32_t)cl[0] + (uint32_t)cl[1] + (uint32_t)cl[2];
-        const int32_t other = (w0 == fl) ? w1 : w0;
-        const int32_t q = (int32_t)(lsum - (uint32_t)w0 - (uint32_t)w1);
-        const int8_t vo = J.lv[other];
-        const int8_t vq = J.lv[q];
-        const bool watched = (w0 == fl) || (w1 == fl);   // else a stale entry: dropped
-        const bool open = active && watched && vo != 1;
-        const bool can_move = q != w0 && q != w1 && vq != -1;
-        const bool move = open && can_move;
-        const bool conf = open && !can_move && vo == -1;
-        const int32_t unit = (open && !can_move && vo == 0) ? other : -1;
-        const bool kept = in_list && !(active && (!watched || move));
-        if (move) {
-            const int32_t pos = atomicAdd(&J.wcnt_o[q], 1);
-            J.Wo[J.wstart[q] + pos] = c;
-            J.wpair[2 * c] = other;
-            J.wpair[2 * c + 1] = q;
-        }
-        const uint64_t km = ballot(kept);
-        if (kept) W[base + keep + prefix_count(km)] = c;
-        keep += popc64(km);
-        const uint64_t cm = ballot(conf);
-        if (cm && confl < 0) confl = uni(readlane(c, ctz64(cm)));
-        uint64_t um = ballot(unit >= 0);
-        while (um && confl < 0) {
-            const int j = ctz64(um);
-            um &= um - 1;
-            const int32_t u = uni(readlane(unit, j));
-            const int32_t rc = uni(readlane(c, j));
-            const int8_t val = J.lv[u];
-            if (val == -1) confl = rc;
-            else if (val == 0) assign(J, u, rc);
-        }
-    }
-    return keep;
-}
-
-__device__ int32_t propagate(Ctx& J)
-{
-    int32_t confl = -1;
-    while (confl < 0 && J.qhead < J.tsize) {
-        const int32_t p = uni(J.trail[J.qhead]);
-        J.qhead++;
-        J.props++;
-        const int32_t fl = p ^ 1;
-        const int32_t wb = uni(J.wstart[fl]), wc = uni(J.wcnt_o[fl]);
-        int32_t k = J.all3 ? walk_list3(J, fl, wb, wc, confl) : walk_list<false>(J, fl, J.Wo, wb, wc, confl);
-        J.wcnt_o[fl] = k;
-        k = walk_list<true>(J, fl, J.Wl, fl * J.slack, uni(J.wcnt_l[fl]), confl);
-        J.wcnt_l[fl] = k;
-    }
-    return confl;
-}
-
-__device__ void backtrack(Ctx& J, int32_t b, bool save_phase)
-{
-    if (J.dl <= b) return;
-    const int32_t start = uni(J.tlim[b + 1]);
-    for (int32_t t = start + lane_id(); t < J.tsize; t += kWave) {
-        const int32_t u = J.trail[t];
-        const int32_t v = u >> 1;
-        J.lv[u] = 0;
-        J.lv[u ^ 1] = 0;
-        J.reason[v] = -1;
-        if (save_phase) J.phase[v] = (int8_t)(u & 1);
-    }
-    wave_mem_sync();
-    J.tsize = start;
-    J.qhead = start;
-    J.dl = b;
-}
-
-// 1-UIP.  Leaves the learned clause in lbuf[0..len) with the asserting literal first and
-// a literal of the backjump level second.
-__device__ int32_t analyze(Ctx& J, int32_t confl, int32_t& bt, int32_t& lbd)
-{
-    const int lane = lane_id();
-    // the loop state is wave-uniform; uni() keeps it in scalar registers, so the trail scan
-    // below is a scalar loop rather than an exec-masked one
-    int32_t nl = 1, pathc = 0, p = -1, idx = uni(J.tsize - 1), c = confl;
-    for (;;) {
-        if (c >= J.m) {
-            const int32_t f = J.lmeta[4 * (c - J.m) + 2];
-            J.lmeta[4 * (c - J.m) + 2] = f | F_USED;
-        }
-        const int32_t* cl;
-        int32_t len;
-        clause_span(J, c, cl, len);
-        for (int32_t k0 = 0; k0 < len; k0 += kWave) {
-            const int32_t k = k0 + lane;
-            // every lane reads (lanes past the clause re-read its last literal and take no
-            // part), so the only divergent regions are the marking and its bookkeeping
-            const int32_t qr = cl[min(k, len - 1)];
-            const int32_t q = k < len ? qr : -1;
-            const int32_t v = qr >> 1;
-            const int32_t lvl = J.level[v];
-            bool mark = false;
-            if (q >= 0 && q != p && lvl > 0) mark = atomicOr(&J.seen[v], 1) == 0;
-            const bool cur = mark && lvl == J.dl;
-            if (mark) {
-                J.act[v] += J.inc;
-                J.bumps[v] += 1;
-            }
-            const uint64_t cmask = ballot(mark && cur);
-            pathc += popc64(cmask);
-            const uint64_t lmask = ballot(mark && !cur);
-            if (mark && !cur) J.lbuf[nl + prefix_count(lmask)] = q;
-            nl += popc64(lmask);
-        }
-        // next marked literal on the trail, walking back from idx
-        bool found = false;
-        while (idx >= 0) {
-            const int32_t t = idx - lane;
-            const int32_t tl = J.trail[max(t, 0)];
-            const bool hit = t >= 0 && J.seen[tl >> 1] != 0;
-            const uint64_t hm = ballot(hit);
-            if (hm) {
-                idx = uni(idx - ctz64(hm));
-                found = true;
-                break;
-            }
-            idx = uni(idx - kWave);
-        }
-        if (!found) return -1;   // no current-level literal: internal error, reported by the caller
-        p = uni(J.trail[idx]);
-        idx--;
-        J.seen[p >> 1] = 0;
-        pathc--;
-        if (pathc <= 0) break;
-        c = uni(J.reason[p >> 1]);
-    }
-    J.lbuf[0] = p ^ 1;
-    wave_mem_sync();
-    // Local minimization: a literal whose reason's other literals are all in the clause (or at
-    // level 0) is implied by the rest and dropped.  First every literal is tested against the
-    // clause as learned (drops are marked ~q, seen flags untouched), then the clause is
-    // compacted and the dropped literals' seen flags cleared, so the result does not depend on
-    // lane order.  Dropping several at once is sound: resolving them out in reverse trail
-    // order only meets literals that stay in the clause or are resolved out earlier.
-    if (nl > 1) {
-        for (int32_t k = 1 + lane; k < nl; k += kWave) {
-            const int32_t q = J.lbuf[k];
-            const int32_t v = q >> 1;
-            const int32_t r = J.reason[v];
-            if (r < 0) continue;
-            const int32_t* cl;
-            int32_t len;
-            clause_span(J, r, cl, len);
-            bool drop = true;
-            for (int32_t j = 0; j < len && drop; j++) {
-                const int32_t vx = cl[j] >> 1;
-                if (vx != v && J.seen[vx] == 0 && J.level[vx] > 0) drop = false;
-            }
-            if (drop) J.lbuf[k] = ~q;
-        }
-        wave_mem_sync();
-        int32_t kept = 1;
-        for (int32_t k0 = 1; k0 < nl; k0 += kWave) {
-            const int32_t k = k0 + lane;
-            const int32_t x = k < nl ? J.lbuf[k] : 0;
-            const bool keep = k < nl && x >= 0;
-            if (k < nl && x < 0) J.seen[(~x) >> 1] = 0;
-            const uint64_t km = ballot(keep);
-            wave_mem_sync();
-            if (keep) J.lbuf[kept + prefix_count(km)] = x;
-            kept += popc64(km);
-        }
-        nl = uni(kept);
-        wave_mem_sync();
-    }
-    // backjump level = highest level among the other literals; LBD = distinct levels
-    J.stamp++;
-    uint64_t best = 0;
-    int32_t distinct = 0;
-    for (int32_t k = 1 + lane; k < nl; k += kWave) {
-        const int32_t q = J.lbuf[k];
-        const int32_t v = q >> 1;
-        J.seen[v] = 0;
-        const int32_t lv = J.level[v];
-        const uint64_t key = ((uint64_t)(uint32_t)lv << 32) | (uint32_t)(0x7fffffff - k);
-        best = key > best ? key : best;
-        if (atomicExch(&J.lstamp[lv], J.stamp) != J.stamp) distinct++;
-    }
-    best = wave_max_u64(best);
-    for (int s = 32; s > 0; s >>= 1) distinct += __shfl_xor(distinct, s);
-    lbd = uni(distinct) + 1;
-    if (nl > 1) {
-        bt = uni((int32_t)(best >> 32));
-        const int32_t bi = uni(0x7fffffff - (int32_t)(uint32_t)best);
-        const int32_t t1 = J.lbuf[1], tb = J.lbuf[bi];
-        wave_mem_sync();
-        J.lbuf[1] = tb;
-        J.lbuf[bi] = t1;
-    } else {
-        bt = 0;
-    }
-    wave_mem_sync();
-    return nl;
-}
-
-// Append lbuf[0..len) as a learned clause.  Returns its clause id.
-__device__ int32_t store_learned(Ctx& J, int32_t len, int32_t lbd)
-{
-    const int32_t id = J.nlearnt;
-    const int32_t start = J.larena_used;
-    for (int32_t k = lane_id(); k < len; k += kWave) J.larena[start + k] = J.lbuf[k];
-    J.lmeta[4 * id + 0] = start;
-    J.lmeta[4 * id + 1] = len;
-    J.lmeta[4 * id + 2] = 0;
-    J.lmeta[4 * id + 3] = lbd;
-    J.nlearnt++;
-    J.larena_used += len;
-    J.learned++;
-    return J.m + id;
-}
-
-// Watch a learned clause on literals a and b (uniform).
-__device__ void watch_learned(Ctx& J, int32_t c, int32_t a, int32_t b)
-{
-    J.wpl[2 * (c - J.m)] = a;
-    J.wpl[2 * (c - J.m) + 1] = b;
-    const int32_t pa = uni(J.wcnt_l[a]);
-    const int32_t pb = uni(J.wcnt_l[b]) + (a == b ? 1 : 0);
-    if (pa < J.slack && pb < J.slack) {
-        J.Wl[a * J.slack + pa] = c;
-        J.wcnt_l[a] = pa + 1;
-        const int32_t pb2 = uni(J.wcnt_l[b]);
-        J.Wl[b * J.slack + pb2] = c;
-        J.wcnt_l[b] = pb2 + 1;
-    } else {
-        J.lmeta[4 * (c - J.m) + 2] |= F_DELETED;
-    }
-}
-
-// At level 0: attach learned clause i (an index into lmeta).  A clause satisfied at
-// level 0 is dropped, a clause with one non-false literal asserts it, a falsified
-// clause means the job is UNSAT (returns false).
-__device__ bool attach_level0(Ctx& J, int32_t i)
-{
-    const int lane = lane_id();
-    const int32_t st = uni(J.lmeta[4 * i]);
-    const int32_t len = uni(J.lmeta[4 * i + 1]);
-    int32_t nf[2] = {-1, -1};
-    int32_t nnf = 0;
-    bool sat = false;
-    for (int32_t k0 = 0; k0 < len && nnf < 2 && !sat; k0 += kWave) {
-        const int32_t k = k0 + lane;
-        const int32_t q = k < len ? J.larena[st + k] : -1;
-        const int8_t v = q >= 0 ? J.lv[q] : (int8_t)-1;
-        if (ballot(v == 1)) sat = true;
-        uint64_t um = ballot(v == 0);
-        while (um && nnf < 2) {
-            const int j = ctz64(um);
-            um &= um - 1;
-            nf[nnf++] = uni(readlane(q, j));
-        }
-    }
-    bool ok = true;
-    if (sat) {
-        J.lmeta[4 * i + 2] = F_DELETED;
-    } else if (nnf == 0) {
-        ok = false;
-    } else if (nnf == 1) {
-        J.lmeta[4 * i + 2] = F_DELETED;
-        if (J.lv[nf[0]] == 0) assign(J, nf[0], -1);
-    } else {
-        watch_learned(J, J.m + i, nf[0], nf[1]);
-    }
-    wave_mem_sync();
-    return ok;
-}
-
-// Reduce the learned DB at the current level.  Survivors: reasons of assigned literals
-// (always), glue clauses (LBD <= 3) and, in mode 0, clauses used since the last
-// reduction; mode 2 keeps the reasons only.  Clause ids are renumbered, reasons are
-// remapped and the learned watch lists are rebuilt from the watch pairs, which keeps
-// the two-watched-literal invariant at any level.
-__device__ void reduce_db(Ctx& J, int mode)
-{
-    const int lane = lane_id();
-    const int32_t m = J.m;
-    int32_t* remap = J.lmeta + 4 * J.learnt_cap;
-    for (int32_t t = lane; t < J.tsize; t += kWave) {
-        const int32_t v = J.trail[t] >> 1;
-        const int32_t r = J.reason[v];
-        if (r >= m && J.level[v] > 0) atomicOr(&J.lmeta[4 * (r - m) + 2], F_LOCKED);   // level-0 reasons are never read
-    }
-    wave_mem_sync();
-    int32_t ns = 0;
-    for (int32_t i0 = 0; i0 < J.nlearnt; i0 += kWave) {
-        const int32_t i = i0 + lane;
-        bool keep = false, del = false;
-        int32_t st = 0, len = 0, lbd = 0, w0 = 0, w1 = 0;
-        if (i < J.nlearnt) {
-            st = J.lmeta[4 * i];
-            len = J.lmeta[4 * i + 1];
-            const int32_t fl = J.lmeta[4 * i + 2];
-            lbd = J.lmeta[4 * i + 3];
-            w0 = J.wpl[2 * i];
-            w1 = J.wpl[2 * i + 1];
-            del = (fl & F_DELETED) != 0;
-            const bool wanted = mode == 0 ? (lbd <= 3 || (fl & F_USED)) : mode == 1 ? lbd <= 3 : false;
-            keep = (fl & F_LOCKED) || (!del && wanted);
-        }
-        const uint64_t km = ballot(keep);
-        wave_mem_sync();
-        const int32_t ni = ns + prefix_count(km);
-        if (i < J.nlearnt) remap[i] = keep ? ni : -1;
-        if (keep) {
-            J.lmeta[4 * ni] = st;
-            J.lmeta[4 * ni + 1] = len;
-            J.lmeta[4 * ni + 2] = del ? F_DELETED : 0;
-            J.lmeta[4 * ni + 3] = lbd;
-            J.wpl[2 * ni] = w0;
-            J.wpl[2 * ni + 1] = w1;
-        }
-        ns += popc64(km);
-        wave_mem_sync();
-    }
-    // compact literals (forward copy; a destination never lies above its source)
-    int32_t pos = 0;
-    for (int32_t i = 0; i < ns; i++) {
-        const int32_t st = uni(J.lmeta[4 * i]);
-        const int32_t len = uni(J.lmeta[4 * i + 1]);
-        for (int32_t k0 = 0; k0 < len; k0 += kWave) {
-            const int32_t k = k0 + lane;
-            const int32_t x = k < len ? J.larena[st + k] : 0;
-            wave_mem_sync();
-            if (k < len) J.larena[pos + k] = x;
-            wave_mem_sync();
-        }
-        J.lmeta[4 * i] = pos;
-        pos += len;
-    }
-    for (int32_t t = lane; t < J.tsize; t += kWave) {
-        const int32_t v = J.trail[t] >> 1;
-        const int32_t r = J.reason[v];
-        if (r >= m) J.reason[v] = remap[r - m] >= 0 ? m + remap[r - m] : -1;
-    }
-    for (int32_t l = lane; l < 2 * J.n; l += kWave) J.wcnt_l[l] = 0;
-    wave_mem_sync();
-    for (int32_t i = lane; i < ns; i += kWave) {
-        if (J.lmeta[4 * i + 2] & F_DELETED) continue;
-        const int32_t c = m + i;
-        const int32_t wl[2] = {J.wpl[2 * i], J.wpl[2 * i + 1]};
-        for (int h = 0; h < 2; h++) {
-            const int32_t p = atomicAdd(&J.wcnt_l[wl[h]], 1);
-            if (p < J.slack) {
-                J.Wl[wl[h] * J.slack + p] = c;
-            } else {
-                atomicSub(&J.wcnt_l[wl[h]], 1);
-                J.lmeta[4 * i + 2] = F_DELETED;
-            }
-        }
-    }
-    J.nlearnt = ns;
-    J.larena_used = pos;
-    wave_mem_sync();
-}
-
-__device__ int32_t pick_branch(Ctx& J, int mode)
-{
-    uint64_t best = 0;
-    for (int32_t v = lane_id(); v < J.n; v += kWave) {
-        if (J.lv[2 * v] == 0) {
-            uint32_t hi = mode == 1 ? 1u : (__float_as_uint(J.act[v]) | 0x80000000u) ;
-            // larger key wins: activity first (non-negative floats order as integers),
-            // then the lower var (VSIDS) or the higher var (reference: last free var)
-            uint32_t lo = mode == 1 ? (uint32_t)v + 1u : 0xffffffffu - (uint32_t)v;
-            uint64_t key = ((uint64_t)hi << 32) | lo;
-            best = key > best ? key : best;
-        }
-    }
-    best = wave_max_u64(best);
-    if (best == 0) return -1;
-    const uint32_t lo = (uint32_t)best;
-    return uni(mode == 1 ? (int32_t)(lo - 1u) : (int32_t)(0xffffffffu - lo));
-}
-
-__device__ void rescale_activity(Ctx& J)
-{
-    for (int32_t v = lane_id(); v < J.n; v += kWave) J.act[v] *= 1e-30f;
-    J.inc *= 1e-30f;
-    wave_mem_sync();
+    return (uint64_t)uniu((uint32_t)x) | (uint64_t)uniu((uint32_t)(x >> 32)) << 32;
 }
 
 __device__ __forceinline__ int32_t load_status(int32_t* p)
 {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return uni(__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 }
 
-// Lay out the per-wave arrays.  The state part always sits in LDS; the clause part
-// sits in LDS (kLds) or in this wave's slice of the HBM workspace.
-struct Layout {
-    static __host__ __device__ size_t state_bytes(int32_t n)
-    {
-        size_t b = 0;
-        b += ((2 * (size_t)n + 3) & ~(size_t)3);        // lv
-        b += (((size_t)n + 3) & ~(size_t)3);            // phase
-        b += 4 * (size_t)n * 5;                         // seen level reason trail act
-        b += 4 * ((size_t)n + 2);                       // tlim
-        b += 4 * (2 * (size_t)n + 1);                   // wstart
-        b += 4 * (2 * (size_t)n) * 2;                   // wcnt_o wcnt_l
-        b += 4 * ((size_t)n + 1);                       // lbuf
-        b += 4 * ((size_t)n + 2);                       // lstamp
-        b += 4 * (size_t)n;                             // bumps
-        return (b + 15) & ~(size_t)15;
-    }
+template <class I> struct Vec;
+template <> struct Vec<uint16_t> {
+    typedef uint16_t x2 __attribute__((ext_vector_type(2)));
+    typedef uint16_t x4 __attribute__((ext_vector_type(4)));
+};
+template <> struct Vec<uint32_t> {
+    typedef uint32_t x2 __attribute__((ext_vector_type(2)));
+    typedef uint32_t x4 __attribute__((ext_vector_type(4)));
 };
 
-__device__ void carve_state(Ctx& J, char* s, int32_t n)
-{
-    J.lv = (int8_t*)s;                 s += ((2 * n + 3) & ~3);
-    J.phase = (int8_t*)s;              s += ((n + 3) & ~3);
-    J.seen = (int32_t*)s;              s += 4 * n;
-    J.level = (int32_t*)s;             s += 4 * n;
-    J.reason = (int32_t*)s;            s += 4 * n;
-    J.trail = (int32_t*)s;             s += 4 * n;
-    J.act = (float*)s;                 s += 4 * n;
-    J.tlim = (int32_t*)s;              s += 4 * (n + 2);
-    J.wstart = (int32_t*)s;            s += 4 * (2 * n + 1);
-    J.wcnt_o = (int32_t*)s;            s += 4 * (2 * n);
-    J.wcnt_l = (int32_t*)s;            s += 4 * (2 * n);
-    J.lbuf = (int32_t*)s;              s += 4 * (n + 1);
-    J.lstamp = (int32_t*)s;            s += 4 * (n + 2);
-    J.bumps = (int32_t*)s;
-}
-
-__device__ void carve_clauses(Ctx& J, int32_t* c, const SolveArgs& a)
-{
-    J.Wo = c;      c += a.wo_cap;
-    J.Wl = c;      c += a.wl_cap;
-    J.wpair = c;
-    J.wpl = c + (a.wpair_cap - 2 * a.o.learnt_cap);
-    c += a.wpair_cap;
-    J.lmeta = c;   c += a.lmeta_cap;
-    J.larena = c;
-}
-
-// Build the per-instance part of a job: watch lists of the original clauses and the
-// formula's unit clauses at level 0.  Returns false if the formula is falsified there.
-__device__ bool setup_instance(Ctx& J, const SolveArgs& a, int32_t inst)
-{
-    const int lane = lane_id();
-    const SolveOptsDev& o = a.o;
-    const InstMeta mi = a.meta[inst];
-    J.inst = inst;
-    J.n = uni(mi.n);
-    J.m = uni(mi.m);
-    J.lits = a.lits + mi.lit_base;
-    J.coff = a.coff + mi.coff_base;
-    J.all3 = a.all3 != 0;
-    const int32_t n = J.n, m = J.m, n2 = 2 * n;
-    const int64_t vb = a.var_base[inst];
-    J.slack = o.watch_slack;
-    J.learnt_cap = o.learnt_cap;
-    J.larena_cap = o.larena_cap;
-    J.dl = 0;
-    J.tsize = 0;
-    J.qhead = 0;
-    J.nlearnt = 0;
-    J.larena_used = 0;
-    J.inc = 1.0f;
-    J.stamp = 0;
-    for (int32_t v = lane; v < n; v += kWave) {
-        J.seen[v] = 0;
-        J.level[v] = 0;
-        J.reason[v] = -1;
-        J.act[v] = a.act_init ? a.act_init[vb + v] : 0.0f;
-        J.phase[v] = a.phase_init ? a.phase_init[vb + v] : (int8_t)o.phase_init;
-        J.bumps[v] = 0;
+// A literal's watch header: where its original-clause list starts and how long its two lists
+// are, in one LDS read.  With 16-bit ids both lengths share a word (original low, learned
+// high), so that one atomic add appends to either list.
+template <class I> struct Hdr;
+template <> struct Hdr<uint16_t> {
+    typedef uint2 type;
+    static __device__ __forceinline__ int32_t no(const type& h) { return (int32_t)(h.y & 0xffffu); }
+    static __device__ __forceinline__ int32_t nl(const type& h) { return (int32_t)(h.y >> 16); }
+    static __device__ __forceinline__ int32_t add_o(type* h) { return (int32_t)(atomicAdd(&h->y, 1u) & 0xffffu); }
+    static __device__ __forceinline__ int32_t add_l(type* h) { return (int32_t)(atomicAdd(&h->y, 0x10000u) >> 16); }
+    static __device__ __forceinline__ void sub_o(type* h) { atomicSub(&h->y, 1u); }
+    static __device__ __forceinline__ void sub_l(type* h) { atomicSub(&h->y, 0x10000u); }
+    static __device__ __forceinline__ void set(type* h, int32_t no, int32_t nl) { h->y = (uint32_t)no | (uint32_t)nl << 16; }
+    static __device__ __forceinline__ void set_l0(type* h) { h->y &= 0xffffu; }
+};
+template <> struct Hdr<uint32_t> {
+    typedef uint4 type;
+    static __device__ __forceinline__ int32_t no(const type& h) { return (int32_t)h.y; }
+    static __device__ __forceinline__ int32_t nl(const type& h) { return (int32_t)h.z; }
+    static __device__ __forceinline__ int32_t add_o(type* h) { return (int32_t)atomicAdd(&h->y, 1u); }
+    static __device__ __forceinline__ int32_t add_l(type* h) { return (int32_t)atomicAdd(&h->z, 1u); }
+    static __device__ __forceinline__ void sub_o(type* h) { atomicSub(&h->y, 1u); }
+    static __device__ __forceinline__ void sub_l(type* h) { atomicSub(&h->z, 1u); }
+    static __device__ __forceinline__ void set(type* h, int32_t no, int32_t nl)
+    {
+        h->y = (uint32_t)no;
+        h->z = (uint32_t)nl;
     }
-    for (int32_t v = lane; v < n + 2; v += kWave) J.lstamp[v] = 0;
-    for (int32_t l = lane; l < n2; l += kWave) {
-        J.lv[l] = 0;
-        J.wcnt_o[l] = 0;
-        J.wcnt_l[l] = 0;
+    static __device__ __forceinline__ void set_l0(type* h) { h->z = 0u; }
+};
+
+// One wavefront's search.  kMode: see k_solve.  I: the type of literal codes, clause ids,
+// levels and positions.  ALL3: every original clause has three literals.
+//
+// The search is one long chain of dependent steps, run by one wavefront at a time at about 5
+// cycles an instruction, 64 a trip to LDS, 20 a branch and 15-20 each time a scalar is made from
+// vector lanes or used by them after a compare (measured on one wavefront).  Before this layout a
+// propagated literal took 2,800 cycles in about 400 instructions, whether 1 or 8,192 wavefronts
+// ran.  So:
+//  * 16-bit ids, so that what a step reads is one record: a literal's header (list start and
+//    both lengths), a clause's record (its watches and literals), a variable's level and
+//    reason; the per-job state shrinks enough to hold the watch structures in LDS.
+//  * both watch lists of a literal are walked in one pass of the wavefront, one entry per lane,
+//    and the next literal's header and entries are fetched while the current one is processed
+//    (a queued literal's negation is false, so nothing moves a watch to its lists meanwhile).
+//  * what a lane decides is computed from value codes (false 0, unassigned 1, true 2) by vector
+//    arithmetic; only a unit, a conflict or an open learned clause leaves the straight line.
+//  * reductions run on DPP and ballots, not on LDS shuffles.
+template <int kMode, class I, bool ALL3>
+struct Search {
+    typedef typename Vec<I>::x2 I2;
+    typedef typename Vec<I>::x4 I4;
+    typedef Hdr<I> H;
+    typedef typename H::type HT;
+    static constexpr I kNone = (I)~(I)0;
+    static constexpr I kDrop = (I)((I)1 << (8 * sizeof(I) - 1));   // a literal dropped by minimization
+
+    // instance (uniform)
+    int32_t n, m, inst;
+    // per-var / per-literal state
+    HT* hdr;             // [2n]
+    I4* vi;              // [n] of an assigned var: level, reason clause (kNone: a decision or a
+                         // level-0 fact), trail index, nonzero at level 0 or while the analysis
+                         // has the var in its clause
+    float* act;          // [n]
+    int32_t* lstamp;     // [n+2] level stamps for LBD
+    I* trail;            // [n]
+    I* tlim;             // [n+2] trail index where each level starts
+    I* lbuf;             // [n+1] clause being learned
+    uint8_t* lv;         // [2n+1] literal value: 0 false, 1 unassigned, 2 true; [2n] is always false
+    int8_t* phase;       // [n]
+    uint8_t* mark;       // [64] scratch of the analysis, zero between its steps
+    // watch structures
+    I* Wo;               // original-clause watch lists (capacity = occurrences)
+    I4* rec;             // [m] ALL3: the three literals in order and the unwatched one; else the
+                         // two watches, first literal / 4 in olits, length
+    I* Wl;               // learned-clause watch lists, slack slots per literal (index of the clause)
+    I4* lrec;            // [learnt_cap] the two watches (kNone: detached), first literal / 8 in larena, length
+    I* llbd;             // [learnt_cap]
+    I* remap;            // [learnt_cap] scratch of reduce_db
+    uint8_t* lused;      // [learnt_cap] used by an analysis since the last reduction
+    I* olits;            // original literals (not ALL3), each clause filled up to a multiple of 4
+                         // with the always-false literal
+    I* larena;           // learned literals, likewise to a multiple of 8
+    int32_t slack, learnt_cap, larena_cap;
+    // search state (uniform)
+    int32_t dl, tsize, qhead;
+    int32_t nlearnt, larena_used, larena_top;   // clauses held, their literals, next free literal / 8
+    float inc;
+    int32_t stamp;
+    bool dups;               // some original clause names a variable twice
+    bool shortl;             // no watch list can outgrow the wavefront
+    int32_t base_trail;      // trail entries of the formula's unit clauses
+    int32_t setup_inst;      // instance whose watch lists are built (-1: none)
+    bool setup_ok;
+    bool ran;                // the current job set up its instance (its per-var state is valid)
+    int64_t conf_reported;   // conflicts of the current job already added to its instance pool
+    uint64_t ph_t;           // telemetry: tick at which the current phase began
+    int32_t ph_cur;          // telemetry: the current phase (Phase)
+    unsigned long long* ph_out;  // telemetry: this job's JS_PH_* counters (null: off)
+    int32_t* bumps;          // the instance's slice of var_bumps (null: off)
+    int64_t conflicts, decisions, props, learned, restarts;
+    int32_t levelmax;
+
+    // Orders this wavefront's accesses across its lanes.  LDS requests of one wavefront are
+    // served in order, so with the state in LDS only the compiler has to be held; state in this
+    // wavefront's HBM slice also waits for its outstanding memory operations.
+    static __device__ __forceinline__ void lsync() { wave_sync(); }
+    static __device__ __forceinline__ void msync()
+    {
+        if (kMode != 1) __builtin_amdgcn_s_waitcnt(0);
+        wave_sync();
     }
-    wave_mem_sync();
-    // occurrence counts give the capacity of every original-clause watch list
-    const int32_t L = uni(J.coff[m]);
-    for (int32_t k = lane; k < L; k += kWave) atomicAdd(&J.wcnt_o[J.lits[k]], 1);
-    wave_mem_sync();
-    int32_t carry = 0;
-    for (int32_t l0 = 0; l0 < n2; l0 += kWave) {
-        const int32_t l = l0 + lane;
-        const int32_t x = l < n2 ? J.wcnt_o[l] : 0;
-        const int32_t inc = wave_inclusive_scan(x);
-        if (l < n2) {
-            J.wstart[l] = carry + inc - x;
-            J.wcnt_o[l] = 0;
+    static __device__ __forceinline__ bool lane0() { return lane_id() == 0; }
+
+    // ---- layout: state part, watch part, learned literals (see solve_layout)
+    __device__ __forceinline__ void carve(char* s, char* w, char* ar, const SolveArgs& a)
+    {
+        const SolveLayout& L = a.lay;
+        hdr = (HT*)(s + L.hdr);
+        vi = (I4*)(s + L.vi);
+        act = (float*)(s + L.act);
+        lstamp = (int32_t*)(s + L.lstamp);
+        trail = (I*)(s + L.trail);
+        tlim = (I*)(s + L.tlim);
+        lbuf = (I*)(s + L.lbuf);
+        lv = (uint8_t*)(s + L.lv);
+        phase = (int8_t*)(s + L.phase);
+        mark = (uint8_t*)(s + L.mark);
+        rec = (I4*)(w + L.rec);
+        lrec = (I4*)(w + L.lrec);
+        Wo = (I*)(w + L.wo);
+        Wl = (I*)(w + L.wl);
+        llbd = (I*)(w + L.llbd);
+        remap = (I*)(w + L.remap);
+        lused = (uint8_t*)(w + L.lused);
+        olits = (I*)(w + L.olits);
+        larena = (I*)ar;
+    }
+
+    // Values of both literals of var v in one store (v's literals are adjacent bytes).
+    __device__ __forceinline__ void set_value(int32_t u) { *(uint16_t*)(lv + (u & ~1)) = (u & 1) ? 0x0200u : 0x0002u; }
+    __device__ __forceinline__ void clear_value(int32_t u) { *(uint16_t*)(lv + (u & ~1)) = 0x0101u; }
+
+    // Uniform assignment of literal u with reason clause r.  One lane stores: 64 lanes storing the
+    // same 1- or 2-byte value to one address are served one after another.
+    __device__ __forceinline__ void assign(int32_t u, I r)
+    {
+        if (lane0()) {
+            set_value(u);
+            I4 x;
+            x.x = (I)dl;
+            x.y = r;
+            x.z = (I)tsize;
+            x.w = dl == 0 ? (I)1 : (I)0;
+            vi[u >> 1] = x;
+            trail[tsize] = (I)u;
         }
-        carry += uni(__shfl(inc, 63));
+        tsize++;
+        lsync();
     }
-    if (lane == 0) J.wstart[n2] = carry;
-    wave_mem_sync();
-    // watch the first two literals of every clause; units and empty clauses at level 0
-    bool unsat = false;
-    for (int32_t c0 = 0; c0 < m && !unsat; c0 += kWave) {
-        const int32_t c = c0 + lane;
-        int32_t len = -1, l0 = -1;
-        if (c < m) {
-            const int32_t b = J.coff[c];
-            len = J.coff[c + 1] - b;
-            if (len >= 1) {
-                l0 = J.lits[b];
-                // the two watches are distinct literals; a clause repeating one literal is a unit
-                int32_t l1 = -1;
-                for (int32_t k = 1; k < len; k++) {
-                    const int32_t q = J.lits[b + k];
-                    if (q != l0) {
-                        l1 = q;
-                        break;
+
+    __device__ __forceinline__ uint32_t value(int32_t u) const { return (uint32_t)lv[u]; }
+
+    // Assigns the units of one step in lane order (mask um: lanes whose clause id is unit on
+    // their literal u, all unassigned before the step).  A literal met again is skipped; the
+    // complement of one assigned here is a conflict in that lane's clause.
+    __device__ __forceinline__ void assign_units(uint64_t um, int32_t u, int32_t id, int32_t& confl)
+    {
+        int j = ctz64(um);
+        int32_t x = readlane(u, j);
+        assign(x, (I)readlane(id, j));
+        um &= um - 1;
+        uint64_t comp = 0;
+        while (um) {
+            um &= ~ballot(u == x);
+            comp |= ballot(u == (x ^ 1));
+            j = ctz64(um);
+            if (um && ((comp >> j) & 1)) {
+                confl = readlane(id, j);
+                um = 0;
+            }
+            if (um) {
+                x = readlane(u, j);
+                assign(x, (I)readlane(id, j));
+                um &= um - 1;
+            }
+        }
+    }
+
+    // The first literal of a clause (its literals at q, filled up to a multiple of W with false
+    // ones) that is neither `other` nor false, kNone if none: W literals per round trip.
+    template <int W>
+    __device__ __forceinline__ uint32_t find_watch(const I* q, int32_t len, uint32_t other) const
+    {
+        uint32_t rep = kNone;
+        for (int32_t k = 0; k < len && rep == (uint32_t)kNone; k += W) {
+            uint32_t x[W], v[W];
+#pragma unroll
+            for (int t = 0; t < W; t += 4) {
+                const I4 y = *(const I4*)(q + k + t);
+                x[t] = y.x;
+                x[t + 1] = y.y;
+                x[t + 2] = y.z;
+                x[t + 3] = y.w;
+            }
+#pragma unroll
+            for (int t = 0; t < W; t++) v[t] = lv[x[t]];
+#pragma unroll
+            for (int t = W - 1; t >= 0; t--) rep = min(v[t], x[t] ^ other) != 0u ? x[t] : rep;
+        }
+        return rep;
+    }
+
+    // One step of an original-clause list of the false literal fl (start ws), 64 entries from i0,
+    // of which lanes `in` hold one (e) and its record (r).  Moves watches, compacts the list in
+    // place from `keep` on, assigns units in lane order and reports the first conflict.
+    __device__ __forceinline__ void step_original(uint32_t fl, uint32_t ws, int32_t i0, int32_t& keep, bool in,
+                                                  uint32_t e, I4 r, int32_t& confl)
+    {
+        uint32_t other, rep;
+        bool open, move;
+        if (ALL3) {
+            // the unwatched literal is the only candidate
+            rep = r.w;
+            other = (uint32_t)r.x + r.y + r.z - fl - rep;
+            open = in && confl < 0 && value(other) != 2;
+            move = open && rep != other && value(rep) != 0;
+        } else {
+            other = (uint32_t)r.x + r.y - fl;
+            open = in && confl < 0 && value(other) != 2;
+            rep = kNone;
+            if (open && r.w > 2) rep = find_watch<4>(olits + 4 * (uint32_t)r.z, r.w, other);
+            move = rep != (uint32_t)kNone;
+        }
+        const bool no = open && !move && value(other) == 0, unit = open && !move && !no;
+        const uint64_t mm = ballot(move);
+        if (move) {
+            const uint32_t at = (uint32_t)hdr[rep].x + H::add_o(&hdr[rep]);
+            H::sub_o(&hdr[fl]);
+            Wo[at] = (I)e;
+            if (ALL3) {
+                rec[e].w = (I)fl;
+            } else {
+                I2 w;
+                w.x = (I)other;
+                w.y = (I)rep;
+                *(I2*)&rec[e] = w;
+            }
+        }
+        const uint64_t km = ballot(in) & ~mm;
+        if ((mm || keep != i0) && in && !move) Wo[ws + keep + prefix_count(km)] = (I)e;
+        keep += popc64(km);
+        lsync();
+        const uint64_t cm = ballot(no), um = ballot(unit);
+        if (cm) confl = readlane(e, ctz64(cm));
+        else if (um) assign_units(um, other, e, confl);
+    }
+
+    // One step of a learned-clause list of fl (start base), as above; other, vo: the entry's
+    // other watch and its value, read after the last assignment.  A clause with no room in its
+    // new list is detached: it stops propagating, but may still be a reason.
+    __device__ __forceinline__ void step_learned(uint32_t fl, uint32_t base, int32_t i0, int32_t& keep, bool in,
+                                                 uint32_t e, I4 r, uint32_t other, uint32_t vo, int32_t& confl)
+    {
+        const bool active = in && confl < 0;
+        const bool dead = active && r.x == kNone;
+        const bool open = active && !dead && vo != 2;
+        uint32_t rep = kNone;
+        uint64_t om = ballot(open);
+        if ((om & (om - 1)) == 0) {
+            // one open clause: its literals across the lanes
+            if (om) {
+                const int j = ctz64(om);
+                const I* q = larena + 8 * readlane(r.z, j);
+                const int32_t len = readlane(r.w, j);
+                const uint32_t oj = readlane(other, j);
+                for (int32_t k = 0; om && k < len; k += kWave) {
+                    const uint32_t x = q[min(k + (int32_t)lane_id(), len - 1)];
+                    const uint64_t hit = ballot(min(value(x), x ^ oj) != 0u);
+                    if (hit) {
+                        const uint32_t f = readlane(x, ctz64(hit));
+                        rep = lane_id() == j ? f : rep;
+                        om = 0;
                     }
+                }
+            }
+        } else if (open) {
+            rep = find_watch<8>(larena + 8 * (uint32_t)r.z, r.w, other);
+        }
+        const bool move = rep != (uint32_t)kNone;
+        const bool no = open && !move && vo == 0, unit = open && !move && vo != 0;
+        const bool drop = move || dead;
+        if (drop) H::sub_l(&hdr[fl]);
+        if (move) {
+            const int32_t pos = H::add_l(&hdr[rep]);
+            I2 w;
+            w.x = (I)other;
+            w.y = (I)rep;
+            if (pos < slack) {
+                Wl[rep * slack + pos] = (I)e;
+            } else {
+                H::sub_l(&hdr[rep]);
+                w.x = w.y = kNone;
+            }
+            *(I2*)&lrec[e] = w;
+        }
+        const uint64_t dm = ballot(drop), km = ballot(in) & ~dm;
+        if ((dm || keep != i0) && in && !drop) Wl[base + keep + prefix_count(km)] = (I)e;
+        keep += popc64(km);
+        lsync();
+        const uint64_t cm = ballot(no), um = ballot(unit);
+        if (cm) confl = m + readlane(e, ctz64(cm));
+        else if (um) assign_units(um, other, e + m, confl);
+    }
+
+    // A learned entry's other watch; a detached clause (and a lane without an entry) gives the
+    // always-false literal, so that it counts as open.
+    __device__ __forceinline__ uint32_t learned_other(I4 r, uint32_t fl) const
+    {
+        return min((uint32_t)r.x + r.y - fl, 2u * (uint32_t)n);
+    }
+
+    // Propagation for lists of any length: 64 entries per step.
+    __device__ __forceinline__ int32_t propagate_long()
+    {
+        const uint32_t lane = lane_id();
+        int32_t confl = -1;
+        while (confl < 0 && qhead < tsize) {
+            const uint32_t fl = uniu(trail[qhead]) ^ 1u;
+            qhead++;
+            props++;
+            const HT h = hdr[fl];
+            const uint32_t ws = uniu(h.x), lb = fl * (uint32_t)slack;
+            const int32_t co = uni(H::no(h)), cl = uni(H::nl(h));
+            int32_t keep = 0;
+            for (int32_t i0 = 0; i0 < co; i0 += kWave) {
+                const uint32_t e = Wo[ws + min(i0 + (int32_t)lane, co - 1)];
+                step_original(fl, ws, i0, keep, i0 + (int32_t)lane < co, e, rec[e], confl);
+            }
+            keep = 0;
+            for (int32_t i0 = 0; i0 < cl; i0 += kWave) {
+                const uint32_t e = Wl[lb + min(i0 + (int32_t)lane, cl - 1)];
+                const I4 r = lrec[e];
+                const uint32_t other = learned_other(r, fl);
+                step_learned(fl, lb, i0, keep, i0 + (int32_t)lane < cl, e, r, other, value(other), confl);
+            }
+        }
+        return confl;
+    }
+
+    // Keeps a wave-uniform value in a vector register: what is computed from it stays on the
+    // vector side, where the loads that need it are.
+    static __device__ __forceinline__ uint32_t vec(uint32_t x)
+    {
+        asm("" : "+v"(x));
+        return x;
+    }
+
+    __device__ __forceinline__ int32_t propagate()
+    {
+        if (!shortl) return propagate_long();
+        if (qhead >= tsize) return -1;
+        const uint32_t lane = lane_id();
+        const uint32_t top = 2u * (uint32_t)n;   // (a lane without an entry reads clause 0, which need not hold fl)
+        int32_t confl = -1;
+        // the current literal (its negation fl), its lists (ws, co original entries; lb, cl
+        // learned) and their entries
+        do {
+            uint32_t fl = vec(trail[qhead]) ^ 1u;
+            HT h = hdr[fl];
+            uint32_t lb = fl * (uint32_t)slack;
+            bool fetched;
+            uint32_t eo = Wo[h.x + lane], el = Wl[lb + lane];
+            for (;;) {
+                qhead++;
+                props++;
+                const uint32_t ws = h.x;
+                const bool ino = lane < (uint32_t)H::no(h), inl = lane < (uint32_t)H::nl(h);
+                eo = ino ? eo : 0u;
+                el = inl ? el : 0u;
+                uint32_t fln = vec(trail[qhead]) ^ 1u;   // the next one, if one is queued
+                const I4 ro = rec[eo], rl = lrec[el];
+                HT hn = hdr[fln];
+                uint32_t lbn = fln * (uint32_t)slack;
+                uint32_t other, rep, vo, vq = 0;
+                if (ALL3) {
+                    rep = ro.w;
+                    other = min((uint32_t)ro.x + ro.y + ro.z - fl - rep, top);
+                    vq = value(rep);
+                    if (dups) vq = rep == other ? 0u : vq;
+                } else {
+                    other = min((uint32_t)ro.x + ro.y - fl, top);
+                }
+                vo = value(other);
+                const uint32_t lother = learned_other(rl, fl);
+                uint32_t vl = value(lother);
+                uint32_t eon = Wo[hn.x + lane], eln = Wl[lbn + lane];
+                vo = ino ? vo : 2u;
+                vl = inl ? vl : 2u;
+                // (decisions are single compares: a ballot of one goes straight to scalar
+                // registers, a ballot of a conjunction takes two vector operations more)
+                uint64_t ev;
+                if (ALL3) {
+                    const uint64_t mm = ballot((2u - vo) * vq != 0u);
+                    if (mm) {
+                        if ((mm >> lane) & 1) {
+                            const uint32_t at = (uint32_t)hdr[rep].x + H::add_o(&hdr[rep]);
+                            H::sub_o(&hdr[fl]);
+                            Wo[at] = (I)eo;
+                            rec[eo].w = (I)fl;
+                        } else if (ino) {
+                            Wo[ws + lane - prefix_count(mm)] = (I)eo;
+                        }
+                        lsync();
+                    }
+                    // a unit or falsified clause (vo < 2, vq false), or a learned clause not satisfied
+                    ev = ballot(min(vq | (vo & 2u), vl & 2u) == 0u);
+                } else {
+                    ev = ballot(min(vo, vl) < 2u);
+                }
+                int32_t queued = tsize;
+                if (ev) {
+                    if (ALL3) {
+                        const uint64_t cm = ballot((vq | vo) == 0u), um = ballot((vq << 2 | vo) == 1u);
+                        if (cm) confl = readlane(eo, ctz64(cm));
+                        else if (um) assign_units(um, other, eo, confl);
+                    } else if (ballot(vo < 2u)) {
+                        int32_t keep = 0;
+                        step_original(fl, ws, 0, keep, ino, eo, ro, confl);
+                    }
+                    if (confl < 0) {
+                        if (tsize != queued) {
+                            vl = value(lother);
+                            vl = inl ? vl : 2u;
+                            if (qhead >= queued) {
+                                // the first of the new ones is next: fetch its lists meanwhile
+                                fln = vec(trail[qhead]) ^ 1u;
+                                hn = hdr[fln];
+                                lbn = fln * (uint32_t)slack;
+                                eon = Wo[hn.x + lane];
+                                eln = Wl[lbn + lane];
+                                queued = tsize;
+                            }
+                        }
+                        if (ballot(vl < 2u)) {
+                            int32_t keep = 0;
+                            step_learned(fl, lb, 0, keep, inl, el, rl, lother, vl, confl);
+                        }
+                    }
+                }
+                fetched = qhead < queued;
+                if (confl >= 0 || !fetched) break;
+                fl = fln;
+                h = hn;
+                lb = lbn;
+                eo = eon;
+                el = eln;
+            }
+        } while (confl < 0 && qhead < tsize);
+        return confl;
+    }
+
+    __device__ __forceinline__ void backtrack(int32_t b, bool save_phase)
+    {
+        if (dl <= b) return;
+        const int32_t start = uni((int32_t)tlim[b + 1]);
+        for (int32_t t = start + lane_id(); t < tsize; t += kWave) {
+            const int32_t u = trail[t];
+            clear_value(u);
+            if (save_phase) phase[u >> 1] = (int8_t)(u & 1);
+        }
+        lsync();
+        tsize = start;
+        qhead = start;
+        dl = b;
+    }
+
+    __device__ __forceinline__ void bump_activity(int32_t v)
+    {
+        if (kMode == 4) act[v] += inc;
+        else __hip_atomic_fetch_add(&act[v], inc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        if (bumps) atomicAdd(&bumps[v], 1);
+    }
+
+    // Where the literals of clause c (uniform) are; ALL3 originals keep theirs in the record.
+    __device__ __forceinline__ const I* clause_lits(int32_t c, int32_t& len) const
+    {
+        if (c < m) {
+            const I4 r = rec[c];
+            len = uni((int32_t)r.w);
+            return olits + 4 * uni((int32_t)r.z);
+        }
+        const I4 r = lrec[c - m];
+        len = uni((int32_t)r.w);
+        return larena + 8 * uni((int32_t)r.z);
+    }
+
+    // Whether every literal of reason clause r is in the clause being learned (as the literal it
+    // is the reason of is) or a level-0 fact.
+    __device__ __forceinline__ bool implied(int32_t r) const
+    {
+        if (ALL3 && r < m) {
+            const I4 x = rec[r];
+            return min(min((uint32_t)vi[x.x >> 1].w, (uint32_t)vi[x.y >> 1].w), (uint32_t)vi[x.z >> 1].w) != 0u;
+        }
+        const I4 x = r < m ? rec[r] : lrec[r - m];
+        const I* lits = r < m ? olits + 4 * (int32_t)x.z : larena + 8 * (int32_t)x.z;
+        const int32_t len = x.w;
+        uint32_t all = 1;
+        for (int32_t k = 0; k < len && all; k += 4) {
+            const I4 q = *(const I4*)(lits + k);
+            const int32_t a = q.x >> 1, b = k + 1 < len ? q.y >> 1 : a, c = k + 2 < len ? q.z >> 1 : a,
+                          d = k + 3 < len ? q.w >> 1 : a;
+            all = min(min((uint32_t)vi[a].w, (uint32_t)vi[b].w), min((uint32_t)vi[c].w, (uint32_t)vi[d].w));
+        }
+        return all != 0u;
+    }
+
+    // Takes the literals q of lanes `take` (below the current level, not yet in it) into the
+    // clause being learned, in lane order.
+    __device__ __forceinline__ void take_lower(uint64_t take, int32_t q, int32_t& nl)
+    {
+        if ((take >> lane_id()) & 1) {
+            vi[q >> 1].w = 1;
+            bump_activity(q >> 1);
+            lbuf[nl + prefix_count(take)] = (I)q;
+        }
+        nl += popc64(take);
+        lsync();
+    }
+
+    // Of the lanes `m64`, the first of each variable (clauses that name one twice).
+    __device__ __forceinline__ uint64_t first_of_var(uint64_t m64, int32_t v) const
+    {
+        uint64_t keep = 0;
+        while (m64) {
+            const int j = ctz64(m64);
+            keep |= 1ull << j;
+            m64 &= ~ballot(v == readlane(v, j));
+        }
+        return keep;
+    }
+
+    // The resolution steps of analyze() when the current level's part of the trail fits the
+    // wavefront: lane i stands for trail entry tsize-1-i, a scalar mask holds the entries still to
+    // resolve, and the current level's literals never touch memory flags.  Returns the clause's
+    // length (-1: no literal of the current level, an internal error) and the asserting literal's
+    // negation p.
+    __device__ __forceinline__ int32_t resolve(int32_t confl, int32_t& p)
+    {
+        const int lane = lane_id();
+        const uint32_t end = (uint32_t)tsize - 1u;
+        const int32_t tl = trail[max((int32_t)end - lane, 0)];
+        const int32_t rs = vi[tl >> 1].y;
+        const uint32_t seg = (uint32_t)tsize - uniu(tlim[dl]);   // entries of the current level (<= 64)
+        uint64_t todo = 0, ever = 0, past = 0;
+        int32_t nl = 1, c = confl, j = 0;
+        do {
+            if (ALL3 && c < m) {
+                const I4 r = rec[c];
+                const int32_t q = lane == 0 ? r.x : lane == 1 ? r.y : r.z;
+                const I4 x = vi[q >> 1];
+                const uint32_t ra = end - (uint32_t)vi[r.x >> 1].z, rb = end - (uint32_t)vi[r.y >> 1].z,
+                               rc = end - (uint32_t)vi[r.z >> 1].z;
+                todo |= ballot((uint32_t)lane == ra) | ballot((uint32_t)lane == rb) | ballot((uint32_t)lane == rc);
+                // lanes past the clause, and those of the current level, are not lower
+                const uint32_t in = min((uint32_t)(lane < 3 ? 1 : 0), end - (uint32_t)x.z < seg ? 0u : 1u);
+                uint64_t low = ballot(((uint32_t)x.w ^ 1u) * in == 1u);
+                if (low) {
+                    if (dups) low = first_of_var(low, q >> 1);
+                    take_lower(low, q, nl);
+                }
+            } else {
+                int32_t len;
+                const I* cl = clause_lits(c, len);
+                if (c >= m && lane == 0) lused[c - m] = 1;
+                for (int32_t k0 = 0; k0 < len; k0 += kWave) {
+                    const int32_t k = k0 + lane;
+                    // every lane reads (lanes past the clause re-read its last literal)
+                    const int32_t q = cl[min(k, len - 1)];
+                    const I4 x = vi[q >> 1];
+                    const uint32_t rq = end - (uint32_t)x.z;
+                    const bool cur = rq < seg;
+                    if (cur) mark[rq] = 1;
+                    uint64_t low = ballot(k < len && !cur && x.w == 0);
+                    if (low) {
+                        if (dups && c < m) low = first_of_var(low, q >> 1);
+                        take_lower(low, q, nl);
+                    }
+                }
+                lsync();
+                todo |= ballot(mark[lane] != 0);
+                mark[lane] = 0;
+                lsync();
+            }
+            todo &= ~0ull >> (64u - seg);
+            ever |= todo;
+            todo &= ~past;
+            j = ctz64(todo);
+            past |= todo & (~todo + 1);
+            past |= past - 1;
+            todo &= todo - 1;
+            c = readlane(rs, j);
+        } while (todo);
+        p = readlane(tl, j);
+        if ((ever >> lane) & 1) bump_activity(tl >> 1);
+        return ever ? nl : -1;
+    }
+
+    // The same for a current level of any length: flags on every literal met, the trail walked
+    // back 64 entries at a time.
+    __device__ __forceinline__ int32_t resolve_long(int32_t confl, int32_t& p)
+    {
+        const int lane = lane_id();
+        int32_t nl = 1, pathc = 0, c = confl;
+        int32_t wb = tsize - 1, off = 0;
+        int32_t tl = trail[max(wb - lane, 0)];
+        p = -1;
+        do {
+            int32_t len = 3;
+            const I* cl = nullptr;
+            I4 r3 = {};
+            if (ALL3 && c < m) r3 = rec[c];
+            else cl = clause_lits(c, len);
+            if (c >= m && lane == 0) lused[c - m] = 1;
+            for (int32_t k0 = 0; k0 < len; k0 += kWave) {
+                const int32_t k = k0 + lane;
+                int32_t q;
+                if (ALL3 && c < m) q = lane == 0 ? r3.x : lane == 1 ? r3.y : r3.z;
+                else q = cl[min(k, len - 1)];
+                const I4 x = vi[q >> 1];
+                uint64_t met = ballot(k < len && q != p && x.w == 0);
+                if (dups && c < m) met = first_of_var(met, q >> 1);
+                const uint64_t low = met & ~ballot((int32_t)x.x == dl);
+                if (((met & ~low) >> lane) & 1) {
+                    vi[q >> 1].w = 1;
+                    bump_activity(q >> 1);
+                }
+                pathc += popc64(met & ~low);
+                take_lower(low, q, nl);
+            }
+            // the next literal met of the current level, walking back
+            uint64_t hm = ballot(lane >= off && wb - lane >= 0 && vi[tl >> 1].w != 0);
+            while (hm == 0 && wb >= kWave) {
+                wb -= kWave;
+                off = 0;
+                tl = trail[max(wb - lane, 0)];
+                hm = ballot(wb - lane >= 0 && vi[tl >> 1].w != 0);
+            }
+            const int j = hm ? ctz64(hm) : 0;
+            off = j + 1;
+            p = readlane(tl, j);
+            c = uni((int32_t)vi[p >> 1].y);
+            if (lane == 0) vi[p >> 1].w = 0;
+            lsync();
+            pathc--;
+        } while (pathc > 0 && c != (int32_t)kNone);
+        return pathc > 0 ? -1 : nl;
+    }
+
+    // 1-UIP.  Leaves the learned clause in lbuf[0..len) with the asserting literal first and
+    // a literal of the backjump level second.
+    __device__ __forceinline__ int32_t analyze(int32_t confl, int32_t& bt, int32_t& lbd)
+    {
+        const int lane = lane_id();
+        int32_t p;
+        int32_t nl = tsize - uni((int32_t)tlim[dl]) <= kWave ? resolve(confl, p) : resolve_long(confl, p);
+        if (lane == 0) lbuf[0] = (I)(p ^ 1);
+        lsync();
+        // Local minimization: a literal whose reason's other literals are all in the clause (or at
+        // level 0) is implied by the rest and dropped.  First every literal is tested against the
+        // clause as learned (drops are marked, the vars' flags untouched), then the clause is
+        // compacted, so the result does not depend on lane order.  Dropping several at once is
+        // sound: resolving them out in reverse trail order only meets literals that stay in the
+        // clause or are resolved out earlier.
+        for (int32_t k = 1 + lane; k < nl; k += kWave) {
+            const int32_t q = lbuf[k];
+            const int32_t r = vi[q >> 1].y;
+            if (r != (int32_t)kNone && implied(r)) lbuf[k] = (I)(q | kDrop);
+        }
+        lsync();
+        // compaction, the vars' flags, backjump level = highest level among the other literals (the
+        // first literal of that level), LBD = distinct levels
+        stamp++;
+        int32_t kept = 1, distinct = 0, best = -1, bi = 0;
+        for (int32_t k0 = 1; k0 < nl; k0 += kWave) {
+            const int32_t k = k0 + lane;
+            const bool in = k < nl;
+            const int32_t x = lbuf[min(k, nl - 1)];
+            const int32_t q = x & (int32_t)(I)~kDrop;
+            const int32_t lvl = vi[q >> 1].x;
+            if (in) vi[q >> 1].w = 0;
+            const bool keep = in && !(x & (int32_t)kDrop);
+            const uint64_t km = ballot(keep);
+            bool first = false;
+            if (keep) first = atomicExch(&lstamp[lvl], stamp) != stamp;
+            lsync();
+            if (keep) lbuf[kept + prefix_count(km)] = (I)q;
+            distinct += popc64(ballot(first));
+            if (km) {
+                const int32_t top = (int32_t)uniu(wave_max_u32(keep ? (uint32_t)lvl + 1u : 0u)) - 1;
+                if (top > best) {
+                    best = top;
+                    bi = kept + popc64(km & ((1ull << ctz64(ballot(keep && lvl == top))) - 1ull));
+                }
+            }
+            kept += popc64(km);
+            lsync();
+        }
+        nl = kept;
+        lbd = distinct + 1;
+        bt = 0;
+        if (nl > 1) {
+            bt = best;
+            const I t1 = lbuf[1], tb = lbuf[bi];
+            lsync();
+            if (lane0()) {
+                lbuf[1] = tb;
+                lbuf[bi] = t1;
+            }
+        }
+        lsync();
+        return nl;
+    }
+
+    __device__ __forceinline__ bool room(int32_t len) const
+    {
+        return nlearnt < learnt_cap && larena_used + len <= larena_cap;
+    }
+
+    // Append lbuf[0..len) as a learned clause, not yet watched.  Returns its index.
+    __device__ __forceinline__ int32_t store_learned(int32_t len, int32_t lbd)
+    {
+        const int32_t id = nlearnt;
+        const int32_t full = (len + 7) & ~7;
+        for (int32_t k = lane_id(); k < full; k += kWave)
+            larena[8 * larena_top + k] = k < len ? lbuf[k] : (I)(2 * n);
+        if (lane0()) {
+            I4 r;
+            r.x = r.y = kNone;
+            r.z = (I)larena_top;
+            r.w = (I)len;
+            lrec[id] = r;
+            llbd[id] = (I)lbd;
+            lused[id] = 0;
+        }
+        nlearnt++;
+        larena_used += len;
+        larena_top += full >> 3;
+        learned++;
+        msync();
+        return id;
+    }
+
+    // Watch learned clause i on literals x and y (uniform); without room in both lists it stays
+    // detached.
+    __device__ __forceinline__ void watch_learned(int32_t i, int32_t x, int32_t y)
+    {
+        const HT hx = hdr[x], hy = hdr[y];
+        const int32_t px = uni(H::nl(hx)), py = uni(H::nl(hy)) + (x == y ? 1 : 0);
+        if (px < slack && py < slack) {
+            if (lane0()) {
+                I2 w;
+                w.x = (I)x;
+                w.y = (I)y;
+                *(I2*)&lrec[i] = w;
+                Wl[x * slack + px] = (I)i;
+                Wl[y * slack + py] = (I)i;
+                (void)H::add_l(&hdr[x]);
+                (void)H::add_l(&hdr[y]);
+            }
+        }
+        lsync();
+    }
+
+    // At level 0: attach learned clause i.  A clause satisfied at level 0 is dropped, a clause
+    // with one non-false literal asserts it, a falsified clause means the job is UNSAT (returns
+    // false).
+    __device__ __forceinline__ bool attach_level0(int32_t i)
+    {
+        const int lane = lane_id();
+        const I4 r = lrec[i];
+        const int32_t st = 8 * uni((int32_t)r.z), len = uni((int32_t)r.w);
+        int32_t nf0 = -1, nf1 = -1;
+        bool sat = false;
+        for (int32_t k0 = 0; k0 < len && nf1 < 0 && !sat; k0 += kWave) {
+            const int32_t k = k0 + lane;
+            const int32_t q = larena[st + min(k, len - 1)];
+            const uint32_t v = k < len ? value(q) : 0u;
+            if (ballot(v == 2)) sat = true;
+            uint64_t um = ballot(v == 1);
+            while (um && nf1 < 0) {
+                const int j = ctz64(um);
+                um &= um - 1;
+                const int32_t x = uni(readlane(q, j));
+                if (nf0 < 0) nf0 = x;
+                else nf1 = x;
+            }
+        }
+        bool ok = true;
+        if (!sat) {
+            if (nf0 < 0) ok = false;
+            else if (nf1 < 0) assign(nf0, kNone);
+            else watch_learned(i, nf0, nf1);
+        }
+        msync();
+        return ok;
+    }
+
+    // Reduce the learned DB at the current level.  Survivors: reasons of assigned literals
+    // (always), glue clauses (LBD <= 3) and, in mode 0, clauses used since the last
+    // reduction; mode 2 keeps the reasons only.  Clause ids are renumbered, reasons are
+    // remapped and the learned watch lists are rebuilt from the watch pairs, which keeps
+    // the two-watched-literal invariant at any level.
+    __device__ __forceinline__ void reduce_db(int mode)
+    {
+        const int lane = lane_id();
+        for (int32_t i = lane; i < nlearnt; i += kWave) remap[i] = 0;
+        msync();
+        for (int32_t t = lane; t < tsize; t += kWave) {
+            const I4 x = vi[trail[t] >> 1];
+            // level-0 reasons are never read
+            if (x.y != kNone && (int32_t)x.y >= m && x.x > 0) remap[(int32_t)x.y - m] = 1;
+        }
+        msync();
+        int32_t ns = 0;
+        for (int32_t i0 = 0; i0 < nlearnt; i0 += kWave) {
+            const int32_t i = i0 + lane;
+            const bool in = i < nlearnt;
+            const int32_t ic = min(i, nlearnt - 1);
+            const I4 r = lrec[ic];
+            const I lbd = llbd[ic];
+            const bool used = lused[ic] != 0, locked = remap[ic] != 0;
+            const bool del = r.x == kNone;
+            const bool wanted = mode == 0 ? (lbd <= 3 || used) : false;
+            const bool keep = in && (locked || (!del && wanted));
+            const uint64_t km = ballot(keep);
+            msync();
+            const int32_t ni = ns + prefix_count(km);
+            if (in) remap[i] = keep ? (I)ni : kNone;
+            if (keep) {
+                lrec[ni] = r;
+                llbd[ni] = lbd;
+                lused[ni] = 0;
+            }
+            ns += popc64(km);
+            msync();
+        }
+        // compact literals (forward copy; a destination never lies above its source)
+        int32_t top = 0, used = 0;
+        for (int32_t i = 0; i < ns; i++) {
+            const I4 r = lrec[i];
+            const int32_t st = uni((int32_t)r.z), len = uni((int32_t)r.w);
+            const int32_t full = (len + 7) & ~7;
+            if (st != top) {
+                for (int32_t k0 = 0; k0 < full; k0 += kWave) {
+                    const int32_t k = k0 + lane;
+                    const I x = larena[8 * st + min(k, full - 1)];
+                    msync();
+                    if (k < full) larena[8 * top + k] = x;
+                    msync();
+                }
+                if (lane0()) lrec[i].z = (I)top;
+            }
+            top += full >> 3;
+            used += len;
+        }
+        for (int32_t t = lane; t < tsize; t += kWave) {
+            const int32_t v = trail[t] >> 1;
+            const I r = vi[v].y;
+            if (r != kNone && (int32_t)r >= m) {
+                const I x = remap[(int32_t)r - m];
+                vi[v].y = x != kNone ? (I)(m + x) : kNone;
+            }
+        }
+        for (int32_t l = lane; l < 2 * n; l += kWave) H::set_l0(&hdr[l]);
+        msync();
+        for (int32_t i = lane; i < ns; i += kWave) {
+            const I2 w = *(const I2*)&lrec[i];
+            if (w.x == kNone) continue;
+            const int32_t wl[2] = {(int32_t)w.x, (int32_t)w.y};
+            for (int h = 0; h < 2; h++) {
+                const int32_t pos = H::add_l(&hdr[wl[h]]);
+                if (pos < slack) {
+                    Wl[wl[h] * slack + pos] = (I)i;
+                } else {
+                    H::sub_l(&hdr[wl[h]]);
+                    I2 none;
+                    none.x = none.y = kNone;
+                    *(I2*)&lrec[i] = none;
+                }
+            }
+        }
+        nlearnt = ns;
+        larena_used = used;
+        larena_top = top;
+        msync();
+    }
+
+    // The branching variable (-1: none free): highest activity, then the lower var (VSIDS), or
+    // the highest free var (the reference's last free var).
+    __device__ __forceinline__ int32_t pick_branch(int mode)
+    {
+        uint32_t best = 0;
+        int32_t bv = 0;
+        for (int32_t v = lane_id(); v < n; v += kWave) {
+            if (lv[2 * v] == 1) {
+                // non-negative floats order as integers
+                const uint32_t key = mode == 1 ? (uint32_t)v + 1u : (__float_as_uint(act[v]) | 0x80000000u);
+                if (key > best) {
+                    best = key;
+                    bv = v;
+                }
+            }
+        }
+        const uint32_t top = uniu(wave_max_u32(best));
+        if (top == 0) return -1;
+        const uint64_t tie = ballot(best == top);
+        const int j = ctz64(tie);
+        if ((tie & (tie - 1)) == 0) return uni(readlane(bv, j));
+        return (int32_t)~uniu(wave_max_u32(best == top ? ~(uint32_t)bv : 0u));
+    }
+
+    __device__ __forceinline__ void rescale_activity()
+    {
+        for (int32_t v = lane_id(); v < n; v += kWave) act[v] *= 1e-30f;
+        inc *= 1e-30f;
+        lsync();
+    }
+
+    // Build the per-instance part of a job: watch lists of the original clauses and the
+    // formula's unit clauses at level 0.  Returns false if the formula is falsified there.
+    __device__ __forceinline__ bool setup_instance(const SolveArgs& a, int32_t ins)
+    {
+        const int lane = lane_id();
+        const SolveOptsDev& o = a.o;
+        const InstMeta mi = a.meta[ins];
+        inst = ins;
+        n = uni(mi.n);
+        m = uni(mi.m);
+        const int32_t* lits = a.lits + mi.lit_base;
+        const int32_t* coff = a.coff + mi.coff_base;
+        const int32_t n2 = 2 * n;
+        const int64_t vb = a.var_base[ins];
+        slack = o.watch_slack;
+        learnt_cap = o.learnt_cap;
+        larena_cap = o.larena_cap;
+        dl = 0;
+        tsize = 0;
+        qhead = 0;
+        nlearnt = 0;
+        larena_used = 0;
+        larena_top = 0;
+        inc = 1.0f;
+        stamp = 0;
+        for (int32_t v = lane; v < n; v += kWave) {
+            act[v] = a.act_init ? a.act_init[vb + v] : 0.0f;
+            phase[v] = a.phase_init ? a.phase_init[vb + v] : (int8_t)o.phase_init;
+        }
+        for (int32_t v = lane; v < n + 2; v += kWave) lstamp[v] = 0;
+        for (int32_t t = lane; t < n + 1; t += kWave) trail[t] = 0;   // entries past the end are read ahead
+        if (lane == 0) lv[n2] = 0;
+        mark[lane] = 0;
+        for (int32_t l = lane; l < n2; l += kWave) {
+            lv[l] = 1;
+            hdr[l].x = 0u;
+            H::set(&hdr[l], 0, 0);
+        }
+        msync();
+        // occurrence counts give the capacity of every original-clause watch list
+        const int32_t L = uni(coff[m]);
+        for (int32_t k = lane; k < L; k += kWave) atomicAdd(&hdr[lits[k]].x, 1u);
+        msync();
+        int32_t carry = 0;
+        bool longl = slack > kWave;
+        for (int32_t l0 = 0; l0 < n2; l0 += kWave) {
+            const int32_t l = l0 + lane;
+            const int32_t x = l < n2 ? (int32_t)hdr[min(l, n2 - 1)].x : 0;
+            longl |= x > kWave;
+            const int32_t s = wave_inclusive_scan(x);
+            if (l < n2) hdr[l].x = (uint32_t)(carry + s - x);
+            carry += readlane(s, 63);
+        }
+        msync();
+        // watch the first two distinct literals of every clause; units and empty clauses at level 0
+        bool unsat = false, twice = false;
+        int32_t top = 0;
+        for (int32_t c0 = 0; c0 < m && !unsat; c0 += kWave) {
+            const int32_t c = c0 + lane;
+            int32_t len = -1, l0 = -1, l1 = -1;
+            int32_t b = 0, full = 0;
+            if (c < m) {
+                b = ALL3 ? 3 * c : coff[c];
+                full = ALL3 ? 3 : coff[c + 1] - b;
+                len = full;
+            }
+            int32_t start = 0;
+            if (!ALL3) {
+                const int32_t quads = (full + 3) >> 2;
+                const int32_t s = wave_inclusive_scan(quads);
+                start = top + s - quads;
+                top += readlane(s, 63);
+            }
+            if (len >= 1) {
+                l0 = lits[b];
+                // the two watches are distinct literals; a clause repeating one literal is a unit
+                if (ALL3) {
+                    const int32_t y = lits[b + 1], z = lits[b + 2];
+                    const int32_t rest = y != l0 ? z : y;
+                    if (y != l0) l1 = y;
+                    else if (z != l0) l1 = z;
+                    twice |= (y >> 1) == (l0 >> 1) || (z >> 1) == (l0 >> 1) || (y >> 1) == (z >> 1);
+                    I4 r;
+                    r.x = (I)l0;
+                    r.y = (I)y;
+                    r.z = (I)z;
+                    r.w = (I)rest;
+                    rec[c] = r;
+                } else {
+                    for (int32_t k = 0; k < full; k++) {
+                        const int32_t q = lits[b + k];
+                        olits[4 * start + k] = (I)q;
+                        if (l1 < 0 && q != l0) l1 = q;
+                        if (full <= 8)
+                            for (int32_t j = 0; j < k; j++) twice |= (lits[b + j] >> 1) == (q >> 1);
+                    }
+                    for (int32_t k = full; k & 3; k++) olits[4 * start + k] = (I)n2;
+                    I4 r;
+                    r.x = (I)l0;
+                    r.y = (I)l1;
+                    r.z = (I)start;
+                    r.w = (I)full;
+                    rec[c] = r;
                 }
                 if (l1 >= 0) {
                     len = 2;
-                    J.wpair[2 * c] = l0;
-                    J.wpair[2 * c + 1] = l1;
-                    J.Wo[J.wstart[l0] + atomicAdd(&J.wcnt_o[l0], 1)] = c;
-                    J.Wo[J.wstart[l1] + atomicAdd(&J.wcnt_o[l1], 1)] = c;
+                    Wo[(int32_t)hdr[l0].x + H::add_o(&hdr[l0])] = (I)c;
+                    Wo[(int32_t)hdr[l1].x + H::add_o(&hdr[l1])] = (I)c;
                 } else {
                     len = 1;
                 }
             }
-        }
-        if (ballot(len == 0)) unsat = true;
-        uint64_t um = ballot(len == 1);
-        while (um && !unsat) {
-            const int j = ctz64(um);
-            um &= um - 1;
-            const int32_t u = uni(readlane(l0, j));
-            const int8_t val = J.lv[u];
-            if (val == -1) unsat = true;
-            else if (val == 0) assign(J, u, -1);
-        }
-    }
-    J.base_trail = J.tsize;
-    wave_mem_sync();
-    return !unsat;
-}
-
-// Next cube of the instance already set up on this wavefront: undo everything above the
-// formula's unit clauses and forget the learned clauses (they may rest on the previous
-// cube).  Every remaining watch pair is repaired by propagating the units again from the
-// start of the trail.  Activities and saved phases carry over.
-__device__ void reset_instance(Ctx& J)
-{
-    const int lane = lane_id();
-    for (int32_t t = J.base_trail + lane; t < J.tsize; t += kWave) {
-        const int32_t u = J.trail[t];
-        J.lv[u] = 0;
-        J.lv[u ^ 1] = 0;
-        J.reason[u >> 1] = -1;
-    }
-    for (int32_t l = lane; l < 2 * J.n; l += kWave) J.wcnt_l[l] = 0;
-    for (int32_t v = lane; v < J.n; v += kWave) J.bumps[v] = 0;
-    wave_mem_sync();
-    J.tsize = J.base_trail;
-    J.qhead = 0;
-    J.dl = 0;
-    J.nlearnt = 0;
-    J.larena_used = 0;
-}
-
-// Telemetry: charge the time since the last switch to the current phase and enter
-// `next`.  The counters are the job's JS_PH_* fields, added to without waiting.
-__device__ __forceinline__ void phase(Ctx& J, int32_t next)
-{
-    if (!J.ph_out) return;
-    const uint64_t now = wall_clock64();
-    if (lane_id() == 0) atomicAdd(&J.ph_out[J.ph_cur], (unsigned long long)(now - J.ph_t));
-    J.ph_t = now;
-    J.ph_cur = next;
-}
-
-// Adds the conflicts of this job not yet reported to its instance's pool; returns the
-// pool's new total (wave-uniform).
-__device__ int64_t report_conflicts(Ctx& J, const SolveArgs& a, int32_t inst)
-{
-    unsigned long long tot = 0;
-    const unsigned long long delta = (unsigned long long)(J.conflicts - J.conf_reported);
-    if (lane_id() == 0) tot = atomicAdd(&a.inst_conf[inst], delta) + delta;
-    J.conf_reported = J.conflicts;
-    return (int64_t)__shfl(tot, 0);
-}
-
-// Testing aid: append the job's held learned clauses and its level-0 literals (as unit
-// clauses) to the dump as one block [inst, slots, then per clause its literals and -1].  The
-// block's space is reserved only if all of it fits, so the dump stays parseable.
-__device__ void dump_learned(Ctx& J, const SolveArgs& a, int32_t inst)
-{
-    const int lane = lane_id();
-    int32_t s = 0;
-    for (int32_t i = lane; i < J.nlearnt; i += kWave) s += J.lmeta[4 * i + 1] + 1;
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    const int32_t n0 = J.dl > 0 ? uni(J.tlim[1]) : J.tsize;   // level-0 part of the trail
-    const int64_t slots = (int64_t)uni(s) + 2 * (int64_t)n0;
-    const unsigned long long total = (unsigned long long)(slots + 2);
-    long long base = -1;
-    if (lane == 0) {
-        atomicAdd(a.learned_need, total);
-        unsigned long long old = __hip_atomic_load(a.learned_pos, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        while (old + total <= (unsigned long long)a.learned_cap) {
-            const unsigned long long prev = atomicCAS(a.learned_pos, old, old + total);
-            if (prev == old) {
-                base = (long long)old;
-                break;
-            }
-            old = prev;
-        }
-    }
-    base = __shfl(base, 0);
-    if (base < 0) return;
-    int32_t* out = a.learned_out + base;
-    if (lane == 0) {
-        out[0] = inst;
-        out[1] = (int32_t)slots;
-    }
-    int64_t p = 2;
-    for (int32_t i = 0; i < J.nlearnt; i++) {
-        const int32_t st = uni(J.lmeta[4 * i]), len = uni(J.lmeta[4 * i + 1]);
-        for (int32_t k = lane; k < len; k += kWave) out[p + k] = J.larena[st + k];
-        if (lane == 0) out[p + len] = -1;
-        p += len + 1;
-    }
-    for (int32_t t = lane; t < n0; t += kWave) {
-        out[p + 2 * t] = J.trail[t];
-        out[p + 2 * t + 1] = -1;
-    }
-}
-
-// Returns the job verdict: 0 SAT, 1 UNSAT, 2 UNDEF (budget), 3 skipped (instance decided).
-// deadline: wall-clock tick after which the job stops as UNDEF (0: none).
-__device__ int32_t run_job(Ctx& J, const SolveArgs& a, const JobDesc& jd, int64_t max_conflicts, uint64_t deadline)
-{
-    const SolveOptsDev& o = a.o;
-    J.conflicts = J.decisions = J.props = J.learned = J.restarts = 0;
-    J.levelmax = 0;
-    J.ran = false;
-    J.conf_reported = 0;
-    if (load_status(&a.inst_status[jd.inst]) != 2) return 3;
-    if (o.inst_conflicts > 0 && (int64_t)__atomic_load_n(&a.inst_conf[jd.inst], __ATOMIC_RELAXED) >= o.inst_conflicts)
-        return 2;
-    const uint64_t t_start = wall_clock64();
-    J.ph_t = t_start;
-    J.ph_cur = PH_SETUP;
-    if (J.setup_inst == jd.inst) {
-        reset_instance(J);
-    } else {
-        J.setup_ok = setup_instance(J, a, jd.inst);
-        J.setup_inst = jd.inst;
-    }
-    J.ran = true;
-    if (!J.setup_ok) return 1;
-    const int32_t m = J.m;
-    bool unsat = false;
-    // the cube's literals are facts of this job
-    for (int32_t k = 0; k < jd.cube_len && !unsat; k++) {
-        const int32_t u = uni(a.cube_lits[jd.cube_off + k]);
-        const int8_t val = J.lv[u];
-        if (val == -1) unsat = true;
-        else if (val == 0) assign(J, u, -1);
-    }
-    wave_mem_sync();
-    if (unsat) return 1;
-    phase(J, PH_BCP);
-    if (propagate(J) >= 0) return 1;
-
-    int32_t restart_thr = o.restart_first, restart_cnt = 0;
-    const float decay_inv = 1.0f / o.var_decay;
-    for (;;) {
-        phase(J, PH_BCP);
-        const int32_t confl = propagate(J);
-        if (confl >= 0) {
-            phase(J, PH_ANALYZE);
-            J.conflicts++;
-            restart_cnt++;
-            if (J.dl == 0) return 1;
-            int32_t bt, lbd;
-            const int32_t nl = analyze(J, confl, bt, lbd);
-            if (nl < 0) return 4;
-            phase(J, PH_BACKTRACK);
-            if (nl == 1) {
-                backtrack(J, 0, o.decision_mode == 0);
-                assign(J, uni(J.lbuf[0]), -1);
-            } else {
-                backtrack(J, bt, o.decision_mode == 0);
-                phase(J, PH_ANALYZE);
-                if (!(J.nlearnt < J.learnt_cap && J.larena_used + nl <= J.larena_cap)) {
-                    reduce_db(J, 0);
-                    if (!(J.nlearnt < J.learnt_cap && J.larena_used + nl <= J.larena_cap)) reduce_db(J, 2);
-                }
-                if (J.nlearnt < J.learnt_cap && J.larena_used + nl <= J.larena_cap) {
-                    const int32_t cid = store_learned(J, nl, lbd);
-                    wave_mem_sync();
-                    watch_learned(J, cid, uni(J.lbuf[0]), uni(J.lbuf[1]));
-                    assign(J, uni(J.lbuf[0]), cid);
-                } else {
-                    // every held clause is a reason: restart, then add the clause at level 0
-                    backtrack(J, 0, o.decision_mode == 0);
-                    J.restarts++;
-                    restart_cnt = 0;
-                    reduce_db(J, 2);
-                    const int32_t cid = store_learned(J, nl, lbd);
-                    wave_mem_sync();
-                    if (!attach_level0(J, cid - m)) return 1;
+            if (ballot(len == 0)) unsat = true;
+            uint64_t um = ballot(len == 1);
+            if (!ALL3) {
+                // a longer clause's variables, a lane each: its stamp shows one met before
+                uint64_t big = ballot(full > 8);
+                while (big) {
+                    const int j = ctz64(big);
+                    big &= big - 1;
+                    const int32_t e = uni(readlane(full, j)), at = uni(readlane(b, j));
+                    for (int32_t k = lane; k < e; k += kWave)
+                        twice |= atomicExch(&lstamp[lits[at + k] >> 1], c0 + j + 1) == c0 + j + 1;
+                    lsync();
                 }
             }
-            wave_mem_sync();
-            J.inc *= decay_inv;
-            if (J.inc > 1e30f) rescale_activity(J);
-            if (max_conflicts > 0 && J.conflicts >= max_conflicts) return 2;
-            if ((J.conflicts & 63) == 0) {
-                const uint64_t now = wall_clock64();
-                if (o.max_ticks > 0 && (int64_t)(now - t_start) > o.max_ticks) return 2;
-                if (deadline && now > deadline) return 2;
-                if (o.inst_conflicts > 0 && report_conflicts(J, a, jd.inst) >= o.inst_conflicts) return 2;
+            while (um && !unsat) {
+                const int j = ctz64(um);
+                um &= um - 1;
+                const int32_t u = uni(readlane(l0, j));
+                const uint32_t val = uniu(value(u));
+                if (val == 0) unsat = true;
+                else if (val == 1) assign(u, kNone);
             }
+        }
+        if (m == 0) {
+            I4 none;
+            none.x = none.y = none.z = none.w = 0;
+            rec[0] = none;
+        }
+        dups = ballot(twice) != 0;
+        shortl = ballot(longl) == 0;
+        if (!ALL3)
+            for (int32_t v = lane; v < n + 2; v += kWave) lstamp[v] = 0;
+        base_trail = tsize;
+        msync();
+        return !unsat;
+    }
+
+    // Next cube of the instance already set up on this wavefront: undo everything above the
+    // formula's unit clauses and forget the learned clauses (they may rest on the previous
+    // cube).  Every remaining watch pair is repaired by propagating the units again from the
+    // start of the trail.  Activities and saved phases carry over.
+    __device__ __forceinline__ void reset_instance()
+    {
+        const int lane = lane_id();
+        for (int32_t t = base_trail + lane; t < tsize; t += kWave) clear_value(trail[t]);
+        for (int32_t l = lane; l < 2 * n; l += kWave) H::set_l0(&hdr[l]);
+        msync();
+        tsize = base_trail;
+        qhead = 0;
+        dl = 0;
+        nlearnt = 0;
+        larena_used = 0;
+        larena_top = 0;
+    }
+
+    // Telemetry: charge the time since the last switch to the current phase and enter
+    // `next`.  The counters are the job's JS_PH_* fields, added to without waiting.
+    __device__ __forceinline__ void enter(int32_t next)
+    {
+        if (!ph_out) return;
+        const uint64_t now = wall_clock64();
+        if (lane0()) atomicAdd(&ph_out[ph_cur], (unsigned long long)(now - ph_t));
+        ph_t = now;
+        ph_cur = next;
+    }
+
+    // Adds the conflicts of this job not yet reported to its instance's pool; returns the
+    // pool's new total (wave-uniform).
+    __device__ __forceinline__ int64_t report_conflicts(const SolveArgs& a, int32_t ins)
+    {
+        unsigned long long tot = 0;
+        const unsigned long long delta = (unsigned long long)(conflicts - conf_reported);
+        if (lane0()) tot = atomicAdd(&a.inst_conf[ins], delta) + delta;
+        conf_reported = conflicts;
+        return (int64_t)lane0_u64(tot);
+    }
+
+    // Testing aid: append the job's held learned clauses and its level-0 literals (as unit
+    // clauses) to the dump as one block [inst, slots, then per clause its literals and -1].  The
+    // block's space is reserved only if all of it fits, so the dump stays parseable.
+    __device__ __forceinline__ void dump_learned(const SolveArgs& a, int32_t ins)
+    {
+        const int lane = lane_id();
+        const int32_t n0 = dl > 0 ? uni((int32_t)tlim[1]) : tsize;   // level-0 part of the trail
+        const int64_t slots = (int64_t)larena_used + nlearnt + 2 * (int64_t)n0;
+        const unsigned long long total = (unsigned long long)(slots + 2);
+        long long base = -1;
+        if (lane == 0) {
+            atomicAdd(a.learned_need, total);
+            unsigned long long old = __hip_atomic_load(a.learned_pos, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            while (old + total <= (unsigned long long)a.learned_cap) {
+                const unsigned long long prev = atomicCAS(a.learned_pos, old, old + total);
+                if (prev == old) {
+                    base = (long long)old;
+                    break;
+                }
+                old = prev;
+            }
+        }
+        base = (long long)lane0_u64((uint64_t)base);
+        if (base < 0) return;
+        int32_t* out = a.learned_out + base;
+        if (lane == 0) {
+            out[0] = ins;
+            out[1] = (int32_t)slots;
+        }
+        int64_t p = 2;
+        for (int32_t i = 0; i < nlearnt; i++) {
+            const I4 r = lrec[i];
+            const int32_t st = 8 * uni((int32_t)r.z), len = uni((int32_t)r.w);
+            for (int32_t k = lane; k < len; k += kWave) out[p + k] = (int32_t)larena[st + k];
+            if (lane == 0) out[p + len] = -1;
+            p += len + 1;
+        }
+        for (int32_t t = lane; t < n0; t += kWave) {
+            out[p + 2 * t] = (int32_t)trail[t];
+            out[p + 2 * t + 1] = -1;
+        }
+    }
+
+    // Returns the job verdict: 0 SAT, 1 UNSAT, 2 UNDEF (budget), 3 skipped (instance decided).
+    // deadline: wall-clock tick after which the job stops as UNDEF (0: none).
+    __device__ __forceinline__ int32_t run_job(const SolveArgs& a, const JobDesc& jd, int64_t max_conflicts,
+                                               uint64_t deadline)
+    {
+        const SolveOptsDev& o = a.o;
+        ran = false;
+        conf_reported = 0;
+        if (load_status(&a.inst_status[jd.inst]) != 2) return 3;
+        if (o.inst_conflicts > 0 &&
+            (int64_t)__atomic_load_n(&a.inst_conf[jd.inst], __ATOMIC_RELAXED) >= o.inst_conflicts)
+            return 2;
+        const uint64_t t_start = wall_clock64();
+        ph_t = t_start;
+        ph_cur = PH_SETUP;
+        bumps = a.var_bumps ? a.var_bumps + a.var_base[jd.inst] : nullptr;
+        if (setup_inst == jd.inst) {
+            reset_instance();
         } else {
-            if (restart_cnt >= restart_thr) {
-                phase(J, PH_BACKTRACK);
-                restart_thr = (int32_t)((float)restart_thr * o.restart_factor);
-                restart_cnt = 0;
-                backtrack(J, 0, o.decision_mode == 0);
-                J.restarts++;
-                if (load_status(&a.inst_status[jd.inst]) != 2) return 3;
-                if (J.nlearnt * 2 >= J.learnt_cap || J.larena_used * 2 >= J.larena_cap) reduce_db(J, 0);
-                continue;
+            setup_ok = setup_instance(a, jd.inst);
+            setup_inst = jd.inst;
+        }
+        ran = true;
+        if (!setup_ok) return 1;
+        bool unsat = false;
+        // the cube's literals are facts of this job
+        for (int32_t k = 0; k < jd.cube_len && !unsat; k++) {
+            const int32_t u = uni(a.cube_lits[jd.cube_off + k]);
+            const uint32_t val = uniu(value(u));
+            if (val == 0) unsat = true;
+            else if (val == 1) assign(u, kNone);
+        }
+        if (unsat) return 1;
+
+        int32_t restart_thr = o.restart_first, restart_cnt = 0;
+        const float decay_inv = 1.0f / o.var_decay;
+        for (;;) {
+            enter(PH_BCP);
+            const int32_t confl = propagate();
+            if (confl >= 0) {
+                // a conflict among the formula's units and the cube counts as none of the search's
+                if (dl == 0 && decisions == 0) return 1;
+                enter(PH_ANALYZE);
+                conflicts++;
+                restart_cnt++;
+                if (dl == 0) return 1;
+                int32_t bt, lbd;
+                const int32_t nl = analyze(confl, bt, lbd);
+                if (nl < 0) return 4;
+                enter(PH_BACKTRACK);
+                const int32_t first = uni((int32_t)lbuf[0]);
+                if (nl == 1) {
+                    backtrack(0, o.decision_mode == 0);
+                    assign(first, kNone);
+                } else {
+                    backtrack(bt, o.decision_mode == 0);
+                    enter(PH_ANALYZE);
+                    if (!room(nl)) {
+                        reduce_db(0);
+                        if (!room(nl)) reduce_db(2);
+                    }
+                    const bool fits = room(nl);
+                    if (!fits) {
+                        // every held clause is a reason: restart, then add the clause at level 0
+                        backtrack(0, o.decision_mode == 0);
+                        restarts++;
+                        restart_cnt = 0;
+                        reduce_db(2);
+                    }
+                    const int32_t id = store_learned(nl, lbd);
+                    if (fits) {
+                        watch_learned(id, first, uni((int32_t)lbuf[1]));
+                        assign(first, (I)(m + id));
+                    } else if (!attach_level0(id)) {
+                        return 1;
+                    }
+                }
+                inc *= decay_inv;
+                if (inc > 1e30f) rescale_activity();
+                if (max_conflicts > 0 && conflicts >= max_conflicts) return 2;
+                if ((conflicts & 63) == 0) {
+                    const uint64_t now = wall_clock64();
+                    if (o.max_ticks > 0 && (int64_t)(now - t_start) > o.max_ticks) return 2;
+                    if (deadline && now > deadline) return 2;
+                    if (o.inst_conflicts > 0 && report_conflicts(a, jd.inst) >= o.inst_conflicts) return 2;
+                }
+            } else {
+                if (restart_cnt >= restart_thr) {
+                    enter(PH_BACKTRACK);
+                    restart_thr = (int32_t)((float)restart_thr * o.restart_factor);
+                    restart_cnt = 0;
+                    backtrack(0, o.decision_mode == 0);
+                    restarts++;
+                    if (load_status(&a.inst_status[jd.inst]) != 2) return 3;
+                    if (nlearnt * 2 >= learnt_cap || larena_used * 2 >= larena_cap) reduce_db(0);
+                    continue;
+                }
+                enter(PH_DECIDE);
+                const int32_t v = pick_branch(o.decision_mode);
+                if (v < 0) return 0;
+                decisions++;
+                if (o.max_decisions > 0 && decisions > o.max_decisions) return 2;
+                if ((decisions & 1023) == 0) {
+                    if (load_status(&a.inst_status[jd.inst]) != 2) return 3;
+                    const uint64_t now = wall_clock64();
+                    if (o.max_ticks > 0 && (int64_t)(now - t_start) > o.max_ticks) return 2;
+                    if (deadline && now > deadline) return 2;
+                }
+                dl++;
+                if (dl > levelmax) levelmax = dl;
+                if (lane0()) tlim[dl] = (I)tsize;
+                const int32_t ph = o.decision_mode == 1 ? 1 : uni((int32_t)phase[v]);
+                assign(2 * v + ph, kNone);
             }
-            phase(J, PH_DECIDE);
-            const int32_t v = pick_branch(J, o.decision_mode);
-            if (v < 0) return 0;
-            J.decisions++;
-            if (o.max_decisions > 0 && J.decisions > o.max_decisions) return 2;
-            if ((J.decisions & 1023) == 0) {
-                if (load_status(&a.inst_status[jd.inst]) != 2) return 3;
-                const uint64_t now = wall_clock64();
-                if (o.max_ticks > 0 && (int64_t)(now - t_start) > o.max_ticks) return 2;
-                if (deadline && now > deadline) return 2;
-            }
-            J.dl++;
-            if (J.dl > J.levelmax) J.levelmax = J.dl;
-            J.tlim[J.dl] = J.tsize;
-            const int32_t ph = o.decision_mode == 1 ? 1 : (int32_t)J.phase[v];
-            assign(J, 2 * v + ph, -1);
         }
     }
-}
+};
 
 }  // namespace
 
-// kMode: where a job's state sits -- 1 all in LDS, 2 the per-var state in LDS and the
-// clause part in this wavefront's slice of the HBM workspace, 3 the per-var state and the
-// watch lists and watch pairs of the original clauses in LDS (read on every propagation
-// step), the learned clauses' lists, pairs, metadata and literals in HBM, 4 everything in
-// the HBM slice (formulas whose per-var state does not fit a workgroup's LDS).
-template <int kMode>
-__global__ __launch_bounds__(kSolveWavesPerBlock * kWave) __attribute__((amdgpu_waves_per_eu(kSolveWavesPerEu, kSolveWavesPerEu)))
+// kMode: where a job's state sits -- 1 all in LDS; 2 the per-var state in LDS, the watch
+// structures and the learned literals in this wavefront's slice of the HBM workspace; 3 the
+// per-var state and the watch structures (read on every propagation step) in LDS, the learned
+// literals in HBM; 4 everything in the HBM slice (formulas whose per-var state does not fit a
+// workgroup's LDS).
+template <int kMode, class I, bool ALL3>
+__global__ __launch_bounds__(kSolveWavesPerBlock * kWave) __attribute__((amdgpu_waves_per_eu(solve_waves_per_eu(kMode), solve_waves_per_eu(kMode))))
 void k_solve(SolveArgs a)
 {
     extern __shared__ __align__(16) char smem_all[];
@@ -1025,26 +1381,17 @@ void k_solve(SolveArgs a)
     // wave-level ordering only)
     const int wslot = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const int64_t gwave = (int64_t)blockIdx.x * (blockDim.x / kWave) + wslot;
-    char* smem = smem_all + (size_t)wslot * a.lds_per_wave;
-    Ctx J;
-    int32_t* cpart;
-    if (kMode == 4) {
-        char* slice = (char*)(a.ws + gwave * a.ws_ints_per_wave);
-        carve_state(J, slice, a.max_n);
-        cpart = (int32_t*)(slice + Layout::state_bytes(a.max_n));
-    } else {
-        carve_state(J, smem, a.max_n);
-        cpart = kMode == 1 ? (int32_t*)(smem + Layout::state_bytes(a.max_n)) : a.ws + gwave * a.ws_ints_per_wave;
-    }
-    carve_clauses(J, cpart, a);
-    if (kMode == 3) {
-        int32_t* l = (int32_t*)(smem + Layout::state_bytes(a.max_n));
-        J.Wo = l;
-        J.wpair = l + a.wo_cap;
-    }
+    char* smem = smem_all + (uint32_t)wslot * (uint32_t)a.lds_per_wave;
+    char* slice = (char*)(a.ws + gwave * a.ws_ints_per_wave);
+    Search<kMode, I, ALL3> J;
+    if (kMode == 4) J.carve(slice, slice + a.lay.state_bytes, slice + a.lay.state_bytes + a.lay.watch_bytes, a);
+    else if (kMode == 2) J.carve(smem, slice, slice + a.lay.watch_bytes, a);
+    else if (kMode == 3) J.carve(smem, smem + a.lay.state_bytes, slice, a);
+    else J.carve(smem, smem + a.lay.state_bytes, smem + a.lay.state_bytes + a.lay.watch_bytes, a);
     J.setup_inst = -1;
     J.setup_ok = false;
     J.n = 0;
+    J.dl = J.tsize = 0;
     int32_t n_jobs = a.n_jobs;
     const int32_t* order = nullptr;
     int64_t budget = a.o.max_conflicts;
@@ -1063,7 +1410,7 @@ void k_solve(SolveArgs a)
             const unsigned long long old = atomicCAS(a.t_start, 0ull, now);
             t0 = old ? old : now;
         }
-        t0 = __shfl(t0, 0);
+        t0 = lane0_u64(t0);
         deadline = (uint64_t)t0 + (uint64_t)a.o.deadline_ticks;
     }
     int32_t j = 0, j_end = 0;
@@ -1072,7 +1419,7 @@ void k_solve(SolveArgs a)
             // grab the next chunk of consecutive jobs (cubes of one instance are adjacent)
             int32_t k = 0;
             if (lane == 0) k = atomicAdd(a.queue_head, 1);
-            k = uni(__shfl(k, 0));
+            k = uni(k);
             j = k * a.chunk;
             if (j >= n_jobs) break;
             j_end = min(j + a.chunk, n_jobs);
@@ -1096,17 +1443,17 @@ void k_solve(SolveArgs a)
             job_budget = min(budget, left);
         }
         const bool spent = a.epoch && a.o.max_conflicts > 0 && a.job_stats && job_budget <= 0;
-        const int32_t st = ((deadline && t_job > deadline) || spent) ? 2 : run_job(J, a, jd, job_budget, deadline);
-        phase(J, PH_SETUP);   // charge the last phase
+        const int32_t st = ((deadline && t_job > deadline) || spent) ? 2 : J.run_job(a, jd, job_budget, deadline);
+        J.enter(PH_SETUP);   // charge the last phase
         const uint64_t job_ticks = wall_clock64() - t_job;
-        wave_mem_sync();
+        J.msync();
         const int32_t inst = jd.inst;
-        if (a.o.inst_conflicts > 0 && J.ran) (void)report_conflicts(J, a, inst);
-        if (a.learned_out && J.ran && J.setup_ok) dump_learned(J, a, inst);
+        if (a.o.inst_conflicts > 0 && J.ran) (void)J.report_conflicts(a, inst);
+        if (a.learned_out && J.ran && J.setup_ok) J.dump_learned(a, inst);
         if (st == 0) {
             int32_t won = 0;
             if (lane == 0) won = atomicCAS(&a.inst_status[inst], 2, 0) == 2;
-            won = uni(__shfl(won, 0));
+            won = uni(won);
             if (won) {
                 const InstMeta mi = a.meta[inst];
                 const int32_t W = words_per_row(mi.n);
@@ -1114,7 +1461,7 @@ void k_solve(SolveArgs a)
                     uint32_t x = 0;
                     for (int b = 0; b < 32; b++) {
                         const int32_t l = 32 * w + b;
-                        if (l < 2 * mi.n && J.lv[l] == 1) x |= 1u << b;
+                        if (l < 2 * mi.n && J.lv[l] == 2) x |= 1u << b;
                     }
                     a.model_rows[mi.word_base + w] = x;
                 }
@@ -1135,13 +1482,6 @@ void k_solve(SolveArgs a)
                 }
             }
         }
-        // per-var state belongs to this job's instance only if the job set it up (a job
-        // skipped because its instance was decided, or because the deadline passed, did not)
-        if (a.var_bumps && J.ran) {
-            const int64_t vb = a.var_base[inst];
-            for (int32_t v = lane; v < J.n; v += kWave)
-                if (J.bumps[v]) atomicAdd(&a.var_bumps[vb + v], J.bumps[v]);
-        }
         if (a.job_stats && lane == 0) {
             int64_t* s = a.job_stats + (int64_t)jd.order * JS_COUNT;
             // counters add up over the epochs a job runs in
@@ -1154,7 +1494,7 @@ void k_solve(SolveArgs a)
             s[JS_LEVELMAX] = max(s[JS_LEVELMAX], (int64_t)J.levelmax);
             s[JS_TICKS] += (int64_t)job_ticks;
         }
-        wave_mem_sync();
+        J.msync();
     }
 }
 
@@ -1207,7 +1547,61 @@ hipError_t launch_epoch_end(const SolveArgs& a, int32_t* remaining, hipStream_t 
     return hipGetLastError();
 }
 
-size_t solve_state_lds_bytes(int32_t max_n) { return Layout::state_bytes(max_n); }
+// Byte offsets of a job's arrays for instances of up to max_n variables, max_m clauses and max_L
+// literals, with ids of id_bytes bytes.
+SolveLayout solve_layout(int32_t max_n, int32_t max_m, int64_t max_L, bool all3, int id_bytes, const SolveOptsDev& o)
+{
+    SolveLayout L{};
+    const int64_t n = max_n, I = id_bytes;
+    int64_t at = 0;
+    const auto take = [&](int64_t bytes) {
+        const int64_t p = at;
+        at = (at + bytes + 15) & ~(int64_t)15;
+        return p;
+    };
+    L.id_bytes = id_bytes;
+    L.lv = take(2 * n + 1);   // at the region's start: its address needs no addition
+    L.hdr = take(2 * n * (id_bytes == 2 ? 8 : 16));
+    L.vi = take(n * 4 * I);
+    L.act = take(n * 4);
+    L.lstamp = take((n + 2) * 4);
+    L.trail = take((n + 1) * I);
+    L.tlim = take((n + 2) * I);
+    L.lbuf = take((n + 1) * I);
+    L.phase = take(n);
+    L.mark = take(64);
+    L.state_bytes = at;
+    at = 0;
+    // a list is read by all 64 lanes, and clause 0 also where there is none
+    L.rec = take((int64_t)(max_m + 1) * 4 * I);
+    L.lrec = take((int64_t)o.learnt_cap * 4 * I);
+    L.wo = take((max_L + 64) * I);
+    L.wl = take((2 * n * o.watch_slack + 64) * I);
+    L.llbd = take(o.learnt_cap * I);
+    L.remap = take(o.learnt_cap * I);
+    L.lused = take(o.learnt_cap);
+    L.olits = take(all3 ? 0 : (max_L + 3 * (int64_t)max_m) * I);
+    L.watch_bytes = at;
+    L.arena_bytes = ((int64_t)o.larena_cap + 7 * (int64_t)o.learnt_cap) * I;
+    L.arena_bytes = (L.arena_bytes + 15) & ~(int64_t)15;
+    return L;
+}
+
+// 16-bit ids hold every literal (with a mark bit), clause id (with a none value), clause start in
+// units of 4 literals, clause length and list length of these sizes.
+bool solve_ids16(int32_t max_n, int32_t max_m, int64_t max_L, const SolveOptsDev& o)
+{
+    return max_n < 16000 && (int64_t)max_m + o.learnt_cap < 65000 && max_L + 3 * (int64_t)max_m < 4 * 65000 &&
+           max_L < 65000 * 4 && (int64_t)o.larena_cap + 7 * (int64_t)o.learnt_cap < 8 * 65000 && o.watch_slack < 65000;
+}
+
+template <bool ALL3>
+static void launch_mode(const SolveArgs& a, int mode, dim3 grid, dim3 block, size_t lds, hipStream_t st)
+{
+    if (mode == 1) hipLaunchKernelGGL((k_solve<1, uint16_t, ALL3>), grid, block, lds, st, a);
+    else if (mode == 3) hipLaunchKernelGGL((k_solve<3, uint16_t, ALL3>), grid, block, lds, st, a);
+    else hipLaunchKernelGGL((k_solve<2, uint16_t, ALL3>), grid, block, lds, st, a);
+}
 
 hipError_t launch_solve(const SolveArgs& a, int clause_mem, int waves, size_t lds_bytes, hipStream_t st)
 {
@@ -1215,14 +1609,16 @@ hipError_t launch_solve(const SolveArgs& a, int clause_mem, int waves, size_t ld
     const int wpb = solve_waves_per_block(lds_bytes);
     if (waves % wpb != 0 || (size_t)a.lds_per_wave != lds_bytes) return hipErrorInvalidValue;
     const dim3 grid(waves / wpb), block(kWave * wpb);
-    if (clause_mem == 1)
-        hipLaunchKernelGGL(k_solve<1>, grid, block, lds_bytes * wpb, st, a);
-    else if (clause_mem == 3)
-        hipLaunchKernelGGL(k_solve<3>, grid, block, lds_bytes * wpb, st, a);
-    else if (clause_mem == 4)
-        hipLaunchKernelGGL(k_solve<4>, grid, block, 0, st, a);
+    const size_t lds = lds_bytes * wpb;
+    const bool ids16 = a.lay.id_bytes == 2;
+    if (clause_mem == 4)
+        hipLaunchKernelGGL((k_solve<4, uint32_t, false>), grid, block, 0, st, a);
+    else if (!ids16)
+        hipLaunchKernelGGL((k_solve<2, uint32_t, false>), grid, block, lds, st, a);
+    else if (a.all3)
+        launch_mode<true>(a, clause_mem, grid, block, lds, st);
     else
-        hipLaunchKernelGGL(k_solve<2>, grid, block, lds_bytes * wpb, st, a);
+        launch_mode<false>(a, clause_mem, grid, block, lds, st);
     return hipGetLastError();
 }
 

@@ -10,9 +10,9 @@ namespace gpsat {
 // Solver options (the strategy surfaces of the reference's compile-time Configs.cuh,
 // chosen at run time here).
 // k_solve launch shape: independent wavefronts per workgroup, and the wavefronts per SIMD
-// the register allocation is held to (8 -> at most 64 VGPRs per lane)
-constexpr int kSolveWavesPerBlock = 4;
-constexpr int kSolveWavesPerEu = 8;
+// the register allocation is held to (8 -> at most 64 VGPRs per lane, 4 -> 128)
+constexpr int kSolveWavesPerBlock = 1;
+constexpr int solve_waves_per_eu(int mode) { return mode == 1 || mode == 3 ? 4 : 8; }
 
 struct SolveOptsDev {
     int32_t decision_mode;    // 0: VSIDS + phase saving; 1: reference scheme (last free var, positive)
@@ -44,6 +44,15 @@ enum JobStat {
     JS_PH_SETUP, JS_PH_BCP, JS_PH_ANALYZE, JS_PH_BACKTRACK, JS_PH_DECIDE, JS_COUNT
 };
 enum Phase { PH_SETUP = 0, PH_BCP, PH_ANALYZE, PH_BACKTRACK, PH_DECIDE, PH_COUNT };
+
+// Byte offsets of a job's arrays inside its state part, its watch part and its learned-literal
+// arena (see solve_layout and the fields of Search in solver.hip).
+struct SolveLayout {
+    int64_t hdr, vi, act, lstamp, trail, tlim, lbuf, lv, phase, mark, state_bytes;
+    int64_t rec, lrec, wo, wl, llbd, remap, lused, olits, watch_bytes;
+    int64_t arena_bytes;
+    int32_t id_bytes;               // 2 or 4
+};
 
 struct SolveArgs {
     const InstMeta* meta;
@@ -82,9 +91,7 @@ struct SolveArgs {
     int64_t learned_cap;
     unsigned long long* learned_pos;    // slots reserved by blocks that fit
     unsigned long long* learned_need;   // slots all blocks asked for
-    // per-wave clause-part layout (ints), identical in LDS and global mode
-    int32_t wo_cap, wl_cap, wpair_cap, lmeta_cap;
-    int32_t max_n;
+    SolveLayout lay;
     int32_t all3;                   // every original clause has 3 literals (clause c at lits + 3c)
     SolveOptsDev o;
 };
@@ -114,10 +121,11 @@ struct RefArgs {
 int64_t solve_ref_ws_ints(int32_t n, int32_t m, int32_t ecap);
 hipError_t launch_solve_ref(const RefArgs& a, hipStream_t st);
 
-size_t solve_state_lds_bytes(int32_t max_n);
+SolveLayout solve_layout(int32_t max_n, int32_t max_m, int64_t max_L, bool all3, int id_bytes, const SolveOptsDev& o);
+bool solve_ids16(int32_t max_n, int32_t max_m, int64_t max_L, const SolveOptsDev& o);
 
 // Launch plan of one solve (solve_plan in capi_solve.cpp): mode 1 all job state in LDS,
-// 2 clause part in HBM, 3 original clauses' watch structures in LDS and learned clauses in
+// 2 the clause part in HBM, 3 the watch structures in LDS and the learned literals in
 // HBM, 4 all in HBM; the persistent wavefronts, jobs per queue grab, and LDS per wavefront.
 struct SolvePlan {
     int mode;

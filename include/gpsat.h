@@ -196,13 +196,13 @@ typedef struct gpsat_solve_opts {
     float var_decay;         /* VSIDS decay per conflict */
     int32_t phase_init;      /* initial phase without a hint: 0 false, 1 true */
     double max_ms;           /* per-job wall-clock budget in ms (<= 0: none), exceeded -> UNDEF */
-    int32_t waves;           /* persistent wavefronts, rounded up to whole workgroups of 4
-                                (0: automatic, up to 32 per CU as LDS allows) */
-    int32_t clause_mem;      /* clause part of the job state: 0 automatic, 1 LDS, 2 HBM, 3 the
-                                original clauses' watch lists and pairs in LDS, the learned
-                                clauses' storage in HBM.  Automatic: with at most 4 jobs per CU,
-                                LDS, else split, else HBM, whichever fits first; with more, LDS
-                                when it takes at most 48 KB per wavefront, else HBM */
+    int32_t waves;           /* persistent wavefronts (0: automatic, up to 16 per CU, 32 with the
+                                clause part in HBM, as LDS allows) */
+    int32_t clause_mem;      /* clause part of the job state: 0 automatic, 1 LDS, 2 HBM, 3 the watch
+                                lists and clause records in LDS, the learned clauses' literals in
+                                HBM, 4 the whole job state in HBM.  Automatic: with at most 4 jobs
+                                per CU, LDS, else split, else HBM, whichever fits first; with more,
+                                whichever is estimated to finish the jobs first */
     int32_t verify;          /* 1: re-check every SAT model with the clause-evaluation kernel */
     int32_t chunk;           /* jobs per queue grab (0: automatic); cubes of one instance in one
                                 chunk reuse its watch lists on the wavefront */
@@ -235,7 +235,7 @@ typedef struct gpsat_solve_info {
     double kernel_ms;        /* solve kernel (HIP events on the batch stream) */
     double verify_ms;        /* model re-verification kernel */
     int32_t waves;
-    int32_t clause_mem;      /* 1 LDS, 2 HBM, 3 split (see gpsat_solve_opts) */
+    int32_t clause_mem;      /* 1 LDS, 2 HBM, 3 split, 4 all in HBM (see gpsat_solve_opts) */
     int64_t lds_bytes;       /* per wavefront */
     int64_t workspace_bytes;
     int32_t n_sat, n_unsat, n_undef, n_verified, n_errors;
