@@ -12,6 +12,13 @@
 // Aggregations, biases, the 2-output head, the loss and Adam are FP32.  Gradients and the
 // loss are summed from per-wavefront (or per-workgroup) partials in a fixed order, never
 // with floating-point atomics, so they are reproducible bit for bit.
+//
+// Each half round is one kernel per direction (gather, product and elementwise work on rows
+// held in registers), as memory traffic and its latency bound the network, not arithmetic: the 172
+// GFLOP of a training pass over 512 x (n=300, m=1278) would take 0.15 ms at half of the MFMA
+// peak, moving its rows of ~4.6 GB about 1 ms.  The pass takes 1.94 ms, where separate gather, product,
+// mask and reduction kernels moved ~9 GB in 3.70 ms; a layer's kernel runs at 3-4.3 TB/s of
+// compulsory bytes.
 #include <hip/hip_runtime.h>
 #include <string.h>
 
@@ -29,7 +36,6 @@ namespace gnn {
 
 constexpr int HID = 64;
 typedef uint16_t bf16_t;
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // parameter layout (FP32 master copy), in this order
@@ -47,92 +53,507 @@ __device__ __forceinline__ bf16_t to_bf16(float f)
 __device__ __forceinline__ float from_bf16(bf16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
 // ---------------------------------------------------------------------------------------
-// MFMA tiles.  v_mfma_f32_16x16x32_bf16 (gfx950) on a wave of 64: lane l supplies the 8
-// consecutive-k values A[l%16][8(l/16) .. 8(l/16)+7] and B[8(l/16) .. 8(l/16)+7][l%16] as one
-// 16-byte read each, and receives D[4(l/16)+j][l%16] (j = 0..3).  LDS tiles are stored
-// with the k index contiguous (transposed where the source is not), rows padded by 16 bytes
-// so the 16 rows a wave reads at once fall in different banks.
+// Fragments.  v_mfma_f32_16x16x32_bf16 (gfx950) on a wave of 64: lane l supplies the 8
+// consecutive-k values A[l%16][8(l/16) .. 8(l/16)+7] and B[8(l/16) .. 8(l/16)+7][l%16] and
+// receives D[4(l/16)+j][l%16] (j = 0..3).  Every product is computed transposed, weights as
+// A and node rows as B, so lane l = 16q + r works on row r of the wavefront's 16: of each 64
+// columns it supplies the 16 columns in(i) = 32 (i/8) + 8q + i%8 and receives the 16 columns
+// out(i) = 16 (i/4) + 4q + i%4, i = 0..15.  (The k index is in the order of the columns: with
+// another order the FP32 sums round differently, and a BF16 rounding after them now and then.)
+// Memory is read and written in another lane order with the same columns: lane 4r + q, so that
+// four neighbouring lanes share a row and a float4 access of theirs falls in one 128-byte line
+// (with the product's own lane order every lane of a quad is on another row, and the address
+// unit takes four times as long: it bounded the clause layer at 168 us where 134 MB were read
+// and 332 MB written).  Registers change order through ds_bpermute, rows in BF16 on the way in
+// and results in FP32 on the way out (to_product, from_product).  So a layer is gather -> BF16
+// -> MFMA -> ReLU -> store without a trip through memory.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ bf16x8 ld8(const bf16_t* p) { return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p)); }
+// (rows kept for the backward pass or the weight gradient: read again only after far more than
+// a cache's worth of other rows, so stored past the caches; clause layer 146 -> 130 us, literal
+// layer 123 -> 102 us at 654,336 clauses and 307,200 literals)
+__device__ __forceinline__ void st8(bf16_t* p, bf16x8 v)
+{
+    typedef int i32x4 __attribute__((ext_vector_type(4)));
+    __builtin_nontemporal_store(__builtin_bit_cast(i32x4, v), reinterpret_cast<i32x4*>(p));
+}
 __device__ __forceinline__ f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
-
-// out[N x 64] = relu(X[N x K] W[64 x K]^T + b); one wave per 16 rows, W staged in LDS.
-template <int K>
-__global__ __launch_bounds__(256) void k_dense_fwd(const bf16_t* __restrict__ X, const bf16_t* __restrict__ Wq,
-                                                   const float* __restrict__ bias, float* __restrict__ out, int N)
+// 8 floats rounded to nearest even (v_cvt_pk_bf16_f32)
+__device__ __forceinline__ bf16x8 pack8(const float* x)
 {
-    constexpr int SK = K + 8;
-    __shared__ __align__(16) bf16_t sW[64 * SK];
-    for (int i = threadIdx.x; i < 64 * K / 8; i += blockDim.x) {
-        const int r = (8 * i) / K, c = (8 * i) % K;
-        *reinterpret_cast<uint4*>(sW + r * SK + c) = reinterpret_cast<const uint4*>(Wq)[i];
+    bf16x8 v;
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = (__bf16)x[i];
+    return v;
+}
+// this lane's 16 values of a 64-wide FP32 row: the columns in(i), or out(i)
+template <bool OUT = false>
+__device__ __forceinline__ void ld_row(float (&x)[16], const float* row, int q)
+{
+    const float4* p = reinterpret_cast<const float4*>(row) + (OUT ? q : 2 * q);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const float4 v = p[OUT ? 4 * k : 8 * (k >> 1) + (k & 1)];
+        x[4 * k] = v.x;
+        x[4 * k + 1] = v.y;
+        x[4 * k + 2] = v.z;
+        x[4 * k + 3] = v.w;
     }
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r0 = (blockIdx.x * 4 + wave) * 16;
-    if (r0 >= N) return;
-    const int ar = r0 + (lane & 15), kq = 8 * (lane >> 4);
-    f32x4 acc[4];
+}
+__device__ __forceinline__ void st_row(float* row, const float (&x)[16], int q)   // columns out(i)
+{
+    float4* p = reinterpret_cast<float4*>(row + 4 * q);
 #pragma unroll
-    for (int ct = 0; ct < 4; ct++) acc[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < 4; k++) p[4 * k] = make_float4(x[4 * k], x[4 * k + 1], x[4 * k + 2], x[4 * k + 3]);
+}
+// the same values of the neighbouring row (l ^ 1: the other polarity of the variable)
+__device__ __forceinline__ bf16x8 flip8(bf16x8 v)
+{
+    uint4 w = __builtin_bit_cast(uint4, v);   // (product lane order)
+    w.x = __builtin_amdgcn_mov_dpp(w.x, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
+    w.y = __builtin_amdgcn_mov_dpp(w.y, 0xB1, 0xF, 0xF, false);
+    w.z = __builtin_amdgcn_mov_dpp(w.z, 0xB1, 0xF, 0xF, false);
+    w.w = __builtin_amdgcn_mov_dpp(w.w, 0xB1, 0xF, 0xF, false);
+    return __builtin_bit_cast(bf16x8, w);
+}
+// between the lane orders of memory (4r + q) and of the products (16q + r)
+__device__ __forceinline__ int lane_perm(int x, int from) { return __builtin_amdgcn_ds_bpermute(from, x); }
+__device__ __forceinline__ bf16x8 to_product(bf16x8 v, int lane)
+{
+    const int from = 4 * (4 * (lane & 15) + (lane >> 4));
+    const uint4 w = __builtin_bit_cast(uint4, v);
+    return __builtin_bit_cast(bf16x8, uint4{(uint32_t)lane_perm(w.x, from), (uint32_t)lane_perm(w.y, from),
+                                            (uint32_t)lane_perm(w.z, from), (uint32_t)lane_perm(w.w, from)});
+}
+__device__ __forceinline__ void from_product(float (&x)[16], int lane)
+{
+    const int from = 4 * (16 * (lane & 3) + (lane >> 2));
 #pragma unroll
-    for (int k0 = 0; k0 < K; k0 += 32) {
-        bf16x8 a = __builtin_bit_cast(bf16x8, uint4{0u, 0u, 0u, 0u});
-        if (ar < N) a = ld8(X + (size_t)ar * K + k0 + kq);
-#pragma unroll
-        for (int ct = 0; ct < 4; ct++) acc[ct] = mfma32(a, ld8(sW + (ct * 16 + (lane & 15)) * SK + k0 + kq), acc[ct]);
+    for (int i = 0; i < 16; i++) x[i] = __int_as_float(lane_perm(__float_as_int(x[i]), from));
+}
+__device__ __forceinline__ float flip1(float x)
+{
+    return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0xB1, 0xF, 0xF, false));
+}
+
+// Weights [R x KW] (row-major BF16) into LDS, rows padded by 16 bytes (the 16 rows a wave
+// reads at once fall in different banks).
+template <int R, int KW>
+__device__ __forceinline__ void stage_weights(bf16_t* s, const bf16_t* __restrict__ W)
+{
+    for (int i = threadIdx.x; i < R * KW / 8; i += blockDim.x) {
+        const int c = (8 * i) / KW, k = (8 * i) % KW;
+        *reinterpret_cast<uint4*>(s + c * (KW + 8) + k) = reinterpret_cast<const uint4*>(W)[i];
     }
-    const int dq = 4 * (lane >> 4);
+}
+// x[i] = the product's output column 64B + out(i): KS k-steps of 32 against the staged rows
+// (f and x in product lane order)
+template <int KS>
+__device__ __forceinline__ void product(float (&x)[16], const bf16_t* s, int B, const bf16x8 (&f)[KS], int lane)
+{
+    constexpr int SK = 32 * KS + 8;
+    int at = (64 * B + (lane & 15)) * SK + 8 * (lane >> 4);
+    asm volatile("" : "+v"(at));   // weights stay in LDS: hoisted out of the tile loop they spill
 #pragma unroll
     for (int ct = 0; ct < 4; ct++) {
-        const int col = ct * 16 + (lane & 15);
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int row = r0 + dq + j;
-            if (row < N) out[(size_t)row * 64 + col] = fmaxf(acc[ct][j] + bias[col], 0.0f);
+        for (int k = 0; k < KS; k++) acc = mfma32(ld8(s + at + 16 * ct * SK + 32 * k), f[k], acc);
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[4 * ct + j] = acc[j];
+    }
+}
+
+// value of lane J of the quad, in each of its four lanes
+template <int J>
+__device__ __forceinline__ int quad_lane(int x) { return __builtin_amdgcn_mov_dpp(x, 0x55 * J, 0xF, 0xF, false); }
+
+__device__ __forceinline__ uint32_t quad_or(uint32_t x)
+{
+    x |= __builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, false);      // quad_perm [1,0,3,2]
+    return x | __builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
+}
+
+// The edges of one row, read ahead: its offsets, and the index of its q-th neighbour of four in
+// lane q (a load costs the address unit as much for one index in all four lanes as for four).
+struct Edges {
+    int e0, e1, id;
+    __device__ __forceinline__ void offsets(const int32_t* __restrict__ off, int row, int q)
+    {
+        const int e = off[row + (q & 1)];
+        e0 = quad_lane<0>(e);
+        e1 = quad_lane<1>(e);
+    }
+    __device__ __forceinline__ void ids(const int32_t* __restrict__ edges, int e, int q)
+    {
+        id = edges[max(0, min(e + q, e1 - 1))];
+    }
+};
+// s += sum over the row's edges of the neighbours' rows X[id], in edge order; two rows in
+// flight, the next four edges' indices read meanwhile
+__device__ __forceinline__ void gather_row(float (&s)[16], const int32_t* __restrict__ edges, Edges& E, int q,
+                                           const float* __restrict__ X)
+{
+    auto add = [&](const float(&x)[16]) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) s[i] += x[i];
+    };
+    for (int e = E.e0; e < E.e1; e += 4) {
+        const int k = E.e1 - e, v = E.id;
+        float a[16], b[16];
+        ld_row(a, X + (size_t)quad_lane<0>(v) * HID, q);
+        if (k > 1) ld_row(b, X + (size_t)quad_lane<1>(v) * HID, q);
+        if (k > 4) E.ids(edges, e + 4, q);
+        add(a);
+        if (k > 1) add(b);
+        if (k > 2) {
+            ld_row(a, X + (size_t)quad_lane<2>(v) * HID, q);
+            if (k > 3) ld_row(b, X + (size_t)quad_lane<3>(v) * HID, q);
+            add(a);
+            if (k > 3) add(b);
         }
     }
 }
 
-// dX[N x K] = dP[N x 64] W[64 x K]; W staged transposed (k = hidden index contiguous).
-template <int K>
-__global__ __launch_bounds__(256) void k_dense_bwd_dx(const bf16_t* __restrict__ dP, const bf16_t* __restrict__ Wq,
-                                                      float* __restrict__ dX, int N)
+// Workgroups go to the XCDs in turn (workgroup b to XCD b % 8): logical block of workgroup b
+// such that each XCD takes one contiguous eighth of the rows, so an instance's rows stay in
+// one XCD's L2 for the gathers of its neighbours.  The grid is a multiple of 8.
+__device__ __forceinline__ int xcd_block() { return (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3); }
+
+// x summed over the 16 rows, in every lane of its column quarter q: two rotations inside each
+// 16 lanes, then the permlane swaps (no LDS); fixed order
+__device__ __forceinline__ float row_sum(float x)
 {
-    constexpr int SH = 64 + 8;
-    __shared__ __align__(16) bf16_t sWt[K * SH];
-    for (int i = threadIdx.x; i < 64 * K; i += blockDim.x) {
-        const int h = i / K, c = i % K;
-        sWt[c * SH + h] = Wq[i];
+    x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x124, 0xF, 0xF, false));   // row_ror:4
+    x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x128, 0xF, 0xF, false));   // row_ror:8
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_int(x), __float_as_int(x), false, false);
+    x = __int_as_float(r[0]) + __int_as_float(r[1]);
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_int(x), __float_as_int(x), false, false);
+    return __int_as_float(h[0]) + __int_as_float(h[1]);
+}
+// Workgroup totals of each wavefront's x[i] (column in(i) or out(i), over its rows) into
+// out[64]; fixed order.  red: 64 floats a wavefront.
+template <bool OUT>
+__device__ __forceinline__ void block_sum(const float (&x)[16], float* red, float* out, int lane, int wave)
+{
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const float v = row_sum(x[i]);
+        if (lane < 4) red[64 * wave + (OUT ? 16 * (i >> 2) + 4 * lane + (i & 3) : 32 * (i >> 3) + 8 * lane + (i & 7))] = v;
     }
     __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r0 = (blockIdx.x * 4 + wave) * 16;
-    if (r0 >= N) return;
-    const int ar = r0 + (lane & 15), kq = 8 * (lane >> 4);
-    constexpr int CT = K / 16;
-    f32x4 acc[CT];
-#pragma unroll
-    for (int ct = 0; ct < CT; ct++) acc[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int h0 = 0; h0 < 64; h0 += 32) {
-        bf16x8 a = __builtin_bit_cast(bf16x8, uint4{0u, 0u, 0u, 0u});
-        if (ar < N) a = ld8(dP + (size_t)ar * 64 + h0 + kq);
-#pragma unroll
-        for (int ct = 0; ct < CT; ct++) acc[ct] = mfma32(a, ld8(sWt + (ct * 16 + (lane & 15)) * SH + h0 + kq), acc[ct]);
+    if (threadIdx.x < 64) {
+        float v = 0.f;
+        for (int w = 0; w < (int)blockDim.x >> 6; w++) v += red[64 * w + threadIdx.x];
+        out[threadIdx.x] = v;
     }
-    const int dq = 4 * (lane >> 4);
+}
+
+// One half round, whole: H' = relu([H | scale * sum of neighbours | (LIT) H of l ^ 1] W^T + b),
+// 16 rows per wavefront, in place (a row is read and written by its own wavefront only, and the
+// two rows of a variable share one).
+//   FIRST  H is the embedding, computed from the degrees instead of read, the neighbours' too:
+//          8 bytes of offsets per edge, looked up by the lane that holds its index, instead of a
+//          256-byte row (added edge by edge in FP32 like any message: from the sum of the
+//          occurrences it would be rounded differently)
+//   TRAIN  X = bf16([H | messages]) and the sign mask of H' are kept for the backward pass
+template <bool LIT, bool FIRST, bool TRAIN>
+__global__ __launch_bounds__(256, 4) void k_layer(const int32_t* __restrict__ off, const int32_t* __restrict__ edges,
+                                                  const int32_t* __restrict__ n_off, int N, const float* __restrict__ th,
+                                                  const bf16_t* __restrict__ W, const float* __restrict__ bias,
+                                                  const float* __restrict__ Hn, float* H, bf16_t* __restrict__ X,
+                                                  uint2* __restrict__ mask)
+{
+    constexpr int K = LIT ? 192 : 128, KS = K / 32;
+    __shared__ __align__(16) bf16_t sW[64 * (K + 8)];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane & 3;
+    const int r = 16 * (xcd_block() * 4 + wave) + (lane >> 2), row = min(r, N - 1);
+    Edges E;
+    E.offsets(off, row, q);
+    stage_weights<64, K>(sW, W);
+    const int deg = E.e1 - E.e0;
+    E.ids(edges, E.e0, q);
+    float h[16], s[16], b[16];
+    bf16x8 f[KS];
+    if constexpr (FIRST) {
+        ld_row(h, th + (LIT ? O_UL : O_UC), q);
+        ld_row(b, th + (LIT ? O_VL : O_VC), q);
 #pragma unroll
-    for (int ct = 0; ct < CT; ct++) {
-        const int col = ct * 16 + (lane & 15);
+        for (int i = 0; i < 16; i++) h[i] = (float)deg * (LIT ? 0.125f : 0.25f) * h[i] + b[i];
+    } else
+        ld_row(h, H + (size_t)row * HID, q);
+    if constexpr (FIRST && !LIT) {
+        float u[16];
+        ld_row(u, th + O_UL, q);
+        ld_row(b, th + O_VL, q);
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int row = r0 + dq + j;
-            if (row < N) dX[(size_t)row * K + col] = acc[ct][j];
+        for (int i = 0; i < 16; i++) s[i] = 0.f;
+        auto add = [&](int occ) {
+            const float w = (float)occ * 0.125f;
+#pragma unroll
+            for (int i = 0; i < 16; i++) s[i] += w * u[i] + b[i];
+        };
+        for (int e = E.e0; e < E.e1; e += 4) {
+            const int k = E.e1 - e, occ = n_off[E.id + 1] - n_off[E.id];
+            if (k > 4) E.ids(edges, e + 4, q);
+            add(quad_lane<0>(occ));
+            if (k > 1) add(quad_lane<1>(occ));
+            if (k > 2) add(quad_lane<2>(occ));
+            if (k > 3) add(quad_lane<3>(occ));
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 16; i++) s[i] = 0.f;
+        gather_row(s, edges, E, q, Hn);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; i++) s[i] *= LIT ? 0.125f : 0.25f;
+    f[0] = pack8(h);
+    f[1] = pack8(h + 8);
+    f[2] = pack8(s);
+    f[3] = pack8(s + 8);
+    if constexpr (TRAIN) {
+        if (r < N) {
+            bf16_t* x = X + (size_t)r * 128 + 8 * q;
+            st8(x, f[0]);
+            st8(x + 32, f[1]);
+            st8(x + 64, f[2]);
+            st8(x + 96, f[3]);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) f[k] = to_product(f[k], lane);
+    if constexpr (LIT) {
+        f[4] = flip8(f[0]);
+        f[5] = flip8(f[1]);
+    }
+    __syncthreads();   // (the staged weights)
+    product<KS>(h, sW, 0, f, lane);
+    from_product(h, lane);
+    ld_row<true>(b, bias, q);
+    uint32_t lo = 0, hi = 0;   // one bit per column
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        h[i] = fmaxf(h[i] + b[i], 0.f);
+        (i < 8 ? lo : hi) |= h[i] > 0.f ? 1u << (16 * (i >> 2 & 1) + (i & 3)) : 0u;
+    }
+    if constexpr (TRAIN) {
+        lo = quad_or(lo << 4 * q);
+        hi = quad_or(hi << 4 * q);
+        if (r < N && q == 0) mask[r] = uint2{lo, hi};
+    }
+    if (r < N) st_row(H + (size_t)r * HID, h, q);
+}
+
+// One half round backward, whole, 16 rows per wavefront: with dH' = S + scale * sum of the
+// neighbours' message gradients G (either may be absent: SELF, GATHER), dP = dH' * [H' > 0]
+// (kept in BF16 for the weight gradient; its FP32 sum is the bias gradient) and dX = dP W: the
+// columns of this row's own H go to S in place (LIT: plus those the other polarity's row has for
+// it, exchanged between neighbouring lanes), the message columns to M.  The clauses' S of the
+// first round (LAST) is the gradient of their embedding and is summed here instead of stored.
+// part: the workgroup's bias sums, 64 floats; part_e: those for u_c and v_c, 128.
+template <bool LIT, bool SELF, bool GATHER, bool LAST>
+__global__ __launch_bounds__(256, 4) void k_layer_bwd(const int32_t* __restrict__ off, const int32_t* __restrict__ edges,
+                                                      int N, const bf16_t* __restrict__ Wt,
+                                                      const uint2* __restrict__ mask, const float* __restrict__ G,
+                                                      float* S, bf16_t* __restrict__ dP, float* __restrict__ M,
+                                                      float* __restrict__ part, float* __restrict__ part_e)
+{
+    constexpr int K = LIT ? 192 : 128;
+    __shared__ __align__(16) bf16_t sW[K * (64 + 8)];
+    __shared__ float red[256];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane & 3;
+    const int block = xcd_block(), r = 16 * (block * 4 + wave) + (lane >> 2), row = min(r, N - 1);
+    Edges E;
+    if constexpr (GATHER || LAST) E.offsets(off, row, q);
+    stage_weights<K, 64>(sW, Wt);
+    const int deg = GATHER || LAST ? E.e1 - E.e0 : 0;
+    if constexpr (GATHER) E.ids(edges, E.e0, q);
+    const uint2 m2 = r < N ? mask[row] : uint2{0u, 0u};
+    const uint32_t m = (m2.x >> 8 * q & 0xFF) | (m2.y >> 8 * q & 0xFF) << 8;
+    float g[16], s[16];
+    if constexpr (SELF)
+        ld_row(g, S + (size_t)row * HID, q);
+    else {
+#pragma unroll
+        for (int i = 0; i < 16; i++) g[i] = 0.f;
+    }
+    if constexpr (GATHER) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) s[i] = 0.f;
+        gather_row(s, edges, E, q, G);
+#pragma unroll
+        for (int i = 0; i < 16; i++) g[i] += (LIT ? 0.25f : 0.125f) * s[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 16; i++) g[i] = m >> i & 1 ? g[i] : 0.f;
+    block_sum<false>(g, red, part + (size_t)block * 64, lane, wave);   // (its barriers: the staged weights too)
+    bf16x8 f[2] = {pack8(g), pack8(g + 8)};
+    if (r < N) {
+        st8(dP + (size_t)r * HID + 8 * q, f[0]);
+        st8(dP + (size_t)r * HID + 32 + 8 * q, f[1]);
+    }
+    f[0] = to_product(f[0], lane);
+    f[1] = to_product(f[1], lane);
+    product<2>(g, sW, 1, f, lane);
+    from_product(g, lane);
+    if (r < N) st_row(M + (size_t)r * HID, g, q);
+    product<2>(g, sW, 0, f, lane);
+    if constexpr (LIT) {
+        product<2>(s, sW, 2, f, lane);
+#pragma unroll
+        for (int i = 0; i < 16; i++) g[i] += flip1(s[i]);
+    }
+    from_product(g, lane);
+    if constexpr (LAST) {
+        // (a row past N has dP = 0, so dX = 0)
+        block_sum<true>(g, red, part_e + (size_t)block * 128 + 64, lane, wave);
+#pragma unroll
+        for (int i = 0; i < 16; i++) g[i] *= (float)deg * 0.25f;
+        block_sum<true>(g, red, part_e + (size_t)block * 128, lane, wave);
+    } else if (r < N)
+        st_row(S + (size_t)r * HID, g, q);
+}
+
+// Readout of 16 variables per wavefront and tile: R = relu([H_{2v+1} | H_{2v}] W_o^T + b_o),
+// Y = R W_y^T + b_y (W_y in BF16); TRAIN: also the loss, dY, dP_o = (dY W_y) * [R > 0] and the
+// gradient of H (S), with Z and dP_o kept in BF16 for the gradient of W_o and this
+// workgroup's sums for b_o, W_y, b_y (laid out as the parameters are) and the loss.
+constexpr int HEAD_PART = 256, HEAD_GRADS = O_BY + 2 - O_BO;
+template <bool TRAIN>
+__global__ __launch_bounds__(256) void k_readout(int V, int tiles_per_wave, const float* __restrict__ H,
+                                                 const bf16_t* __restrict__ Wo, const bf16_t* __restrict__ Wot,
+                                                 const bf16_t* __restrict__ Wyq, const float* __restrict__ th,
+                                                 float* __restrict__ Y, const float* __restrict__ target,
+                                                 const float* __restrict__ phase, const float* __restrict__ mask,
+                                                 float alpha, bf16_t* __restrict__ Z, bf16_t* __restrict__ dP,
+                                                 float* __restrict__ S, float* __restrict__ part)
+{
+    __shared__ __align__(16) bf16_t sW[64 * (128 + 8)];
+    __shared__ __align__(16) bf16_t sWt[TRAIN ? 128 * (64 + 8) : 8];
+    constexpr int SP = 64 + 8;
+    __shared__ __align__(16) bf16_t sP[TRAIN ? 64 * SP : 8];
+    __shared__ float red[256];
+    stage_weights<64, 128>(sW, Wo);
+    if constexpr (TRAIN) stage_weights<128, 64>(sWt, Wot);
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane & 3;
+    const int block = xcd_block(), t0 = (block * 4 + wave) * tiles_per_wave;
+    float w0[16], w1[16], gb[16], gw0[16], gw1[16], lsum = 0.f, gy0 = 0.f, gy1 = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const int d = 16 * (i >> 2) + 4 * q + (i & 3);
+        w0[i] = from_bf16(Wyq[d]);
+        w1[i] = from_bf16(Wyq[64 + d]);
+        gb[i] = gw0[i] = gw1[i] = 0.f;
+    }
+    for (int t = t0; t < t0 + tiles_per_wave && 16 * t < V; t++) {
+        const int v = 16 * t + (lane >> 2), row = min(v, V - 1);
+        float x[16], b[16];
+        bf16x8 f[4];
+        ld_row(x, H + (size_t)(2 * row + 1) * HID, q);
+        f[0] = pack8(x);
+        f[1] = pack8(x + 8);
+        ld_row(x, H + (size_t)(2 * row) * HID, q);
+        f[2] = pack8(x);
+        f[3] = pack8(x + 8);
+        if constexpr (TRAIN) {
+            if (v < V) {
+                bf16_t* z = Z + (size_t)v * 128 + 8 * q;
+                st8(z, f[0]);
+                st8(z + 32, f[1]);
+                st8(z + 64, f[2]);
+                st8(z + 96, f[3]);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) f[k] = to_product(f[k], lane);
+        product<4>(x, sW, 0, f, lane);
+        from_product(x, lane);
+        ld_row<true>(b, th + O_BO, q);
+        float y0 = 0.f, y1 = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            x[i] = fmaxf(x[i] + b[i], 0.f);
+            y0 += x[i] * w0[i];
+            y1 += x[i] * w1[i];
+        }
+        y0 += __shfl_xor(y0, 1);
+        y1 += __shfl_xor(y1, 1);
+        y0 += __shfl_xor(y0, 2);
+        y1 += __shfl_xor(y1, 2);
+        y0 += th[O_BY];
+        y1 += th[O_BY + 1];
+        if (q == 0 && v < V) *reinterpret_cast<float2*>(Y + 2 * (size_t)v) = make_float2(y0, y1);
+        if constexpr (TRAIN) {
+            const float tg = target[row], p = phase[row], mk = mask[row];
+            const float sig = 1.0f / (1.0f + expf(-y1));
+            const float bce = fmaxf(y1, 0.f) - y1 * p + log1pf(expf(-fabsf(y1)));
+            const bool live = v < V;
+            const float da = live ? 2.0f * (y0 - tg) / (float)V : 0.f;
+            const float db = live ? alpha * mk * (sig - p) / (float)V : 0.f;
+            if (q == 0 && live) {
+                lsum += ((y0 - tg) * (y0 - tg) + alpha * mk * bce) / (float)V;
+                gy0 += da;
+                gy1 += db;
+            }
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                if (live) {
+                    gw0[i] += da * x[i];
+                    gw1[i] += db * x[i];
+                }
+                x[i] = live && x[i] > 0.f ? da * w0[i] + db * w1[i] : 0.f;
+                gb[i] += x[i];
+            }
+            // dP is in columns out(i); the product and the stored row take in(i): through LDS
+            const bf16x8 o[2] = {pack8(x), pack8(x + 8)};
+            const uint4 w[2] = {__builtin_bit_cast(uint4, o[0]), __builtin_bit_cast(uint4, o[1])};
+            bf16_t* tile = sP + wave * 16 * SP;
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                *reinterpret_cast<uint2*>(tile + (lane >> 2) * SP + 16 * k + 4 * q) =
+                    k & 1 ? uint2{w[k >> 1].z, w[k >> 1].w} : uint2{w[k >> 1].x, w[k >> 1].y};
+            wave_sync();
+            if (live) {
+                st8(dP + (size_t)v * HID + 8 * q, ld8(tile + (lane >> 2) * SP + 8 * q));
+                st8(dP + (size_t)v * HID + 32 + 8 * q, ld8(tile + (lane >> 2) * SP + 32 + 8 * q));
+            }
+            const bf16x8 g[2] = {ld8(tile + (lane & 15) * SP + 8 * (lane >> 4)),
+                                 ld8(tile + (lane & 15) * SP + 32 + 8 * (lane >> 4))};
+            wave_sync();
+            product<2>(x, sWt, 0, g, lane);
+            from_product(x, lane);
+            if (live) st_row(S + (size_t)(2 * v + 1) * HID, x, q);
+            product<2>(x, sWt, 1, g, lane);
+            from_product(x, lane);
+            if (live) st_row(S + (size_t)(2 * v) * HID, x, q);
+        }
+    }
+    if constexpr (TRAIN) {
+        float* o = part + (size_t)block * HEAD_PART;
+        block_sum<true>(gb, red, o, lane, wave);
+        block_sum<true>(gw0, red, o + (O_WY - O_BO), lane, wave);
+        block_sum<true>(gw1, red, o + (O_WY - O_BO) + 64, lane, wave);
+        gy0 = row_sum(gy0);
+        gy1 = row_sum(gy1);
+        lsum = row_sum(lsum);
+        __syncthreads();
+        if (lane == 0) {
+            red[wave] = gy0;
+            red[4 + wave] = gy1;
+            red[8 + wave] = lsum;
+        }
+        __syncthreads();
+        if (threadIdx.x < 64) {
+            const int k = threadIdx.x;
+            o[(O_BY - O_BO) + k] = k < 3 ? (red[4 * k] + red[4 * k + 1]) + (red[4 * k + 2] + red[4 * k + 3]) : 0.f;
         }
     }
 }
@@ -153,49 +574,63 @@ __device__ __forceinline__ bf16x8 ld8_tr(const bf16_t* p, int row_stride)
     return __builtin_bit_cast(bf16x8, v);
 }
 
-// Partial weight gradient of this workgroup: part[blockIdx.x][64 x K] = sum over its
-// 64-node chunks of dP[N x 64]^T X[N x K] (the reduction adds the workgroups' partials in
-// order).  A chunk is staged row-major in LDS (node index = row, 16-byte stores, rows padded
-// by 32 bytes) by all four wavefronts, and the MFMA operands, whose k index is the node, come
-// out of it through transposing reads; wavefront w computes output rows h = 16w .. 16w+15.
+// Partial weight gradient of this workgroup: part[blockIdx.x][64 x K] = sum over its 64-row
+// chunks of dP[N x 64]^T X[N x K], N the rows of all rounds (the reduction adds the
+// workgroups' partials in order).  X holds 128 columns a row; for K = 192 the other 64 are the
+// first 64 of row n ^ 1.  A chunk is staged row-major in LDS (rows padded by 32 bytes) by all
+// four wavefronts while the next chunk's reads are in flight, and the MFMA operands, whose k
+// index is the row, come out of it through transposing reads; wavefront w computes output rows
+// h = 16w .. 16w+15.
 template <int K>
-__global__ __launch_bounds__(256) void k_dense_bwd_dw(const bf16_t* __restrict__ dP, const bf16_t* __restrict__ X,
-                                                      float* __restrict__ part, int N)
+__global__ __launch_bounds__(256) void k_dense_dw(const bf16_t* __restrict__ dP, const bf16_t* __restrict__ X,
+                                                  float* __restrict__ part, int64_t N)
 {
-    constexpr int SP = 64 + 16, SX = K + 16;   // row strides (elements) of the staged tiles
+    constexpr int SP = 64 + 16, SX = 128 + 16, CT = K / 16;   // row strides (elements) of the staged tiles
     __shared__ __align__(16) bf16_t sP[64 * SP];
     __shared__ __align__(16) bf16_t sX[64 * SX];
-    constexpr int CT = K / 16;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     // this lane's place in a transposing read: row 8(lane/16) + (lane%16)/4 of the k block,
     // columns 4(lane%4) .. +3 of the 16-column tile
     const int tr_row = 8 * (lane >> 4) + ((lane & 15) >> 2), tr_col = 4 * (lane & 3);
+    uint4 p[2], x[4];
+    auto load = [&](int64_t n0) {
+        const int64_t rows = N - n0;
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const int r = (t >> 3) + 32 * k;
+            p[k] = uint4{0u, 0u, 0u, 0u};
+            if (r < rows) p[k] = *reinterpret_cast<const uint4*>(dP + (size_t)(n0 + r) * 64 + 8 * (t & 7));
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int r = (t >> 4) + 16 * k;
+            x[k] = uint4{0u, 0u, 0u, 0u};
+            if (r < rows) x[k] = *reinterpret_cast<const uint4*>(X + (size_t)(n0 + r) * 128 + 8 * (t & 15));
+        }
+    };
     f32x4 acc[CT];
 #pragma unroll
     for (int ct = 0; ct < CT; ct++) acc[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int n0 = blockIdx.x * 64; n0 < N; n0 += gridDim.x * 64) {
-        const int rows = min(64, N - n0);
+    int64_t n0 = (int64_t)blockIdx.x * 64;
+    const int64_t step = (int64_t)gridDim.x * 64;
+    if (n0 < N) load(n0);
+    for (; n0 < N; n0 += step) {
         __syncthreads();
-        for (int q = t; q < 64 * 8; q += 256) {
-            const int r = q >> 3, c = (q & 7) * 8;
-            uint4 v = {0u, 0u, 0u, 0u};
-            if (r < rows) v = *reinterpret_cast<const uint4*>(dP + (size_t)(n0 + r) * 64 + c);
-            *reinterpret_cast<uint4*>(sP + r * SP + c) = v;
-        }
-        for (int q = t; q < 64 * (K / 8); q += 256) {
-            const int r = q / (K / 8), c = (q % (K / 8)) * 8;
-            uint4 v = {0u, 0u, 0u, 0u};
-            if (r < rows) v = *reinterpret_cast<const uint4*>(X + (size_t)(n0 + r) * K + c);
-            *reinterpret_cast<uint4*>(sX + r * SX + c) = v;
-        }
+#pragma unroll
+        for (int k = 0; k < 2; k++) *reinterpret_cast<uint4*>(sP + ((t >> 3) + 32 * k) * SP + 8 * (t & 7)) = p[k];
+#pragma unroll
+        for (int k = 0; k < 4; k++) *reinterpret_cast<uint4*>(sX + ((t >> 4) + 16 * k) * SX + 8 * (t & 15)) = x[k];
         __syncthreads();
+        if (n0 + step < N) load(n0 + step);
 #pragma unroll
         for (int s = 0; s < 64; s += 32) {
             // A[h][n] = dP[n][h] (16 h x 32 n), B[n][col] = X[n][col] (32 n x 16 col)
             const bf16x8 a = ld8_tr(sP + (s + tr_row) * SP + 16 * wave + tr_col, SP);
 #pragma unroll
-            for (int ct = 0; ct < CT; ct++)
-                acc[ct] = mfma32(a, ld8_tr(sX + (s + tr_row) * SX + 16 * ct + tr_col, SX), acc[ct]);
+            for (int ct = 0; ct < CT; ct++) {
+                const int r = ct < 8 ? s + tr_row : s + (tr_row ^ 1), c = ct < 8 ? 16 * ct : 16 * (ct - 8);
+                acc[ct] = mfma32(a, ld8_tr(sX + r * SX + c + tr_col, SX), acc[ct]);
+            }
         }
     }
     float* out = part + (size_t)blockIdx.x * 64 * K;
@@ -208,342 +643,127 @@ __global__ __launch_bounds__(256) void k_dense_bwd_dw(const bf16_t* __restrict__
     }
 }
 
-// Fixed-order reductions of per-slot partials: out[i] (+)= the sum over slots of
-// part[slot * width + i].  Every gradient and the loss are summed this way, never with
-// floating-point atomics, so a gradient is the same bit for bit on every run.
-// Wide (weight matrices, few slots): one thread per element adds its slots in order.
-template <bool ACCUMULATE>
-__global__ void k_reduce_wide(const float* __restrict__ part, int slots, int width, float* __restrict__ out)
-{
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < width; i += gridDim.x * blockDim.x) {
-        float s = 0.f;
-        for (int k = 0; k < slots; k++) s += part[(size_t)k * width + i];
-        out[i] = ACCUMULATE ? out[i] + s : s;
-    }
-}
-
-// Wide with many slots (weight-gradient partials of up to 1024 workgroups): first each
-// of `groups` workgroup rows adds its own contiguous run of slots, four columns per
-// thread, into part2[group * width + i]; k_reduce_wide then adds the groups in order.
-__global__ __launch_bounds__(256) void k_reduce_wide_split(const float* __restrict__ part, int slots, int width,
-                                                           float* __restrict__ part2)
-{
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;  // column quad
-    if (4 * q >= width) return;
-    const int per = (slots + gridDim.y - 1) / gridDim.y;
-    const int k0 = blockIdx.y * per, k1 = min(slots, k0 + per);
-    const float4* p = reinterpret_cast<const float4*>(part) + q;
-    const size_t stride = (size_t)width / 4;
-    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll 8
-    for (int k = k0; k < k1; k++) {
-        const float4 v = p[(size_t)k * stride];
-        s.x += v.x;
-        s.y += v.y;
-        s.z += v.z;
-        s.w += v.w;
-    }
-    reinterpret_cast<float4*>(part2)[(size_t)blockIdx.y * stride + q] = s;
-}
-
-// Narrow (biases, embeddings, the loss; thousands of slots): one workgroup per element,
-// each thread adds a fixed stride of slots, then a fixed binary tree in LDS.
-template <bool ACCUMULATE>
-__global__ __launch_bounds__(256) void k_reduce_tree(const float* __restrict__ part, int slots, int width,
-                                                     float* __restrict__ out)
-{
-    __shared__ float sh[256];
-    const int t = threadIdx.x;
-    for (int i = blockIdx.x; i < width; i += gridDim.x) {
-        float s = 0.f;
-        for (int k = t; k < slots; k += 256) s += part[(size_t)k * width + i];
-        sh[t] = s;
-        __syncthreads();
-        for (int o = 128; o > 0; o >>= 1) {
-            if (t < o) sh[t] += sh[t + o];
-            __syncthreads();
-        }
-        if (t == 0) out[i] = ACCUMULATE ? out[i] + sh[0] : sh[0];
-        __syncthreads();
-    }
-}
-
-// ---------------------------------------------------------------------------------------
-// Aggregation, embedding, head and bookkeeping kernels: one wave per node row, lane = dim.
-
-__global__ void k_embed(const int32_t* __restrict__ l_off, const int32_t* __restrict__ c_off, int L, int C,
-                        const float* __restrict__ th, float* __restrict__ Hl, float* __restrict__ Hc)
-{
-    const int64_t total = (int64_t)(L + C) * HID;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-        const int d = (int)(i & 63);
-        const int64_t r = i >> 6;
-        if (r < L) {
-            const float occ = (float)(l_off[r + 1] - l_off[r]);
-            Hl[i] = occ * 0.125f * th[O_UL + d] + th[O_VL + d];
-        } else {
-            const int64_t c = r - L;
-            const float len = (float)(c_off[c + 1] - c_off[c]);
-            Hc[c * HID + d] = len * 0.25f * th[O_UC + d] + th[O_VC + d];
-        }
-    }
-}
-
-__device__ __forceinline__ int wave_global() { return (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6); }
-__device__ __forceinline__ int wave_count() { return (int)((gridDim.x * blockDim.x) >> 6); }
-
-// The gather kernels give each wavefront 4 rows at once, 16 lanes per row, each lane on 4
-// consecutive dimensions: a 256-byte row is one float4 load per lane, and a wavefront
-// keeps 4 rows' dependent offset -> edge -> neighbour loads in flight together.
-__device__ __forceinline__ int row_slot() { return (threadIdx.x & 63) >> 4; }
-__device__ __forceinline__ int col4() { return 4 * (threadIdx.x & 15); }
+// This workgroup's partial gradients of the literals' embeddings u_l, v_l (parameters 0..127)
+// from dH^0 = S + 1/4 (sum of M over the clauses); 16 lanes per row, each on 4 consecutive
+// dimensions.
 __device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
-__device__ __forceinline__ void add4(float4& s, const float4& x)
+__device__ __forceinline__ void fma4(float4& s, float a, const float4& x)
 {
-    s.x += x.x;
-    s.y += x.y;
-    s.z += x.z;
-    s.w += x.w;
+    s.x += a * x.x;
+    s.y += a * x.y;
+    s.z += a * x.z;
+    s.w += a * x.w;
 }
-__device__ __forceinline__ float4 mul4(float a, const float4& x) { return make_float4(a * x.x, a * x.y, a * x.z, a * x.w); }
-__device__ __forceinline__ void st_bf16x4(bf16_t* p, const float4& v)
+__global__ __launch_bounds__(256) void k_bwd_embed(const int32_t* __restrict__ off, const int32_t* __restrict__ edges,
+                                                   int L, const float* __restrict__ S, const float* __restrict__ M,
+                                                   float* __restrict__ part)
 {
-    uint2 w;
-    w.x = (uint32_t)to_bf16(v.x) | (uint32_t)to_bf16(v.y) << 16;
-    w.y = (uint32_t)to_bf16(v.z) | (uint32_t)to_bf16(v.w) << 16;
-    *reinterpret_cast<uint2*>(p) = w;
+    __shared__ float4 red[16][32];
+    const int k16 = threadIdx.x & 15, d = 4 * k16, slot = threadIdx.x >> 4;
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 gu = zero, gv = zero;
+    const int block = xcd_block(), per = (L + gridDim.x - 1) / gridDim.x;
+    for (int l = block * per + slot, end = min(L, (block + 1) * per); l < end; l += 16) {
+        const int e0 = off[l], e1 = off[l + 1];
+        float4 m = zero;
+        for (int e = e0; e < e1; e += 4) {
+            const int k = e1 - e;
+            const int i0 = edges[e], i1 = edges[k > 1 ? e + 1 : e], i2 = edges[k > 2 ? e + 2 : e],
+                      i3 = edges[k > 3 ? e + 3 : e];
+            const float4 x0 = ld4(M + (size_t)i0 * HID + d), x1 = ld4(M + (size_t)i1 * HID + d);
+            const float4 x2 = ld4(M + (size_t)i2 * HID + d), x3 = ld4(M + (size_t)i3 * HID + d);
+            fma4(m, 1.f, x0);
+            if (k > 1) fma4(m, 1.f, x1);
+            if (k > 2) fma4(m, 1.f, x2);
+            if (k > 3) fma4(m, 1.f, x3);
+        }
+        float4 g = ld4(S + (size_t)l * HID + d);
+        fma4(g, 0.25f, m);
+        fma4(gu, (float)(e1 - e0) * 0.125f, g);
+        fma4(gv, 1.f, g);
+    }
+    red[slot][k16] = gu;
+    red[slot][16 + k16] = gv;
+    __syncthreads();
+    if (threadIdx.x < 32) {
+        float4 s = zero;
+        for (int i = 0; i < 16; i++) fma4(s, 1.f, red[i][threadIdx.x]);
+        *reinterpret_cast<float4*>(part + (size_t)block * O_UC + 4 * threadIdx.x) = s;
+    }
 }
 
-// Sum over edges e0 .. e1-1 of X[edges[e] * stride + col .. col + 3], four neighbour rows in
-// flight at a time (a slot past e1 re-reads edge e0 of its quad and is not added), added in
-// edge order.
-__device__ __forceinline__ float4 gather_sum(const int32_t* __restrict__ edges, int e0, int e1,
-                                             const float* __restrict__ X, int stride, int col)
+// Fixed-order reductions of the workgroups' partials, all of a pass's in two launches: every
+// gradient and the loss are summed this way, never with floating-point atomics, so a gradient
+// is the same bit for bit on every run.  Job: `slots` rows of `quads` float4; stage 1 splits
+// the slots into `groups` contiguous runs (16 column quads x 16 interleaved slots per
+// workgroup), stage 2 adds the groups in order and writes the first n floats to out and the
+// rest, if out2 is given, to out2.
+struct RedJob {
+    const float* part;
+    float* part2;
+    float* out;
+    float* out2;
+    int slots, quads, groups, n;
+};
+constexpr int RED_JOBS = 8;
+struct RedJobs {
+    RedJob j[RED_JOBS];
+    int count;
+};
+__global__ __launch_bounds__(256) void k_reduce_groups(RedJobs jobs)
 {
+    __shared__ float4 sh[16][16];
+    int b = blockIdx.x, k = 0;
+    for (; k < jobs.count - 1; k++) {
+        const int nb = jobs.j[k].quads / 16 * jobs.j[k].groups;
+        if (b < nb) break;
+        b -= nb;
+    }
+    const RedJob& J = jobs.j[k];
+    const int nx = J.quads / 16, group = b / nx, quad = 16 * (b % nx) + (threadIdx.x & 15), sub = threadIdx.x >> 4;
+    if (group >= J.groups) return;
+    const int per = (J.slots + J.groups - 1) / J.groups, k1 = min(J.slots, (group + 1) * per);
     float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int e = e0; e < e1; e += 4) {
-        const int k = e1 - e;
-        const int i0 = edges[e], i1 = edges[k > 1 ? e + 1 : e], i2 = edges[k > 2 ? e + 2 : e],
-                  i3 = edges[k > 3 ? e + 3 : e];
-        const float4 x0 = ld4(X + (size_t)i0 * stride + col), x1 = ld4(X + (size_t)i1 * stride + col);
-        const float4 x2 = ld4(X + (size_t)i2 * stride + col), x3 = ld4(X + (size_t)i3 * stride + col);
-        add4(s, x0);
-        if (k > 1) add4(s, x1);
-        if (k > 2) add4(s, x2);
-        if (k > 3) add4(s, x3);
+#pragma unroll 4
+    for (int i = group * per + sub; i < k1; i += 16) fma4(s, 1.f, reinterpret_cast<const float4*>(J.part)[(size_t)i * J.quads + quad]);
+    sh[sub][threadIdx.x & 15] = s;
+    __syncthreads();
+    if (sub == 0) {
+        for (int i = 1; i < 16; i++) fma4(s, 1.f, sh[i][threadIdx.x]);
+        reinterpret_cast<float4*>(J.part2)[(size_t)group * J.quads + quad] = s;
     }
-    return s;
 }
-
-// Xc = bf16([Hc | 1/4 sum_{l in c} Hl])
-__global__ void k_gather_clause(const int32_t* __restrict__ c_off, const int32_t* __restrict__ c_edges, int C,
-                                const float* __restrict__ Hl, const float* __restrict__ Hc, bf16_t* __restrict__ Xc)
+__global__ __launch_bounds__(256) void k_reduce_final(RedJobs jobs)
 {
-    const int d = col4();
-    for (int c0 = 4 * wave_global(); c0 < C; c0 += 4 * wave_count()) {
-        const int c = c0 + row_slot();
-        if (c >= C) continue;
-        const float4 s = gather_sum(c_edges, c_off[c], c_off[c + 1], Hl, HID, d);
-        st_bf16x4(Xc + (size_t)c * 128 + d, ld4(Hc + (size_t)c * HID + d));
-        st_bf16x4(Xc + (size_t)c * 128 + 64 + d, mul4(0.25f, s));
+    int b = blockIdx.x, k = 0;
+    for (; k < jobs.count - 1; k++) {
+        const int nb = (4 * jobs.j[k].quads + 255) / 256;
+        if (b < nb) break;
+        b -= nb;
     }
+    const RedJob& J = jobs.j[k];
+    const int i = 256 * b + threadIdx.x;
+    if (i >= 4 * J.quads) return;
+    float s = 0.f;
+#pragma unroll 4
+    for (int g = 0; g < J.groups; g++) s += J.part2[(size_t)g * 4 * J.quads + i];
+    if (i < J.n)
+        J.out[i] = s;
+    else if (J.out2)
+        J.out2[i - J.n] = s;
 }
 
-// Xl = bf16([Hl | 1/8 sum_{c ni l} Hc' | H_{l^1}])
-__global__ void k_gather_lit(const int32_t* __restrict__ l_off, const int32_t* __restrict__ l_edges, int L,
-                             const float* __restrict__ Hl, const float* __restrict__ Hc1, bf16_t* __restrict__ Xl)
-{
-    const int d = col4();
-    for (int l0 = 4 * wave_global(); l0 < L; l0 += 4 * wave_count()) {
-        const int l = l0 + row_slot();
-        if (l >= L) continue;
-        const float4 s = gather_sum(l_edges, l_off[l], l_off[l + 1], Hc1, HID, d);
-        st_bf16x4(Xl + (size_t)l * 192 + d, ld4(Hl + (size_t)l * HID + d));
-        st_bf16x4(Xl + (size_t)l * 192 + 64 + d, mul4(0.125f, s));
-        st_bf16x4(Xl + (size_t)l * 192 + 128 + d, ld4(Hl + (size_t)(l ^ 1) * HID + d));
-    }
-}
-
-// Z = bf16([H_{2v+1} | H_{2v}])
-__global__ void k_build_z(int V, const float* __restrict__ Hl, bf16_t* __restrict__ Z)
-{
-    const int d = threadIdx.x & 63;
-    for (int v = wave_global(); v < V; v += wave_count()) {
-        Z[(size_t)v * 128 + d] = to_bf16(Hl[(size_t)(2 * v + 1) * HID + d]);
-        Z[(size_t)v * 128 + 64 + d] = to_bf16(Hl[(size_t)(2 * v) * HID + d]);
-    }
-}
-
-// Y = R W_y^T + b_y (W_y in BF16); with labels also the loss and dY.
-__global__ void k_head(int V, const float* __restrict__ Rv, const bf16_t* __restrict__ Wyq, const float* __restrict__ th,
-                       float* __restrict__ Y, const float* __restrict__ target, const float* __restrict__ phase,
-                       const float* __restrict__ mask, float alpha, float* __restrict__ dY, float* __restrict__ loss_part)
-{
-    const int d = threadIdx.x & 63;
-    float lsum = 0.f;
-    for (int v = wave_global(); v < V; v += wave_count()) {
-        const float r = Rv[(size_t)v * HID + d];
-        float y0 = r * from_bf16(Wyq[d]);
-        float y1 = r * from_bf16(Wyq[64 + d]);
-        for (int s = 32; s > 0; s >>= 1) {
-            y0 += __shfl_xor(y0, s);
-            y1 += __shfl_xor(y1, s);
-        }
-        y0 += th[O_BY];
-        y1 += th[O_BY + 1];
-        if (d == 0) {
-            Y[2 * (size_t)v] = y0;
-            Y[2 * (size_t)v + 1] = y1;
-            if (target) {
-                const float t = target[v], p = phase[v], mk = mask[v];
-                const float sig = 1.0f / (1.0f + expf(-y1));
-                const float bce = fmaxf(y1, 0.f) - y1 * p + log1pf(expf(-fabsf(y1)));
-                lsum += ((y0 - t) * (y0 - t) + alpha * mk * bce) / (float)V;
-                dY[2 * (size_t)v] = 2.0f * (y0 - t) / (float)V;
-                dY[2 * (size_t)v + 1] = alpha * mk * (sig - p) / (float)V;
-            }
-        }
-    }
-    // this wavefront's share of the loss (k_reduce sums the shares in order)
-    if (target && d == 0) loss_part[wave_global()] = lsum;
-}
-
-// dPo = (dY W_y) * [R > 0] -> BF16, plus this wavefront's partial gradients of b_o, W_y
-// and b_y, laid out as the parameters are (b_o at O_BO, then W_y, then b_y).
-constexpr int HEAD_PART = O_BY + 2 - O_BO;
-__global__ void k_head_bwd(int V, const float* __restrict__ Rv, const float* __restrict__ dY,
-                           const bf16_t* __restrict__ Wyq, bf16_t* __restrict__ dPo, float* __restrict__ part)
-{
-    const int d = threadIdx.x & 63;
-    const float w0 = from_bf16(Wyq[d]), w1 = from_bf16(Wyq[64 + d]);
-    float gw0 = 0.f, gw1 = 0.f, gb = 0.f, gy0 = 0.f, gy1 = 0.f;
-    for (int v = wave_global(); v < V; v += wave_count()) {
-        const float r = Rv[(size_t)v * HID + d];
-        const float a = dY[2 * (size_t)v], b = dY[2 * (size_t)v + 1];
-        gw0 += a * r;
-        gw1 += b * r;
-        const float dp = r > 0.f ? a * w0 + b * w1 : 0.f;
-        gb += dp;
-        dPo[(size_t)v * HID + d] = to_bf16(dp);
-        if (d == 0) {
-            gy0 += a;
-            gy1 += b;
-        }
-    }
-    float* o = part + (size_t)wave_global() * HEAD_PART;
-    o[d] = gb;
-    o[O_WY - O_BO + d] = gw0;
-    o[O_WY - O_BO + 64 + d] = gw1;
-    if (d == 0) {
-        o[O_BY - O_BO] = gy0;
-        o[O_BY - O_BO + 1] = gy1;
-    }
-}
-
-// dH_l^R from dZ
-__global__ void k_bwd_z(int V, const float* __restrict__ dZ, float* __restrict__ dHl)
-{
-    const int d = threadIdx.x & 63;
-    for (int v = wave_global(); v < V; v += wave_count()) {
-        dHl[(size_t)(2 * v + 1) * HID + d] = dZ[(size_t)v * 128 + d];
-        dHl[(size_t)(2 * v) * HID + d] = dZ[(size_t)v * 128 + 64 + d];
-    }
-}
-
-// dP = dH * [H > 0] -> BF16, and this wavefront's partial bias gradient.
-__global__ void k_bwd_mask(int N, const float* __restrict__ dH, const float* __restrict__ H, bf16_t* __restrict__ dP,
-                           float* __restrict__ part)
-{
-    const int d = threadIdx.x & 63;
-    float gb = 0.f;
-    for (int r = wave_global(); r < N; r += wave_count()) {
-        const size_t i = (size_t)r * HID + d;
-        const float g = H[i] > 0.f ? dH[i] : 0.f;
-        gb += g;
-        dP[i] = to_bf16(g);
-    }
-    part[(size_t)wave_global() * HID + d] = gb;
-}
-
-// dH_c' = self part (from the next round, stride sstride) + 1/8 sum_{l in c} dXl[l][64 + d];
-// then masked by [H_c' > 0] into dPc (BF16) with the bias gradient.  Row layout as in the
-// gather kernels; the 4 row slots' bias partials are added (slot 0+1, 2+3, then both)
-// before the wavefront writes its partial.
-__global__ void k_bwd_clause(const int32_t* __restrict__ c_off, const int32_t* __restrict__ c_edges, int C,
-                             const float* __restrict__ self, int sstride, const float* __restrict__ dXl,
-                             const float* __restrict__ Hc1, bf16_t* __restrict__ dPc, float* __restrict__ part)
-{
-    const int d = col4();
-    float4 gb = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int c0 = 4 * wave_global(); c0 < C; c0 += 4 * wave_count()) {
-        const int c = c0 + row_slot();
-        if (c >= C) continue;
-        float4 s = self ? ld4(self + (size_t)c * sstride + d) : make_float4(0.f, 0.f, 0.f, 0.f);
-        add4(s, mul4(0.125f, gather_sum(c_edges, c_off[c], c_off[c + 1], dXl, 192, 64 + d)));
-        const float4 h = ld4(Hc1 + (size_t)c * HID + d);
-        const float4 g = make_float4(h.x > 0.f ? s.x : 0.f, h.y > 0.f ? s.y : 0.f, h.z > 0.f ? s.z : 0.f,
-                                     h.w > 0.f ? s.w : 0.f);
-        add4(gb, g);
-        st_bf16x4(dPc + (size_t)c * HID + d, g);
-    }
-    for (int o = 16; o <= 32; o <<= 1) {
-        gb.x += __shfl_xor(gb.x, o);
-        gb.y += __shfl_xor(gb.y, o);
-        gb.z += __shfl_xor(gb.z, o);
-        gb.w += __shfl_xor(gb.w, o);
-    }
-    if (row_slot() == 0) *reinterpret_cast<float4*>(part + (size_t)wave_global() * HID + d) = gb;
-}
-
-// dH_l = dXl[l][d] + dXl[l^1][128 + d] + 1/4 sum_{c ni l} dXc[c][64 + d]
-__global__ void k_bwd_lit(const int32_t* __restrict__ l_off, const int32_t* __restrict__ l_edges, int L,
-                          const float* __restrict__ dXl, const float* __restrict__ dXc, float* __restrict__ dHl)
-{
-    const int d = col4();
-    for (int l0 = 4 * wave_global(); l0 < L; l0 += 4 * wave_count()) {
-        const int l = l0 + row_slot();
-        if (l >= L) continue;
-        const float4 m = gather_sum(l_edges, l_off[l], l_off[l + 1], dXc, 128, 64 + d);
-        float4 h = ld4(dXl + (size_t)l * 192 + d);
-        add4(h, ld4(dXl + (size_t)(l ^ 1) * 192 + 128 + d));
-        add4(h, mul4(0.25f, m));
-        *reinterpret_cast<float4*>(dHl + (size_t)l * HID + d) = h;
-    }
-}
-
-// this wavefront's partial gradients of the embeddings u_l, v_l, u_c, v_c (parameters
-// 0..255) from dH^0 (the self part of dXc for clauses, stride 128)
-__global__ void k_bwd_embed(const int32_t* __restrict__ l_off, const int32_t* __restrict__ c_off, int L, int C,
-                            const float* __restrict__ dHl, const float* __restrict__ dXc, float* __restrict__ part)
-{
-    const int d = threadIdx.x & 63;
-    float gu = 0.f, gv = 0.f, cu = 0.f, cv = 0.f;
-    for (int r = wave_global(); r < L + C; r += wave_count()) {
-        if (r < L) {
-            const float g = dHl[(size_t)r * HID + d];
-            gu += (float)(l_off[r + 1] - l_off[r]) * 0.125f * g;
-            gv += g;
-        } else {
-            const int c = r - L;
-            const float g = dXc[(size_t)c * 128 + d];
-            cu += (float)(c_off[c + 1] - c_off[c]) * 0.25f * g;
-            cv += g;
-        }
-    }
-    float* o = part + (size_t)wave_global() * O_WC;
-    o[O_UL + d] = gu;
-    o[O_VL + d] = gv;
-    o[O_UC + d] = cu;
-    o[O_VC + d] = cv;
-}
-
+// BF16 copies of the weights: as they are (forward) and transposed (backward)
 __global__ void k_quantize(const float* __restrict__ th, bf16_t* __restrict__ Wc, bf16_t* __restrict__ Wl,
-                           bf16_t* __restrict__ Wo, bf16_t* __restrict__ Wy)
+                           bf16_t* __restrict__ Wo, bf16_t* __restrict__ Wct, bf16_t* __restrict__ Wlt,
+                           bf16_t* __restrict__ Wot, bf16_t* __restrict__ Wy)
 {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < 64 * 192; i += gridDim.x * blockDim.x) {
-        if (i < 64 * 128) Wc[i] = to_bf16(th[O_WC + i]);
-        Wl[i] = to_bf16(th[O_WL + i]);
-        if (i < 64 * 128) Wo[i] = to_bf16(th[O_WO + i]);
+        Wl[i] = Wlt[(i % 192) * 64 + i / 192] = to_bf16(th[O_WL + i]);
+        if (i < 64 * 128) {
+            Wc[i] = Wct[(i % 128) * 64 + i / 128] = to_bf16(th[O_WC + i]);
+            Wo[i] = Wot[(i % 128) * 64 + i / 128] = to_bf16(th[O_WO + i]);
+        }
         if (i < 128) Wy[i] = to_bf16(th[O_WY + i]);
     }
 }
@@ -569,39 +789,36 @@ __global__ void k_adam(float* __restrict__ th, const float* __restrict__ g, floa
 using namespace gpsat;
 using namespace gpsat::gnn;
 
-// Kernels that leave per-wavefront partials run on a fixed grid of RED_BLOCKS workgroups
-// of 4 wavefronts (one partial slot per wavefront; 16 wavefronts per CU to hide the gather
-// latency); the weight-gradient products on at most DW_BLOCKS workgroups of 4 wavefronts
-// (one partial matrix each).
-constexpr int RED_BLOCKS = 4096;
-constexpr int RED_WAVES = 4 * RED_BLOCKS;
-constexpr int DW_BLOCKS = 1024;
-constexpr size_t PART_FLOATS = std::max<size_t>((size_t)DW_BLOCKS * 64 * 192, (size_t)RED_WAVES * O_WC);
-// Slot groups of the two-stage weight-gradient reduction, and their partials after
-// PART_FLOATS in the same buffer.
-constexpr int WIDE_GROUPS = 32;
-constexpr size_t PART2_FLOATS = (size_t)WIDE_GROUPS * 64 * 192;
+// Workgroups of the weight-gradient products (one partial matrix each; two workgroups per CU, as
+// more of them write more partials and gain nothing) and of the embedding gradient.
+constexpr int DW_BLOCKS = 512;
+constexpr int EMBED_BLOCKS = 2048;
+constexpr int MAX_GROUPS = 32;
 
-// One batch's activations, carved from the model's arena (see gpsat_gnn_model).
+// One pass's activations, carved from the model's arena (see gpsat_gnn_model); the second part
+// only for a pass with gradients.
 struct Acts {
-    std::vector<float*> Hl, Hc;
-    std::vector<bf16_t*> Xc, Xl;
-    bf16_t *Z = nullptr, *dP = nullptr;
-    float *Rv = nullptr, *dY = nullptr, *dXa = nullptr, *dXb = nullptr, *dHl = nullptr, *loss = nullptr;
+    float *Hl = nullptr, *Hc = nullptr;
+    bf16_t *Xc = nullptr, *Xl = nullptr, *Z = nullptr;                        // [rounds][rows][128]
+    bf16_t *dPc = nullptr, *dPl = nullptr, *dPo = nullptr;                    // [rounds][rows][64]
+    uint2 *mask_c = nullptr, *mask_l = nullptr;                               // [rounds][rows]
+    float *Sl = nullptr, *Ml = nullptr, *Sc = nullptr, *Mc = nullptr, *loss = nullptr;
+    float *part_o = nullptr, *part_l = nullptr, *part_c = nullptr, *part_el = nullptr, *part_ec = nullptr;
+    float *part_wl = nullptr, *part_wc = nullptr, *part_wo = nullptr, *part2 = nullptr;
 };
 
-// A model: FP32 master parameters, gradient, Adam moments, BF16 weight copies, the partials
-// of the gradient reductions, and a grow-only arena that holds the activations of the graph
-// being run.  Graphs own only their incidence structure and labels, so a training loop keeps
-// every batch's graph across steps without holding every batch's activations; calls on one
-// model therefore run one at a time.
+// A model: FP32 master parameters, gradient, Adam moments, BF16 weight copies, and a grow-only
+// arena that holds the activations and gradient partials of the pass being run.  Graphs own
+// only their incidence structure and labels, so a training loop keeps every batch's graph
+// across steps without holding every batch's activations; calls on one model therefore run
+// one at a time.
 struct gpsat_gnn_model {
     float* th = nullptr;
     float* grad = nullptr;
     float* m = nullptr;
     float* v = nullptr;
-    float* part = nullptr;
     bf16_t *Wc = nullptr, *Wl = nullptr, *Wo = nullptr, *Wy = nullptr;
+    bf16_t *Wct = nullptr, *Wlt = nullptr, *Wot = nullptr;
     char* arena = nullptr;
     size_t arena_bytes = 0;
     int64_t step = 0;
@@ -643,15 +860,18 @@ struct gpsat_gnn_graph {
 
 namespace {
 
-int grid_rows(int64_t rows, int waves_per_block = 4)
-{
-    const int64_t b = (rows + waves_per_block - 1) / waves_per_block;
-    return (int)std::max<int64_t>(1, std::min<int64_t>(b, 65536));
-}
+// Workgroups that cover N rows, 16 per wavefront and `tiles` of those one after another: a
+// multiple of 8, see xcd_block.
+int row_blocks(int64_t N, int tiles = 1) { return (int)(((N + 64 * tiles - 1) / (64 * tiles) + 7) / 8 * 8); }
+// The readout's wavefronts take several tiles in turn where there are enough to fill the GPU:
+// both forms of W_o are staged per workgroup.
+int readout_tiles(int V) { return std::max(1, std::min(4, V / (16 * 2048))); }
+int dw_blocks(int64_t rows) { return (int)std::max<int64_t>(1, std::min<int64_t>(DW_BLOCKS, (rows + 63) / 64)); }
+int red_groups(int64_t slots) { return (int)std::max<int64_t>(1, std::min<int64_t>(MAX_GROUPS, slots / 64)); }
 
-// Lay a graph's activations out in `base` (nullptr: only count); returns the bytes used.
+// Lay a pass's activations out in `base` (nullptr: only count); returns the bytes used.
 // Every piece starts 256-byte aligned.
-size_t carve(const gpsat_gnn_graph* g, char* base, Acts& a)
+size_t carve(const gpsat_gnn_graph* g, bool train, char* base, Acts& a)
 {
     size_t off = 0;
     auto take = [&](auto*& p, size_t count) {
@@ -660,32 +880,38 @@ size_t carve(const gpsat_gnn_graph* g, char* base, Acts& a)
         off += (std::max<size_t>(count, 1) * sizeof(T) + 255) & ~(size_t)255;
     };
     const size_t L = g->L, C = g->C, V = g->V, R = g->R;
-    a.Hl.assign(R + 1, nullptr);
-    a.Hc.assign(R + 1, nullptr);
-    a.Xc.assign(R, nullptr);
-    a.Xl.assign(R, nullptr);
-    for (size_t t = 0; t <= R; t++) {
-        take(a.Hl[t], L * HID);
-        take(a.Hc[t], C * HID);
-        if (t < R) take(a.Xc[t], C * 128);
-        if (t < R) take(a.Xl[t], L * 192);
-    }
-    const size_t maxn = std::max({L, C, V});
+    take(a.Hl, L * HID);
+    take(a.Hc, C * HID);
+    if (!train) return off;
+    take(a.Xc, R * C * 128);
+    take(a.Xl, R * L * 128);
     take(a.Z, V * 128);
-    take(a.dP, maxn * HID);
-    take(a.Rv, V * HID);
-    take(a.dY, V * 2);
-    take(a.dXa, std::max(L * 192, V * 128));
-    take(a.dXb, C * 128);
-    take(a.dHl, L * HID);
-    take(a.loss, 1);
+    take(a.dPc, R * C * HID);
+    take(a.dPl, R * L * HID);
+    take(a.dPo, V * HID);
+    take(a.mask_c, R * C);
+    take(a.mask_l, R * L);
+    take(a.Sl, L * HID);
+    take(a.Ml, L * HID);
+    take(a.Sc, C * HID);
+    take(a.Mc, C * HID);
+    take(a.loss, HEAD_PART - HEAD_GRADS);   // (the rest of a readout partial's row)
+    take(a.part_o, (size_t)row_blocks(V, readout_tiles((int)V)) * HEAD_PART);
+    take(a.part_l, R * row_blocks(L) * HID);
+    take(a.part_c, R * row_blocks(C) * HID);
+    take(a.part_el, (size_t)EMBED_BLOCKS * 2 * HID);
+    take(a.part_ec, (size_t)row_blocks(C) * 2 * HID);
+    take(a.part_wl, (size_t)dw_blocks(R * L) * 64 * 192);
+    take(a.part_wc, (size_t)dw_blocks(R * C) * 64 * 128);
+    take(a.part_wo, (size_t)dw_blocks(V) * 64 * 128);
+    take(a.part2, (size_t)MAX_GROUPS * (HEAD_PART + 6 * HID + 64 * (192 + 128 + 128)));
     return off;
 }
 
-// The activations of graph g in model m's arena (grown if g needs more).
-hipError_t acts_for(gpsat_gnn_model* m, gpsat_gnn_graph* g, Acts& a)
+// The activations of a pass of graph g in model m's arena (grown if it needs more).
+hipError_t acts_for(gpsat_gnn_model* m, gpsat_gnn_graph* g, bool train, Acts& a)
 {
-    const size_t need = carve(g, nullptr, a);
+    const size_t need = carve(g, train, nullptr, a);
     if (need > m->arena_bytes) {
         hipError_t e = hipDeviceSynchronize();
         if (e != hipSuccess) return e;
@@ -696,97 +922,102 @@ hipError_t acts_for(gpsat_gnn_model* m, gpsat_gnn_graph* g, Acts& a)
         if (e != hipSuccess) return e;
         m->arena_bytes = need;
     }
-    carve(g, m->arena, a);
+    carve(g, train, m->arena, a);
     return hipSuccess;
 }
 
-template <bool ACC>
-void reduce(const float* part, int slots, int width, float* out, hipStream_t st)
+template <bool LIT, bool FIRST, bool TRAIN>
+void layer(gpsat_gnn_model* m, gpsat_gnn_graph* g, const Acts& a, int t)
 {
-    if (width >= 4096 && slots > 2 * WIDE_GROUPS && width % 4 == 0 && (size_t)width * WIDE_GROUPS <= PART2_FLOATS) {
-        float* part2 = const_cast<float*>(part) + PART_FLOATS;
-        hipLaunchKernelGGL(k_reduce_wide_split, dim3((width / 4 + 255) / 256, WIDE_GROUPS), dim3(256), 0, st, part,
-                           slots, width, part2);
-        hipLaunchKernelGGL(k_reduce_wide<ACC>, dim3((width + 255) / 256), dim3(256), 0, st, part2, WIDE_GROUPS, width,
-                           out);
-    } else if (width >= 4096)
-        hipLaunchKernelGGL(k_reduce_wide<ACC>, dim3((width + 255) / 256), dim3(256), 0, st, part, slots, width, out);
-    else
-        hipLaunchKernelGGL(k_reduce_tree<ACC>, dim3(width), dim3(256), 0, st, part, slots, width, out);
+    const int N = LIT ? g->L : g->C;
+    if (N == 0) return;
+    hipLaunchKernelGGL((k_layer<LIT, FIRST, TRAIN>), dim3(row_blocks(N)), dim3(256), 0, g->st, LIT ? g->l_off : g->c_off,
+                       LIT ? g->l_edges : g->c_edges, LIT ? g->c_off : g->l_off, N, m->th,
+                       LIT ? m->Wl : m->Wc, m->th + (LIT ? O_BL : O_BC), LIT ? a.Hc : a.Hl, LIT ? a.Hl : a.Hc,
+                       TRAIN ? (LIT ? a.Xl : a.Xc) + (size_t)t * N * 128 : nullptr,
+                       TRAIN ? (LIT ? a.mask_l : a.mask_c) + (size_t)t * N : nullptr);
 }
 
-// gW += dP^T X over N nodes (weight gradient of one dense layer)
-template <int K>
-void dense_dw(gpsat_gnn_model* m, const bf16_t* dP, const bf16_t* X, int N, float* gW, hipStream_t st)
+// Forward pass, readout included (TRAIN: with the loss and the readout's gradients).
+template <bool TRAIN>
+hipError_t forward_pass(gpsat_gnn_model* m, gpsat_gnn_graph* g, const Acts& a, float alpha)
 {
-    const int nb = std::max(1, std::min(DW_BLOCKS, (N + 63) / 64));
-    hipLaunchKernelGGL((k_dense_bwd_dw<K>), dim3(nb), dim3(256), 0, st, dP, X, m->part, N);
-    reduce<true>(m->part, nb, 64 * K, gW, st);
-}
-
-hipError_t forward_pass(gpsat_gnn_model* m, gpsat_gnn_graph* g, const Acts& a)
-{
-    hipStream_t st = g->st;
     if (m->dirty) {
-        hipLaunchKernelGGL(k_quantize, dim3(48), dim3(256), 0, st, m->th, m->Wc, m->Wl, m->Wo, m->Wy);
+        hipLaunchKernelGGL(k_quantize, dim3(48), dim3(256), 0, g->st, m->th, m->Wc, m->Wl, m->Wo, m->Wct, m->Wlt, m->Wot,
+                           m->Wy);
         m->dirty = false;
     }
-    const int64_t rows = (int64_t)(g->L + g->C) * HID;
-    hipLaunchKernelGGL(k_embed, dim3((int)std::min<int64_t>((rows + 255) / 256, 65536)), dim3(256), 0, st, g->l_off,
-                       g->c_off, g->L, g->C, m->th, a.Hl[0], a.Hc[0]);
-    for (int t = 0; t < g->R; t++) {
-        hipLaunchKernelGGL(k_gather_clause, dim3(grid_rows((g->C + 3) / 4)), dim3(256), 0, st, g->c_off, g->c_edges, g->C,
-                           a.Hl[t], a.Hc[t], a.Xc[t]);
-        hipLaunchKernelGGL((k_dense_fwd<128>), dim3((g->C + 63) / 64), dim3(256), 0, st, a.Xc[t], m->Wc,
-                           m->th + O_BC, a.Hc[t + 1], g->C);
-        hipLaunchKernelGGL(k_gather_lit, dim3(grid_rows((g->L + 3) / 4)), dim3(256), 0, st, g->l_off, g->l_edges, g->L, a.Hl[t],
-                           a.Hc[t + 1], a.Xl[t]);
-        hipLaunchKernelGGL((k_dense_fwd<192>), dim3((g->L + 63) / 64), dim3(256), 0, st, a.Xl[t], m->Wl,
-                           m->th + O_BL, a.Hl[t + 1], g->L);
+    layer<false, true, TRAIN>(m, g, a, 0);
+    layer<true, true, TRAIN>(m, g, a, 0);
+    for (int t = 1; t < g->R; t++) {
+        layer<false, false, TRAIN>(m, g, a, t);
+        layer<true, false, TRAIN>(m, g, a, t);
     }
-    hipLaunchKernelGGL(k_build_z, dim3(grid_rows(g->V)), dim3(256), 0, st, g->V, a.Hl[g->R], a.Z);
-    hipLaunchKernelGGL((k_dense_fwd<128>), dim3((g->V + 63) / 64), dim3(256), 0, st, a.Z, m->Wo, m->th + O_BO, a.Rv,
-                       g->V);
+    const int tiles = readout_tiles(g->V);
+    if (g->V)
+        hipLaunchKernelGGL((k_readout<TRAIN>), dim3(row_blocks(g->V, tiles)), dim3(256), 0, g->st, g->V, tiles, a.Hl, m->Wo, m->Wot,
+                           m->Wy, m->th, g->Y, g->target, g->phase, g->mask, alpha, a.Z, a.dPo, a.Sl, a.part_o);
     return hipGetLastError();
 }
 
-hipError_t head(gpsat_gnn_model* m, gpsat_gnn_graph* g, const Acts& a, bool labels, float alpha)
+template <bool LIT, bool SELF, bool GATHER, bool LAST>
+void layer_bwd(gpsat_gnn_model* m, gpsat_gnn_graph* g, const Acts& a, int t)
 {
-    hipLaunchKernelGGL(k_head, dim3(RED_BLOCKS), dim3(256), 0, g->st, g->V, a.Rv, m->Wy, m->th, g->Y,
-                       labels ? g->target : nullptr, g->phase, g->mask, alpha, a.dY, m->part);
-    if (labels) reduce<false>(m->part, RED_WAVES, 1, a.loss, g->st);
-    return hipGetLastError();
+    const int N = LIT ? g->L : g->C;
+    if (N == 0) return;
+    hipLaunchKernelGGL((k_layer_bwd<LIT, SELF, GATHER, LAST>), dim3(row_blocks(N)), dim3(256), 0, g->st,
+                       LIT ? g->l_off : g->c_off, LIT ? g->l_edges : g->c_edges, N, LIT ? m->Wlt : m->Wct,
+                       (LIT ? a.mask_l : a.mask_c) + (size_t)t * N, LIT ? a.Mc : a.Ml, LIT ? a.Sl : a.Sc,
+                       (LIT ? a.dPl : a.dPc) + (size_t)t * N * HID, LIT ? a.Ml : a.Mc,
+                       (LIT ? a.part_l : a.part_c) + (size_t)t * row_blocks(N) * HID, a.part_ec);
 }
 
+// Backward pass from the readout's gradients to m->grad (every element written) and the loss.
 hipError_t backward_pass(gpsat_gnn_model* m, gpsat_gnn_graph* g, const Acts& a)
 {
     hipStream_t st = g->st;
-    // head and readout
-    hipLaunchKernelGGL(k_head_bwd, dim3(RED_BLOCKS), dim3(256), 0, st, g->V, a.Rv, a.dY, m->Wy, a.dP, m->part);
-    reduce<true>(m->part, RED_WAVES, HEAD_PART, m->grad + O_BO, st);
-    dense_dw<128>(m, a.dP, a.Z, g->V, m->grad + O_WO, st);
-    hipLaunchKernelGGL((k_dense_bwd_dx<128>), dim3((g->V + 63) / 64), dim3(256), 0, st, a.dP, m->Wo, a.dXa, g->V);
-    hipLaunchKernelGGL(k_bwd_z, dim3(grid_rows(g->V)), dim3(256), 0, st, g->V, a.dXa, a.dHl);
-    // dXa holds dXl (L x 192), dXb holds dXc (C x 128)
-    const float* self = nullptr;
-    for (int t = g->R - 1; t >= 0; t--) {
-        hipLaunchKernelGGL(k_bwd_mask, dim3(RED_BLOCKS), dim3(256), 0, st, g->L, a.dHl, a.Hl[t + 1], a.dP, m->part);
-        reduce<true>(m->part, RED_WAVES, HID, m->grad + O_BL, st);
-        dense_dw<192>(m, a.dP, a.Xl[t], g->L, m->grad + O_WL, st);
-        hipLaunchKernelGGL((k_dense_bwd_dx<192>), dim3((g->L + 63) / 64), dim3(256), 0, st, a.dP, m->Wl, a.dXa, g->L);
-        // the self part of dH_c^{t+1} comes from round t+1's clause update (dXc of that round)
-        hipLaunchKernelGGL(k_bwd_clause, dim3(RED_BLOCKS), dim3(256), 0, st, g->c_off, g->c_edges, g->C, self, 128,
-                           a.dXa, a.Hc[t + 1], a.dP, m->part);
-        reduce<true>(m->part, RED_WAVES, HID, m->grad + O_BC, st);
-        dense_dw<128>(m, a.dP, a.Xc[t], g->C, m->grad + O_WC, st);
-        hipLaunchKernelGGL((k_dense_bwd_dx<128>), dim3((g->C + 63) / 64), dim3(256), 0, st, a.dP, m->Wc, a.dXb, g->C);
-        hipLaunchKernelGGL(k_bwd_lit, dim3(grid_rows((g->L + 3) / 4)), dim3(256), 0, st, g->l_off, g->l_edges, g->L, a.dXa,
-                           a.dXb, a.dHl);
-        self = a.dXb;
+    const int R = g->R, L = g->L, C = g->C, V = g->V;
+    const int sl = L ? row_blocks(L) : 0, sc = C ? row_blocks(C) : 0;
+    for (int t = R - 1; t >= 0; t--) {
+        const bool top = t == R - 1;
+        if (top)
+            layer_bwd<true, true, false, false>(m, g, a, t);
+        else
+            layer_bwd<true, true, true, false>(m, g, a, t);
+        if (top && t)
+            layer_bwd<false, false, true, false>(m, g, a, t);
+        else if (top)
+            layer_bwd<false, false, true, true>(m, g, a, t);
+        else if (t)
+            layer_bwd<false, true, true, false>(m, g, a, t);
+        else
+            layer_bwd<false, true, true, true>(m, g, a, t);
     }
-    hipLaunchKernelGGL(k_bwd_embed, dim3(RED_BLOCKS), dim3(256), 0, st, g->l_off, g->c_off, g->L, g->C, a.dHl, a.dXb,
-                       m->part);
-    reduce<true>(m->part, RED_WAVES, O_WC, m->grad, st);
+    const int bl = dw_blocks((int64_t)R * L), bc = dw_blocks((int64_t)R * C), bo = dw_blocks(V);
+    hipLaunchKernelGGL((k_dense_dw<192>), dim3(bl), dim3(256), 0, st, a.dPl, a.Xl, a.part_wl, (int64_t)R * L);
+    hipLaunchKernelGGL((k_dense_dw<128>), dim3(bc), dim3(256), 0, st, a.dPc, a.Xc, a.part_wc, (int64_t)R * C);
+    hipLaunchKernelGGL((k_dense_dw<128>), dim3(bo), dim3(256), 0, st, a.dPo, a.Z, a.part_wo, (int64_t)V);
+    hipLaunchKernelGGL(k_bwd_embed, dim3(EMBED_BLOCKS), dim3(256), 0, st, g->l_off, g->l_edges, L, a.Sl, a.Mc, a.part_el);
+    RedJobs jobs{};
+    int nb1 = 0, nb2 = 0;
+    float* part2 = a.part2;
+    auto job = [&](const float* part, int slots, int width, float* out, int n, float* out2 = nullptr) {
+        const int gr = red_groups(slots);
+        jobs.j[jobs.count++] = RedJob{part, part2, out, out2, slots, width / 4, gr, n};
+        part2 += (size_t)gr * width;
+        nb1 += width / 64 * gr;
+        nb2 += (width + 255) / 256;
+    };
+    job(a.part_o, V ? row_blocks(V, readout_tiles(V)) : 0, HEAD_PART, m->grad + O_BO, HEAD_GRADS, a.loss);
+    job(a.part_l, R * sl, HID, m->grad + O_BL, HID);
+    job(a.part_c, R * sc, HID, m->grad + O_BC, HID);
+    job(a.part_el, EMBED_BLOCKS, 2 * HID, m->grad + O_UL, 2 * HID);
+    job(a.part_ec, sc, 2 * HID, m->grad + O_UC, 2 * HID);
+    job(a.part_wl, bl, 64 * 192, m->grad + O_WL, 64 * 192);
+    job(a.part_wc, bc, 64 * 128, m->grad + O_WC, 64 * 128);
+    job(a.part_wo, bo, 64 * 128, m->grad + O_WO, 64 * 128);
+    hipLaunchKernelGGL(k_reduce_groups, dim3(nb1), dim3(256), 0, st, jobs);
+    hipLaunchKernelGGL(k_reduce_final, dim3(nb2), dim3(256), 0, st, jobs);
     return hipGetLastError();
 }
 
@@ -819,13 +1050,15 @@ int gpsat_gnn_model_create(const float* theta, gpsat_gnn_model** out)
     gpsat_gnn_model* m = new gpsat_gnn_model();
     hipError_t e = hipMalloc(&m->th, 4 * N_PARAMS);
     if (e == hipSuccess) e = hipMalloc(&m->grad, 4 * N_PARAMS);
-    if (e == hipSuccess) e = hipMalloc(&m->part, 4 * (PART_FLOATS + PART2_FLOATS));
     if (e == hipSuccess) e = hipMalloc(&m->m, 4 * N_PARAMS);
     if (e == hipSuccess) e = hipMalloc(&m->v, 4 * N_PARAMS);
     if (e == hipSuccess) e = hipMalloc(&m->Wc, 2 * 64 * 128);
     if (e == hipSuccess) e = hipMalloc(&m->Wl, 2 * 64 * 192);
     if (e == hipSuccess) e = hipMalloc(&m->Wo, 2 * 64 * 128);
     if (e == hipSuccess) e = hipMalloc(&m->Wy, 2 * 128);
+    if (e == hipSuccess) e = hipMalloc(&m->Wct, 2 * 64 * 128);
+    if (e == hipSuccess) e = hipMalloc(&m->Wlt, 2 * 64 * 192);
+    if (e == hipSuccess) e = hipMalloc(&m->Wot, 2 * 64 * 128);
     if (e == hipSuccess) e = hipMemcpy(m->th, theta, 4 * N_PARAMS, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemset(m->m, 0, 4 * N_PARAMS);
     if (e == hipSuccess) e = hipMemset(m->v, 0, 4 * N_PARAMS);
@@ -842,8 +1075,8 @@ int gpsat_gnn_model_destroy(gpsat_gnn_model* m)
 {
     if (!m) return GPSAT_OK;
     (void)hipDeviceSynchronize();
-    for (void* p : {(void*)m->th, (void*)m->grad, (void*)m->m, (void*)m->v, (void*)m->part, (void*)m->arena,
-                    (void*)m->Wc, (void*)m->Wl, (void*)m->Wo, (void*)m->Wy})
+    for (void* p : {(void*)m->th, (void*)m->grad, (void*)m->m, (void*)m->v, (void*)m->arena, (void*)m->Wc,
+                    (void*)m->Wl, (void*)m->Wo, (void*)m->Wy, (void*)m->Wct, (void*)m->Wlt, (void*)m->Wot})
         (void)hipFree(p);
     delete m;
     return GPSAT_OK;
@@ -944,9 +1177,8 @@ int gpsat_gnn_forward(gpsat_gnn_model* m, gpsat_gnn_graph* g, float* y)
         return GPSAT_ERR_ARG;
     }
     Acts a;
-    GNN_TRY(acts_for(m, g, a));
-    GNN_TRY(forward_pass(m, g, a));
-    GNN_TRY(head(m, g, a, false, 0.f));
+    GNN_TRY(acts_for(m, g, false, a));
+    GNN_TRY(forward_pass<false>(m, g, a, 0.f));
     GNN_TRY(hipMemcpyAsync(y, g->Y, 8 * (size_t)g->V, hipMemcpyDeviceToHost, g->st));
     GNN_TRY(hipStreamSynchronize(g->st));
     return GPSAT_OK;
@@ -959,10 +1191,8 @@ int gpsat_gnn_loss_grad(gpsat_gnn_model* m, gpsat_gnn_graph* g, float alpha, flo
         return GPSAT_ERR_ARG;
     }
     Acts a;
-    GNN_TRY(acts_for(m, g, a));
-    GNN_TRY(hipMemsetAsync(m->grad, 0, 4 * N_PARAMS, g->st));
-    GNN_TRY(forward_pass(m, g, a));
-    GNN_TRY(head(m, g, a, true, alpha));
+    GNN_TRY(acts_for(m, g, true, a));
+    GNN_TRY(forward_pass<true>(m, g, a, alpha));
     GNN_TRY(backward_pass(m, g, a));
     if (loss) GNN_TRY(hipMemcpyAsync(loss, a.loss, 4, hipMemcpyDeviceToHost, g->st));
     if (grad) GNN_TRY(hipMemcpyAsync(grad, m->grad, 4 * N_PARAMS, hipMemcpyDeviceToHost, g->st));
@@ -978,10 +1208,8 @@ int gpsat_gnn_train_step(gpsat_gnn_model* m, gpsat_gnn_graph* g, float alpha, fl
         return GPSAT_ERR_ARG;
     }
     Acts a;
-    GNN_TRY(acts_for(m, g, a));
-    GNN_TRY(hipMemsetAsync(m->grad, 0, 4 * N_PARAMS, g->st));
-    GNN_TRY(forward_pass(m, g, a));
-    GNN_TRY(head(m, g, a, true, alpha));
+    GNN_TRY(acts_for(m, g, true, a));
+    GNN_TRY(forward_pass<true>(m, g, a, alpha));
     GNN_TRY(backward_pass(m, g, a));
     m->step++;
     const float b1 = 0.9f, b2 = 0.999f;
