@@ -288,6 +288,20 @@ static void packk_instance(const int32_t* lits, const int64_t* coff, int32_t m, 
     }
 }
 
+// The wide form: four 16-bit slots, in clause order (no placement pass, which would cost the
+// caller about 1 us a clause).
+static void packk_wide_instance(const int32_t* lits, const int64_t* coff, int32_t m, int32_t W, uint32_t* out)
+{
+    const uint32_t fl = 32u * (uint32_t)W + 1u;
+    for (int32_t c = 0; c < m; c++) {
+        uint32_t code[kPkkWideMaxLen] = {fl, fl, fl, fl};
+        const int len = (int)(coff[c + 1] - coff[c]);
+        for (int k = 0; k < len; k++) code[k] = (uint32_t)lits[coff[c] + k];
+        out[2 * c] = code[0] | code[1] << 16;
+        out[2 * c + 1] = code[2] | code[3] << 16;
+    }
+}
+
 int gpsat_batch_create(const int32_t* lits, const int64_t* clause_off, const int64_t* inst_clause_off,
                        const int32_t* n_vars, int32_t n_inst, gpsat_batch** out)
 {
@@ -313,7 +327,7 @@ int gpsat_batch_create(const int32_t* lits, const int64_t* clause_off, const int
     d.h_coff.resize(M + n_inst);
     d.h_lits.assign(lits ? lits + l0 : nullptr, lits ? lits + l0 + L : nullptr);
     int64_t wbase = 0;
-    bool fast3 = true, every3 = true, packk = true;
+    bool fast3 = true, every3 = true, packk = true, packw = true;
     std::vector<uint8_t> h_klen(n_inst, 0);
     for (int32_t i = 0; i < n_inst; i++) {
         const int64_t cb = inst_clause_off[i], ce = inst_clause_off[i + 1];
@@ -353,6 +367,7 @@ int gpsat_batch_create(const int32_t* lits, const int64_t* clause_off, const int
             max_len = std::max(max_len, len);
         }
         packk = packk && pkk_fits(mi.n, (int)std::min<int64_t>(max_len, INT32_MAX));
+        packw = packw && pkk_wide_fits(mi.n, (int)std::min<int64_t>(max_len, INT32_MAX));
         h_klen[i] = (uint8_t)std::min<int64_t>(max_len, 255);
         fast3 = fast3 && all3 && fast3_fits(mi.n, mi.m);
         every3 = every3 && all3;
@@ -387,7 +402,8 @@ int gpsat_batch_create(const int32_t* lits, const int64_t* clause_off, const int
     // (GPSAT_PKK_FOR_FAST3=1 builds them for 3-literal batches too, so both kernels can be
     // compared on one batch with eval_fast3 = 0)
     const char* pf3 = getenv("GPSAT_PKK_FOR_FAST3");
-    const bool use_pkk = packk && (!d.fast3 || (pf3 && atoi(pf3) != 0)) && n_inst > 0 && M > 0;
+    const bool use_pkk = (packk || packw) && (!d.fast3 || (pf3 && atoi(pf3) != 0)) && n_inst > 0 && M > 0;
+    d.pkk_wide = use_pkk && !packk;
     if (use_pkk) {
         h_pkk.resize(2 * M);
         const int32_t T = (int32_t)std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
@@ -395,8 +411,11 @@ int gpsat_batch_create(const int32_t* lits, const int64_t* clause_off, const int
         const auto work = [&](int32_t t) {
             for (int32_t i = t; i < n_inst; i += nt) {
                 const int64_t cb = inst_clause_off[i];
-                packk_instance(lits, clause_off + cb, d.h_meta[i].m, words_per_row(d.h_meta[i].n),
-                               std::max<int>(3, h_klen[i]), h_pkk.data() + 2 * (cb - c0));
+                const int32_t m = d.h_meta[i].m, W = words_per_row(d.h_meta[i].n);
+                if (d.pkk_wide)
+                    packk_wide_instance(lits, clause_off + cb, m, W, h_pkk.data() + 2 * (cb - c0));
+                else
+                    packk_instance(lits, clause_off + cb, m, W, std::max<int>(3, h_klen[i]), h_pkk.data() + 2 * (cb - c0));
             }
         };
         std::vector<std::thread> pool;

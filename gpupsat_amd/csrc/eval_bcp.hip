@@ -924,14 +924,24 @@ __global__ __launch_bounds__(256) void k_eval_bcp3(const InstMeta* __restrict__ 
 }
 
 // ---------------------------------------------------------------------------------------
-// Packed general path: instances whose clauses hold at most 6 literals (any mix of lengths),
-// with n <= 496 (W <= 31 words per row) and any m.  Clause c is one 8-byte word pair of the
-// batch's pkk array: slot k's 10-bit literal code sits at bit 10 * (k % 3) of word k / 3.
+// Packed general path: instances whose clauses hold at most 6 literals (any mix of lengths)
+// with n <= 496 (W <= 31 words per row), or at most 4 literals with n <= 2016 (WIDE), and any
+// m.  A clause is one 8-byte word pair of the batch's pkk array: six slots of 10 bits, slot k's
+// literal code at bit 10 * (k % 3) of word k / 3, or (WIDE) four of 16 bits, slot k's at bit
+// 16 * (k % 2) of word k / 2.
 // Slots past the clause's length name the always-false slot 32W + 1, which is false in every
 // row and never implied, so a padded clause has the status and the unit literal of the
 // clause itself; lanes past m name the zero slot 32W (neither true nor false), which gives
 // no status and no unit.  The body runs for K = the instance's longest clause (at least 3),
 // so a 3-SAT instance reads three slots per clause and a 5-SAT one five.
+//
+// Why WIDE: the CSR kernel chases offsets and literals from HBM with one wavefront per instance.
+// On 1,000 4-colourings of n = 600 (150 clauses of 4 literals, 2,250 of 2, p = 0.05) it takes
+// 167-184 us, where the rows and clauses of the batch take 10 at the HBM rate; four wavefronts
+// over word pairs take 32 (n = 500, 1,024, 1,600 in smaller batches: 128 -> 22, 161 -> 26, 214
+// -> 32).  The limits are the mask table's: 512 bytes per row word, 64 KB at W = 126.  Sweeping
+// the clauses of at most 2 literals apart, with 2 slot reads each, gained nothing at n = 500-600
+// (9% at n = 1,024) and cost the 10-bit form 14% on small colourings (81 instead of 72 VGPRs).
 //
 // One workgroup of NW wavefronts per instance: the waves share the instance's mask table in
 // LDS (the 3-literal kernel's slot l = {T(l), T(l ^ 1)}, 16 bytes, partner slot at address
@@ -951,7 +961,15 @@ constexpr int kPkAhead = 4;
 
 __host__ __device__ constexpr int pk_lds_words(int W) { return 128 * W + 8 + 8 + 192; }
 
-template <int K>
+// literal code in slot k of a clause word pair: six of 10 bits, or (WIDE) four of 16
+template <bool WIDE>
+__device__ __forceinline__ uint32_t pk_code(const uint2& w, int k)
+{
+    return WIDE ? __builtin_amdgcn_ubfe(k < 2 ? w.x : w.y, 16 * (k % 2), 16)
+                : __builtin_amdgcn_ubfe(k < 3 ? w.x : w.y, 10 * (k % 3), 10);
+}
+
+template <int K, bool WIDE>
 struct PkGroup {
     uint2 w;            // the lane's clause word pair (slot addresses are formed again from it
                         // where an implication is written, so they are not held in registers)
@@ -959,44 +977,44 @@ struct PkGroup {
 };
 
 // byte address of slot k of the clause word pair w in the table at tabb
-template <int K>
+template <bool WIDE>
 __device__ __forceinline__ uint32_t pk_addr(const uint2& w, uint32_t tabb, int k)
 {
-    return tabb + 16u * __builtin_amdgcn_ubfe(k < 3 ? w.x : w.y, 10 * (k % 3), 10);
+    return tabb + 16u * pk_code<WIDE>(w, k);
 }
 
-template <int K>
-__device__ __forceinline__ void pk_fetch(uint2 w, uint32_t tabb, PkGroup<K>& gr)
+template <int K, bool WIDE>
+__device__ __forceinline__ void pk_fetch(uint2 w, uint32_t tabb, PkGroup<K, WIDE>& gr)
 {
     gr.w = w;
 #pragma unroll
-    for (int k = 0; k < K; k++) gr.q[k] = lds_read16(pk_addr<K>(w, tabb, k));
+    for (int k = 0; k < K; k++) gr.q[k] = lds_read16(pk_addr<WIDE>(w, tabb, k));
 }
 
 // A group's slots in the compacted table of at most 32 open rows: 8-byte slots {T, F}.
-template <int K>
+template <int K, bool WIDE>
 struct PkGroup32 {
     uint2 w;
     uint2 q[K];
 };
 
-template <int K>
+template <bool WIDE>
 __device__ __forceinline__ uint32_t pk_addr8(const uint2& w, uint32_t tabb, int k)
 {
-    return tabb + 8u * __builtin_amdgcn_ubfe(k < 3 ? w.x : w.y, 10 * (k % 3), 10);
+    return tabb + 8u * pk_code<WIDE>(w, k);
 }
 
-template <int K>
-__device__ __forceinline__ void pk_fetch(uint2 w, uint32_t tabb, PkGroup32<K>& gr)
+template <int K, bool WIDE>
+__device__ __forceinline__ void pk_fetch(uint2 w, uint32_t tabb, PkGroup32<K, WIDE>& gr)
 {
     gr.w = w;
 #pragma unroll
-    for (int k = 0; k < K; k++) gr.q[k] = lds_read8(pk_addr8<K>(w, tabb, k));
+    for (int k = 0; k < K; k++) gr.q[k] = lds_read8(pk_addr8<WIDE>(w, tabb, k));
 }
 
 // The same over the compacted rows: one 32-bit word each.
-template <int K>
-__device__ __forceinline__ void pk_status32(const PkGroup32<K>& gr, uint32_t& T, uint32_t& N0, uint32_t& N1)
+template <int K, bool WIDE>
+__device__ __forceinline__ void pk_status32(const PkGroup32<K, WIDE>& gr, uint32_t& T, uint32_t& N0, uint32_t& N1)
 {
     if (K == 3) {
         T = gr.q[0].x | gr.q[1].x | gr.q[2].x;
@@ -1017,8 +1035,8 @@ __device__ __forceinline__ void pk_status32(const PkGroup32<K>& gr, uint32_t& T,
 
 // Per 32-bit half h: T = some literal true, N0 = every literal false, N1 = exactly one
 // literal not false.
-template <int K>
-__device__ __forceinline__ void pk_status(const PkGroup<K>& gr, uint32_t (&T)[2], uint32_t (&N0)[2],
+template <int K, bool WIDE>
+__device__ __forceinline__ void pk_status(const PkGroup<K, WIDE>& gr, uint32_t (&T)[2], uint32_t (&N0)[2],
                                           uint32_t (&N1)[2])
 {
     if (K == 3) {
@@ -1056,7 +1074,7 @@ __device__ __forceinline__ void pk_status(const PkGroup<K>& gr, uint32_t (&T)[2]
 // group's implication writes, so a pass sees every implication made before it in the same
 // wavefront (reading ahead would miss them until the next pass: 9-10% more time at p = 0.05
 // and 0.1 on mixed k-SAT).  process(group) returns true to stop the sweep.
-template <int K, bool PIPE, class Grp = PkGroup<K>, class F>
+template <int K, bool PIPE, class Grp, class F>
 __device__ __forceinline__ void pk_sweep(const uint2* __restrict__ ipk, int m, int G, int g0, int step, int lane,
                                          uint32_t tabb, uint2 zw, F&& process)
 {
@@ -1074,7 +1092,7 @@ __device__ __forceinline__ void pk_sweep(const uint2* __restrict__ ipk, int m, i
     constexpr bool kPipe = PIPE && K <= 3;
     Grp buf[kPipe ? 2 : 1];
     if constexpr (kPipe) {
-        if (cnt > 0) pk_fetch<K>(word(pw[0], 0), tabb, buf[0]);
+        if (cnt > 0) pk_fetch(word(pw[0], 0), tabb, buf[0]);
     }
     bool stop = false;
     for (int t0 = 0; t0 < cnt && !stop; t0 += kPkAhead) {
@@ -1083,11 +1101,11 @@ __device__ __forceinline__ void pk_sweep(const uint2* __restrict__ ipk, int m, i
             const int t = t0 + u;
             if (t < cnt && !stop) {
                 if constexpr (kPipe) {
-                    if (t + 1 < cnt) pk_fetch<K>(word(pw[(u + 1) % kPkAhead], t + 1), tabb, buf[(u + 1) & 1]);
+                    if (t + 1 < cnt) pk_fetch(word(pw[(u + 1) % kPkAhead], t + 1), tabb, buf[(u + 1) & 1]);
                     if (t + kPkAhead < cnt) pw[u] = load(t + kPkAhead);
                     stop = process(buf[u & 1]);
                 } else {
-                    pk_fetch<K>(word(pw[u], t), tabb, buf[0]);
+                    pk_fetch(word(pw[u], t), tabb, buf[0]);
                     if (t + kPkAhead < cnt) pw[u] = load(t + kPkAhead);
                     stop = process(buf[0]);
                 }
@@ -1105,7 +1123,7 @@ __device__ __forceinline__ uint64_t lds_ld64(const uint64_t* p)
     return __hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-template <int K, bool DO_EVAL, bool DO_BCP>
+template <int K, bool WIDE, bool DO_EVAL, bool DO_BCP>
 __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int wv, int NW, int lane, uint32_t* lds,
                                                const uint2* __restrict__ pkk, const uint32_t* __restrict__ rows, int A,
                                                int32_t* __restrict__ counts, uint32_t* __restrict__ out_rows,
@@ -1125,7 +1143,7 @@ __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int
     uint64_t* sh_chg = sh_frozen + 1;                        // [3]
     uint32_t* sh_tot = lds + 128 * W + 16;                   // [64][3]
     const uint32_t zslot = 32u * (uint32_t)W;
-    const uint32_t zc = zslot | (zslot << 10) | (zslot << 20);
+    const uint32_t zc = WIDE ? zslot | (zslot << 16) : zslot | (zslot << 10) | (zslot << 20);
     const uint2 zw = make_uint2(zc, zc);
     const Transposer tp(lane);
     const int half = lane >> 5, i = lane & 31;
@@ -1155,15 +1173,16 @@ __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int
     uint64_t unsat_any = 0;
     if (DO_EVAL) {
         uint32_t acc[2][3] = {{0, 0, 0}, {0, 0, 0}};
-        pk_sweep<K, true>(ipk, m, G, wv, NW, lane, tabb, zw, [&](const PkGroup<K>& gr) {
+        const auto count = [&](const PkGroup<K, WIDE>& gr) {
             uint32_t T[2], N0[2], N1[2];
-            pk_status<K>(gr, T, N0, N1);
+            pk_status(gr, T, N0, N1);
             // SAT|UNIT and UNSAT|UNIT per clause
             const uint64_t b0 = u64(T[0] | N1[0], T[1] | N1[1]);
             const uint64_t b1 = u64((N0[0] | N1[0]) & ~T[0], (N0[1] | N1[1]) & ~T[1]);
             count_group(b0, b1, tp, acc);
             return false;
-        });
+        };
+        pk_sweep<K, true, PkGroup<K, WIDE>>(ipk, m, G, wv, NW, lane, tabb, zw, count);
         uint32_t tot[3];
         finish_counts(acc, lane, tot);
         if (lane < A) {
@@ -1204,9 +1223,9 @@ __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int
             pass++;
             frozen |= lds_ld64(sh_frozen);
             uint64_t chg = 0;       // rows in which this lane's clauses implied a literal
-            if ((frozen & amask) != amask) pk_sweep<K, false>(ipk, m, G, wv, NW, lane, tabb, zw, [&](const PkGroup<K>& gr) {
+            const auto imply = [&](const PkGroup<K, WIDE>& gr) {
                 uint32_t T[2], N0[2], N1[2];
-                pk_status<K>(gr, T, N0, N1);
+                pk_status(gr, T, N0, N1);
                 const uint32_t fl = (uint32_t)frozen, fh = (uint32_t)(frozen >> 32);
                 const uint64_t newconf = u64(andn2(N0[0], T[0], fl), andn2(N0[1], T[1], fh));
                 const uint64_t U = u64(andn2(N1[0], T[0], fl), andn2(N1[1], T[1], fh));
@@ -1216,7 +1235,7 @@ __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int
                     for (int k = 0; k < K; k++) {
                         const uint64_t Uk = U & ~u64(gr.q[k].z, gr.q[k].w);
                         if (Uk) {
-                            const uint32_t a = pk_addr<K>(gr.w, tabb, k);
+                            const uint32_t a = pk_addr<WIDE>(gr.w, tabb, k);
                             lds_or64(a, Uk);
                             lds_or64((a ^ 16u) + 8u, Uk);
                         }
@@ -1228,7 +1247,9 @@ __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int
                     return (frozen & amask) == amask;
                 }
                 return false;
-            });
+            };
+            if ((frozen & amask) != amask)
+                pk_sweep<K, false, PkGroup<K, WIDE>>(ipk, m, G, wv, NW, lane, tabb, zw, imply);
             // rows this wave found in conflict, rows it still moved; the next pass's slot is
             // cleared before the barrier (every wave read it two barriers ago)
             const uint64_t moved = wave_or64(chg) & ~frozen;
@@ -1312,30 +1333,31 @@ __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int
                 pass++;
                 fz |= __hip_atomic_load(sh_fz, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 uint32_t chg = 0;
-                if ((fz & amask32) != amask32)
-                    pk_sweep<K, false, PkGroup32<K>>(ipk, m, G, wv, NW, lane, ctb, zw, [&](const PkGroup32<K>& gr) {
+                const auto imply = [&](const PkGroup32<K, WIDE>& gr) {
                         uint32_t T, N0, N1;
-                        pk_status32<K>(gr, T, N0, N1);
-                        const uint32_t newconf = andn2(N0, T, fz);
-                        const uint32_t U = andn2(N1, T, fz);
-                        if (U) {
+                    pk_status32(gr, T, N0, N1);
+                    const uint32_t newconf = andn2(N0, T, fz);
+                    const uint32_t U = andn2(N1, T, fz);
+                    if (U) {
 #pragma unroll
-                            for (int k = 0; k < K; k++) {
-                                const uint32_t Uk = U & ~gr.q[k].y;
-                                if (Uk) {
-                                    const uint32_t a = pk_addr8<K>(gr.w, ctb, k);
-                                    lds_or32(a, Uk);
-                                    lds_or32((a ^ 8u) + 4u, Uk);
-                                }
+                        for (int k = 0; k < K; k++) {
+                            const uint32_t Uk = U & ~gr.q[k].y;
+                            if (Uk) {
+                                const uint32_t a = pk_addr8<WIDE>(gr.w, ctb, k);
+                                lds_or32(a, Uk);
+                                lds_or32((a ^ 8u) + 4u, Uk);
                             }
                         }
-                        chg |= U;
-                        if (ballot(newconf != 0u)) {
-                            fz |= wave_or32(newconf);
-                            return (fz & amask32) == amask32;
-                        }
-                        return false;
-                    });
+                    }
+                    chg |= U;
+                    if (ballot(newconf != 0u)) {
+                        fz |= wave_or32(newconf);
+                        return (fz & amask32) == amask32;
+                    }
+                    return false;
+                };
+                if ((fz & amask32) != amask32)
+                    pk_sweep<K, false, PkGroup32<K, WIDE>>(ipk, m, G, wv, NW, lane, ctb, zw, imply);
                 const uint32_t moved = wave_or32(chg) & ~fz;
                 if (lane == 0) {
                     if (fz) lds_or32(lds_addr(sh_fz), fz);
@@ -1417,7 +1439,7 @@ __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int
 
 // Workgroup b takes instance order[b]: the batch's instances by decreasing m * K, so the
 // longest sweeps start first and the short ones fill the end of the launch.
-template <bool DO_EVAL, bool DO_BCP>
+template <bool WIDE, bool DO_EVAL, bool DO_BCP>
 __global__ __launch_bounds__(256) void k_eval_bcpk(const InstMeta* __restrict__ meta, const uint2* __restrict__ pkk,
                                                     const uint8_t* __restrict__ klen, const int32_t* __restrict__ order,
                                                     const uint32_t* __restrict__ rows, int A,
@@ -1432,18 +1454,41 @@ __global__ __launch_bounds__(256) void k_eval_bcpk(const InstMeta* __restrict__ 
     const int inst = __builtin_amdgcn_readfirstlane(order[blockIdx.x]);
     const InstMeta mi = meta[inst];
     const int K = __builtin_amdgcn_readfirstlane((int)klen[inst]);
+#define GPSAT_PK_BODY(KB)                                                                                              \
+    eval_bcpk_body<KB, WIDE, DO_EVAL, DO_BCP>(mi, inst, wv, NW, lane, lds_all, pkk, rows, A, counts, out_rows,         \
+                                              conflict, props, passes_out, compact_max)
     if (K <= 3)
-        eval_bcpk_body<3, DO_EVAL, DO_BCP>(mi, inst, wv, NW, lane, lds_all, pkk, rows, A, counts, out_rows, conflict,
-                                           props, passes_out, compact_max);
-    else if (K == 4)
-        eval_bcpk_body<4, DO_EVAL, DO_BCP>(mi, inst, wv, NW, lane, lds_all, pkk, rows, A, counts, out_rows, conflict,
-                                           props, passes_out, compact_max);
-    else if (K == 5)
-        eval_bcpk_body<5, DO_EVAL, DO_BCP>(mi, inst, wv, NW, lane, lds_all, pkk, rows, A, counts, out_rows, conflict,
-                                           props, passes_out, compact_max);
+        GPSAT_PK_BODY(3);
+    else if (WIDE || K == 4)
+        GPSAT_PK_BODY(4);
+    else if constexpr (!WIDE) {
+        if (K == 5)
+            GPSAT_PK_BODY(5);
+        else
+            GPSAT_PK_BODY(6);
+    }
+#undef GPSAT_PK_BODY
+}
+
+template <bool WIDE>
+static void launch_packed(const DeviceBatch& b, const uint32_t* rows, int A, int32_t* counts, uint32_t* out_rows,
+                          int32_t* conflict, int32_t* props, int32_t* passes, bool do_eval, bool do_bcp, hipStream_t st)
+{
+    // one workgroup of eval_pkk_waves wavefronts per instance (the largest instance's table)
+    const int nw = std::max(1, std::min(4, tuning().eval_pkk_waves));
+    dim3 grid(b.n_inst), block(kWave * nw);
+    const size_t lds = (size_t)pk_lds_words(words_per_row(b.max_n)) * 4;
+    const uint2* pk = reinterpret_cast<const uint2*>(b.pkk);
+    const int cmax = std::max(0, std::min(32, tuning().eval_pkk_compact));
+    if (do_eval && do_bcp)
+        hipLaunchKernelGGL((k_eval_bcpk<WIDE, true, true>), grid, block, lds, st, b.meta, pk, b.klen, b.korder, rows, A,
+                           counts, out_rows, conflict, props, passes, cmax);
+    else if (do_eval)
+        hipLaunchKernelGGL((k_eval_bcpk<WIDE, true, false>), grid, block, lds, st, b.meta, pk, b.klen, b.korder, rows, A,
+                           counts, out_rows, conflict, props, passes, cmax);
     else
-        eval_bcpk_body<6, DO_EVAL, DO_BCP>(mi, inst, wv, NW, lane, lds_all, pkk, rows, A, counts, out_rows, conflict,
-                                           props, passes_out, compact_max);
+        hipLaunchKernelGGL((k_eval_bcpk<WIDE, false, true>), grid, block, lds, st, b.meta, pk, b.klen, b.korder, rows, A,
+                           counts, out_rows, conflict, props, passes, cmax);
 }
 
 // LDS words of one wavefront's region in the general kernel (literal masks, row staging,
@@ -1531,21 +1576,10 @@ hipError_t launch_eval_bcp(const DeviceBatch& b, const uint32_t* rows, int A, in
         return hipGetLastError();
     }
     if (ek == EK_PACKED) {
-        // one workgroup of eval_pkk_waves wavefronts per instance (the largest instance's table)
-        const int nw = std::max(1, std::min(4, tuning().eval_pkk_waves));
-        dim3 grid(b.n_inst), block(kWave * nw);
-        const size_t lds = (size_t)pk_lds_words(words_per_row(b.max_n)) * 4;
-        const uint2* pk = reinterpret_cast<const uint2*>(b.pkk);
-        const int cmax = std::max(0, std::min(32, tuning().eval_pkk_compact));
-        if (do_eval && do_bcp)
-            hipLaunchKernelGGL((k_eval_bcpk<true, true>), grid, block, lds, st, b.meta, pk, b.klen, b.korder, rows, A,
-                               counts, out_rows, conflict, props, passes, cmax);
-        else if (do_eval)
-            hipLaunchKernelGGL((k_eval_bcpk<true, false>), grid, block, lds, st, b.meta, pk, b.klen, b.korder, rows, A,
-                               counts, out_rows, conflict, props, passes, cmax);
+        if (b.pkk_wide)
+            launch_packed<true>(b, rows, A, counts, out_rows, conflict, props, passes, do_eval, do_bcp, st);
         else
-            hipLaunchKernelGGL((k_eval_bcpk<false, true>), grid, block, lds, st, b.meta, pk, b.klen, b.korder, rows, A,
-                               counts, out_rows, conflict, props, passes, cmax);
+            launch_packed<false>(b, rows, A, counts, out_rows, conflict, props, passes, do_eval, do_bcp, st);
         return hipGetLastError();
     }
     // stage the arena in LDS when the largest instance keeps the wavefront under 40 KB

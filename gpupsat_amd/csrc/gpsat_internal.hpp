@@ -27,9 +27,10 @@ struct DeviceBatch {
     // 20-29 (codes are below 2n <= 512); instance i's clauses start at meta.coff_base - i
     uint32_t* pk3 = nullptr;
     // device [2 * n_clauses] when every instance fits the packed general path (and the batch
-    // is not fast3): clause c's word pair, six 10-bit slots (see pkk_fits); klen [n_inst]
-    // holds each instance's longest clause
+    // is not fast3): a clause's word pair, six 10-bit or (pkk_wide) four 16-bit slots (see
+    // pkk_fits, pkk_wide_fits); klen [n_inst] holds each instance's longest clause
     uint32_t* pkk = nullptr;
+    bool pkk_wide = false;
     uint8_t* klen = nullptr;
     int32_t* korder = nullptr;    // device [n_inst]: instances by decreasing m * max(3, klen)
     // HBM slices for the eval/BCP mask tables of instances too large for LDS (allocated by
@@ -76,6 +77,11 @@ inline bool fast3_fits(int n, int m) { return words_per_row(n) <= kFast3MaxWords
 constexpr int kPkkMaxWords = 31;
 constexpr int kPkkMaxLen = 6;
 inline bool pkk_fits(int n, int max_len) { return words_per_row(n) <= kPkkMaxWords && max_len <= kPkkMaxLen; }
+// ... with wide slots, for batches that hold a larger instance: clauses of at most 4 literals,
+// and the mask table of 512 bytes per row word within 64 KB of LDS (W <= 126, n <= 2016)
+constexpr int kPkkWideMaxWords = 126;
+constexpr int kPkkWideMaxLen = 4;
+inline bool pkk_wide_fits(int n, int max_len) { return words_per_row(n) <= kPkkWideMaxWords && max_len <= kPkkWideMaxLen; }
 
 size_t eval_bcp_lds_bytes(int max_n);
 // gtab_ext: caller-provided HBM slices for the mask tables of instances too large for LDS

@@ -80,8 +80,8 @@ int gpsat_copy_dev(gpsat_batch *b, void *dst_dev, const void *src_dev, int64_t b
  *   "eval_pkk_compact"  packed general kernel: from the second BCP pass on, long instances with
  *                       at most this many rows still moving continue on 32-bit masks of those
  *                       rows, 0-32 (default 32; 0: never)
- *   "eval_pkk"          1: evaluate batches of clauses with at most 6 literals and n <= 496
- *                       (that the register-resident kernel does not take) with the packed
+ *   "eval_pkk"          1: evaluate batches of clauses with at most 6 literals and n <= 496, or
+ *                       at most 4 literals and n <= 2016 (that the register-resident kernel does not take) with the packed
  *                       general kernel (default); 0: the CSR general kernel
  * The GPSAT_TUNE_EVAL_FAST3 / GPSAT_TUNE_EVAL_STAGE / GPSAT_TUNE_EVAL_WPB /
  * GPSAT_TUNE_EVAL_FAST3_SMALL64 / GPSAT_TUNE_EVAL_PKK / GPSAT_TUNE_EVAL_PKK_WAVES /
