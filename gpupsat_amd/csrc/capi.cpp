@@ -374,6 +374,8 @@ int gpsat_batch_create(const int32_t* lits, const int64_t* clause_off, const int
         wbase += words_per_row(mi.n);
         d.max_n = std::max(d.max_n, mi.n);
         d.max_m = std::max(d.max_m, mi.m);
+        d.max_len = std::max(d.max_len, max_len);
+        d.max_lits = std::max<int64_t>(d.max_lits, clause_off[ce] - clause_off[cb]);
     }
     d.total_words = wbase;
     d.fast3 = fast3 && n_inst > 0;

@@ -15,13 +15,6 @@
 #include "solver.hpp"
 
 namespace gpsat {
-// Per-device cache of device blocks that earlier calls no longer use, by rounded size
-// (at most 1 GiB per device is kept; the rest is freed).  A solve repeated on the same shape
-// then runs without hipMalloc/hipFree, which cost ~1 ms of a 12 ms solve of 20,000 instances.
-void* devmem_cache_take(int dev, size_t bytes);
-bool devmem_cache_give(int dev, void* p, size_t bytes);   // false: not kept (the caller frees)
-size_t devmem_round(size_t bytes);
-
 // Device memory of one call.  Pieces come from the cache or hipMalloc; when the call returns
 // they go back to the cache if the call marked its device work finished (mark_synced), and
 // are freed otherwise (hipFree waits for work still using them).

@@ -67,3 +67,27 @@ def test_forward_and_gradient(sizes, lens, rounds):
         a, r = grad[o:o + k], rgrad[o:o + k]
         o += k
         assert np.linalg.norm(a - r) <= 5e-3 * max(np.linalg.norm(r), 1e-12), name
+
+
+@pytest.mark.parametrize("m,lo,hi", [(0, 1, 1), (1, 1, 1), (63, 1, 1), (64, 1, 1), (65, 1, 1), (128, 2, 2), (85, 3, 3),
+                                     (86, 3, 3), (400, 1, 8), (1300, 3, 3), (40, 40, 64)])
+def test_graph_built_on_device_and_host(m, lo, hi):
+    """The incidence structure built on the GPU against the host's: an instance above its size
+    limits sends the whole batch to the host.  Sums over neighbours are in edge order, so equal
+    structures give equal bits."""
+    print("[gnn graph]", m, lo, hi, flush=True)
+    rng = np.random.default_rng([m, hi])
+    n = max(hi + 3, m // 4)
+    empty = Formula(3, np.zeros(0, np.int32), np.zeros(1, np.int64))
+    f = formula(rng, n, m, lo, hi) if m else empty
+    small = [f, formula(rng, 5, 9, 2, 2), empty, f]
+    big = Formula(2000, np.arange(4, dtype=np.int32), np.array([0, 2, 4], dtype=np.int64))
+    theta = R.init_params(13)
+    got = []
+    for fs in (small, small + [big]):
+        with G.GpuBatch(Batch.from_formulas(fs)) as gb:
+            g = Lr.GnnGraph(gb)
+            V = sum(x.n_vars for x in small)
+            got.append(g.forward(Lr.GnnModel(theta))[:V])
+            g.close()
+    np.testing.assert_array_equal(got[0], got[1])
