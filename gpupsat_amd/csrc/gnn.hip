@@ -23,7 +23,6 @@
 #include <string.h>
 
 #include <algorithm>
-#include <mutex>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -912,45 +911,10 @@ struct gpsat_gnn_model {
     bool dirty = true;
 };
 
-// Streams of destroyed graphs, for the next ones (creating and destroying one costs ~75 us): at
-// most kIdleStreams are kept, each idle, and used by one graph at a time.
-namespace {
-struct IdleStream {
-    int dev;
-    hipStream_t st;
-};
-std::mutex g_streams_mu;
-std::vector<IdleStream>& g_streams = *new std::vector<IdleStream>;   // (never destroyed: graphs may outlive it)
-constexpr size_t kIdleStreams = 16;
-
-hipError_t take_stream(int dev, hipStream_t& st)
-{
-    {
-        std::lock_guard<std::mutex> lk(g_streams_mu);
-        for (size_t i = g_streams.size(); i-- > 0;)
-            if (g_streams[i].dev == dev) {
-                st = g_streams[i].st;
-                g_streams.erase(g_streams.begin() + i);
-                return hipSuccess;
-            }
-    }
-    return hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
-}
-void give_stream(int dev, hipStream_t st)
-{
-    {
-        std::lock_guard<std::mutex> lk(g_streams_mu);
-        if (g_streams.size() < kIdleStreams) {
-            g_streams.push_back(IdleStream{dev, st});
-            return;
-        }
-    }
-    (void)hipStreamDestroy(st);
-}
-}  // namespace
-
 // A graph's arrays are pieces of one block of the device-memory cache (devmem_cache_*), which
-// takes it back once the graph's stream is idle.
+// takes it back once the graph's stream is idle.  The stream is created and destroyed with the
+// graph (~75 us): kept for the next graph it would hold a hardware queue meanwhile, and two
+// batches evaluated at the same time then shared one (31 -> 43 us a pass).
 struct gpsat_gnn_graph {
     int32_t V = 0, L = 0, C = 0, R = 3;
     int64_t E = 0;
@@ -965,10 +929,7 @@ struct gpsat_gnn_graph {
     {
         const bool idle = st && hipStreamSynchronize(st) == hipSuccess;
         if (block && !(idle && devmem_cache_give(dev, block, block_bytes))) (void)hipFree(block);
-        if (idle)
-            give_stream(dev, st);
-        else if (st)
-            (void)hipStreamDestroy(st);
+        if (st) (void)hipStreamDestroy(st);
     }
     // the pieces, laid out in `base` (nullptr: only count); returns the bytes used
     size_t carve(char* base, int32_t n_inst)
@@ -994,7 +955,7 @@ struct gpsat_gnn_graph {
     hipError_t alloc(int32_t n_inst)
     {
         hipError_t e = hipGetDevice(&dev);
-        if (e == hipSuccess) e = take_stream(dev, st);
+        if (e == hipSuccess) e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
         if (e != hipSuccess) return e;
         const size_t bytes = devmem_round(carve(nullptr, n_inst));
         block = devmem_cache_take(dev, bytes);
