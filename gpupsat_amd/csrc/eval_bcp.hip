@@ -337,6 +337,7 @@ __device__ __forceinline__ int64_t uni64(int64_t x)
 constexpr int kFastW = kFast3MaxWords;
 constexpr int kFastG = kFast3MaxGroups;
 
+__device__ __forceinline__ int uni32(int x) { return __builtin_amdgcn_readfirstlane(x); }
 __device__ __forceinline__ uint64_t u64(uint32_t lo, uint32_t hi) { return (uint64_t)lo | ((uint64_t)hi << 32); }
 
 // Symmetric 3-input bit functions as one v_bitop3_b32 each (the truth tables are invariant
@@ -938,8 +939,7 @@ __global__ __launch_bounds__(256) void k_eval_bcp3(const InstMeta* __restrict__ 
 // Why WIDE: the CSR kernel chases offsets and literals from HBM with one wavefront per instance.
 // On 1,000 4-colourings of n = 600 (150 clauses of 4 literals, 2,250 of 2, p = 0.05) it takes
 // 167-184 us, where the rows and clauses of the batch take 10 at the HBM rate; four wavefronts
-// over word pairs take 32 (n = 500, 1,024, 1,600 in smaller batches: 128 -> 22, 161 -> 26, 214
-// -> 32).  The limits are the mask table's: 512 bytes per row word, 64 KB at W = 126.  Sweeping
+// over word pairs take 27 (n = 1,600 x 250, p = 0.02: 207 -> 24).  The limits are the mask table's: 512 bytes per row word, 64 KB at W = 126.  Sweeping
 // the clauses of at most 2 literals apart, with 2 slot reads each, gained nothing at n = 500-600
 // (9% at n = 1,024) and cost the 10-bit form 14% on small colourings (81 instead of 72 VGPRs).
 //
@@ -948,8 +948,8 @@ __global__ __launch_bounds__(256) void k_eval_bcp3(const InstMeta* __restrict__ 
 // bit 4) and take its clause groups in turn (wave v: groups v, v + NW, ...), so a long
 // instance is swept NW times faster than by one wave.  Implications go straight into the
 // shared table; each BCP pass ends at one barrier, where the waves' "implied something"
-// rows and conflict rows are combined in LDS.  The table is built straight from the input
-// rows in HBM and the closure rows go straight back.  On long instances, once at most 32 rows
+// rows and conflict rows are combined in LDS.  The rows pass through the table's own LDS on
+// their way in and out, so that their copies are coalesced.  On long instances, once at most 32 rows
 // still move, the rows at their fixpoint are written out and the passes go on over a table of
 // 8-byte slots {T, F} holding 32-bit masks of the moving rows, built in place of the first.
 //
@@ -1123,6 +1123,30 @@ __device__ __forceinline__ uint64_t lds_ld64(const uint64_t* p)
     return __hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// (row, word) of the words tid, tid + nthreads, ... of rows of W words.  The quotients (of
+// tid < nthreads <= 256 by W <= 126) by reciprocal: (x + 1/2) / W is at least 1/252 away from
+// any integer, far above its rounding error (integer divisions cost short rows 2%).
+struct RowWalk {
+    int row, j, drow, dj, W;
+    __device__ RowWalk(int tid, int nthreads, int W_) : W(W_)
+    {
+        const float inv = __builtin_amdgcn_rcpf((float)W);
+        row = (int)(((float)tid + 0.5f) * inv);
+        j = tid - row * W;
+        drow = uni32((int)(((float)nthreads + 0.5f) * inv));
+        dj = nthreads - drow * W;
+    }
+    __device__ __forceinline__ void next()
+    {
+        j += dj;
+        row += drow;
+        if (j >= W) {
+            j -= W;
+            row++;
+        }
+    }
+};
+
 template <int K, bool WIDE, bool DO_EVAL, bool DO_BCP>
 __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int wv, int NW, int lane, uint32_t* lds,
                                                const uint2* __restrict__ pkk, const uint32_t* __restrict__ rows, int A,
@@ -1149,15 +1173,49 @@ __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int
     const int half = lane >> 5, i = lane & 31;
     const int tid = wv * kWave + lane, nthreads = NW * kWave;
 
-    // the mask table: lane a reads word j of row a, the transpose hands lane (half, i) the
-    // masks of literal 32j + i over rows 32*half .. 32*half + 31 (wave v: words v, v + NW, ...)
-    for (int j0 = wv; j0 < W; j0 += 8 * NW) {
+    // The rows come in as one coalesced copy (read word by word, lane a on row a, an instruction
+    // touches 64 lines: ~7,000 cycles of the address unit per instance of W = 38, in and out:
+    // 31.7 -> 26.7 us on 1,000 4-colourings of n = 600, mixed k-SAT 55.8 -> 53.7 at p = 0.1), put
+    // down word by word: word j of row a at stage[65j + a], conflict-free both ways.  The stage
+    // ends where the table ends; a batch of 8 NW words is read from it before any of the batch's
+    // slots are written, and those end below the stage's later words (128 * 8NW(b + 1) <= 63W +
+    // 65 * 8NW(b + 1) while W > 8NW(b + 1)).
+    RowWalk walk(tid, nthreads, W);
+    {
+        uint32_t* stage = tab + 63 * W;
+        const int nw = A * W;
+        for (int ub = 0; ub < nw; ub += 8 * nthreads) {
+            uint32_t r[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                r[u] = 0u;
+                if (ub + u * nthreads < nw) r[u] = src[min(ub + u * nthreads + tid, nw - 1)];
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                if (ub + u * nthreads < nw) {
+                    if (ub + tid + u * nthreads < nw) stage[65 * walk.j + walk.row] = r[u];
+                    walk.next();
+                }
+            }
+        }
+        __syncthreads();
+    }
+    // the mask table: the transpose of word j, lane a on row a, hands lane (half, i) the masks of
+    // literal 32j + i over rows 32*half .. 32*half + 31 (wave v: words v, v + NW, ...)
+    int in_pop = 0;      // lane a: literals of row a in this wave's words
+    for (int jb = 0; jb < W; jb += 8 * NW) {
         uint32_t r[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) r[u] = (j0 + u * NW < W && lane < A) ? src[lane * W + j0 + u * NW] : 0u;
+        for (int u = 0; u < 8; u++) {
+            const int j = jb + wv + u * NW;
+            r[u] = (j < W && lane < A) ? tab[63 * W + 65 * j + lane] : 0u;
+            in_pop += __builtin_popcount(r[u]);
+        }
+        __syncthreads();
 #pragma unroll
         for (int u = 0; u < 8; u++) {
-            const int j = j0 + u * NW;
+            const int j = jb + wv + u * NW;
             if (j < W) {
                 const uint32_t x = tp(r[u]);
                 const int l = 32 * j + i;
@@ -1213,6 +1271,11 @@ __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int
             if (lane == 0 && cm) lds_or64p(sh_frozen, cm);
         }
         __syncthreads();
+        // the evaluation's totals are no longer needed: their place keeps this wave's input counts
+        // (16 bits: a row has at most 2 n <= 4,032 literals), so no register does over the passes
+        uint16_t* sh_in = reinterpret_cast<uint16_t*>(sh_tot);   // [NW][64]
+        uint32_t* sh_cnt = sh_tot + 128;                         // [64]: implied literals of row a
+        sh_in[wv * kWave + lane] = (uint16_t)in_pop;
         // Every wave leaves the pass loop on the same value: the pass's "moved" slot, which no
         // wave writes between the barrier that ends the pass and the next pass's barrier.  The
         // conflict rows only grow, and any snapshot of them is a valid one.
@@ -1280,6 +1343,7 @@ __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int
             }
             cm = wave_or64(cm) | frozen;
             if (lane == 0 && cm) lds_or64p(sh_frozen, cm);
+            if (wv == 0) sh_cnt[lane] = 0u;
         }
         __syncthreads();
         // no wave writes the conflict rows from here on: every wave reads the same ones
@@ -1405,42 +1469,58 @@ __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int
             if (passes_out && lane == 0) passes_out[inst] = pass;
             return;
         }
-        if (wv != 0) return;
+        // The closure rows go out as the input rows came in: the waves transpose their words back
+        // and put word j of row a at tab[65j + a] (a batch's slots are read before they are
+        // written over, and later batches' lie above), then all copy the rows out coalesced.  A
+        // conflicting row's output is its input.
         const bool my_conflict = (frozen >> lane) & 1ull;
         const bool all_conflict = (frozen & amask) == amask;
-        uint32_t* orow = out_rows + row0;
-        int cnt = 0, in_pop = 0;
-        for (int j0 = 0; j0 < W; j0 += 8) {
-            uint32_t x[8];
+        if (!all_conflict) {
+            int cnt = -(int)sh_in[wv * kWave + lane];
+            for (int jb = 0; jb < W; jb += 8 * NW) {
+                uint32_t x[8];
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
-                x[u] = 0u;
-                if (j0 + u < W && !all_conflict) x[u] = tp(tab[4 * (32 * (j0 + u) + i) + half]);   // lane a: row a
-            }
+                for (int u = 0; u < 8; u++) {
+                    const int j = jb + wv + u * NW;
+                    x[u] = j < W ? tab[4 * (32 * j + i) + half] : 0u;
+                }
+                __syncthreads();
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
-                if (j0 + u < W && lane < A) {
-                    const uint32_t in = src[lane * W + j0 + u];
-                    const uint32_t o = my_conflict ? in : x[u];
-                    in_pop += __builtin_popcount(in);
-                    cnt += __builtin_popcount(o);
-                    orow[lane * W + j0 + u] = o;
+                for (int u = 0; u < 8; u++) {
+                    const int j = jb + wv + u * NW;
+                    if (j < W) {
+                        const uint32_t o = tp(x[u]);     // lane a: row a
+                        cnt += __builtin_popcount(o);
+                        tab[65 * j + lane] = o;
+                    }
                 }
             }
+            // the closure contains the input, so the implied literals are the difference of the counts
+            if (lane < A && !my_conflict) atomicAdd(&sh_cnt[lane], (uint32_t)cnt);
+            __syncthreads();
         }
-        // the closure contains the input, so the implied literals are the difference of the counts
-        if (lane < A) {
+        uint32_t* orow = out_rows + row0;
+        RowWalk out(tid, nthreads, W);
+        for (int k = tid; k < A * W; k += nthreads) {
+            const uint32_t o = (frozen >> out.row) & 1ull ? src[k] : tab[65 * out.j + out.row];
+            __builtin_nontemporal_store(o, orow + k);
+            out.next();
+        }
+        if (wv == 0 && lane < A) {
             conflict[(int64_t)inst * A + lane] = my_conflict ? 1 : 0;
-            props[(int64_t)inst * A + lane] = cnt - in_pop;
+            props[(int64_t)inst * A + lane] = (int32_t)sh_cnt[lane];
         }
+        if (wv != 0) return;
         if (passes_out && lane == 0) passes_out[inst] = pass;
     }
 }
 
+// (7 wavefronts per SIMD: at the 75 VGPRs the compiler would take, 6, mixed k-SAT at p = 0.1 takes
+// 56.5 us instead of 53.7.)
 // Workgroup b takes instance order[b]: the batch's instances by decreasing m * K, so the
 // longest sweeps start first and the short ones fill the end of the launch.
 template <bool WIDE, bool DO_EVAL, bool DO_BCP>
-__global__ __launch_bounds__(256) void k_eval_bcpk(const InstMeta* __restrict__ meta, const uint2* __restrict__ pkk,
+__global__ __launch_bounds__(256, 7) void k_eval_bcpk(const InstMeta* __restrict__ meta, const uint2* __restrict__ pkk,
                                                     const uint8_t* __restrict__ klen, const int32_t* __restrict__ order,
                                                     const uint32_t* __restrict__ rows, int A,
                                                     int32_t* __restrict__ counts, uint32_t* __restrict__ out_rows,

@@ -62,3 +62,25 @@ def test_colorings(orc, n_nodes):
                 with G.tuned(**over):
                     for g, w in zip(gb.bcp_fixpoint(rows, 64), orc.bcp_batch(b, rows, 64)):
                         np.testing.assert_array_equal(g, w)
+
+
+@pytest.mark.parametrize("n", [1, 16, 17, 127, 128, 129, 496, 511, 512, 513, 1024, 2016])
+def test_row_lengths(orc, n):
+    """Rows copied in and out a word at a time over all wavefronts: rows of 1 word, of the words
+    one batch of transposes takes (8, 16, 24 or 32, by the wavefronts) and one more, of the most
+    a table holds; beside an instance without variables."""
+    print("[packed forms] rows", n, flush=True)
+    rng = np.random.default_rng(n)
+    k = min(n, 4)
+    none = Formula(0, np.zeros(0, np.int32), np.zeros(1, np.int64))
+    b = Batch.from_formulas([formula(rng, n, [k] * 30 + [min(n, 2)] * (2 * n)), none, formula(rng, n, [1] * 3)])
+    for A, p in ((1, 0.2), (33, 0.02), (64, 0.1)):
+        rows = W.random_assignments(b, A, p, seed=n)
+        want = orc.eval_batch(b, rows, A), *orc.bcp_batch(b, rows, A)
+        with G.GpuBatch(b) as gb:
+            assert gb.eval_kernel() == "packed"
+            for nw in (1, 2, 3, 4):
+                with G.tuned(eval_pkk_waves=nw):
+                    got = gb.clause_eval(rows, A), *gb.bcp_fixpoint(rows, A)
+                for g, w in zip(got, want):
+                    np.testing.assert_array_equal(g, w)
