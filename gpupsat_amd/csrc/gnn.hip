@@ -355,13 +355,18 @@ __global__ __launch_bounds__(256, 4) void k_layer(const int32_t* __restrict__ of
 // neighbours' message gradients G (either may be absent: SELF, GATHER), dP = dH' * [H' > 0]
 // (kept in BF16 for the weight gradient; its FP32 sum is the bias gradient) and dX = dP W: the
 // columns of this row's own H go to S in place (LIT: plus those the other polarity's row has for
-// it, exchanged between neighbouring lanes), the message columns to M.  The clauses' S of the
-// first round (LAST) is the gradient of their embedding and is summed here instead of stored.
-// part: the workgroup's bias sums, 64 floats; part_e: those for u_c and v_c, 128.
+// it, exchanged between neighbouring lanes), the message columns to M.
+// In the first round (LAST) what remains is the gradient of the embeddings, and dX is summed
+// here instead of stored: H_l^0 = occ(l)/8 u_l + v_l, so the own columns of a literal enter the
+// gradients of (u_l, v_l) with weights (occ(l)/8, 1), those of a clause (u_c, v_c) with
+// (len/4, 1), and a clause's message columns, a quarter of which goes to each of its literals,
+// (u_l, v_l) with (sum of occ(l)/8, len) / 4 -- a kernel that gathered them to the literals
+// again took 88 us, and the rows' stores 50, of 1.94 ms.
+// part: the workgroup's bias sums, 64 floats; part_e: those for u_l, v_l, u_c, v_c, 256.
 template <bool LIT, bool SELF, bool GATHER, bool LAST>
 __global__ __launch_bounds__(256, 4) void k_layer_bwd(const int32_t* __restrict__ off, const int32_t* __restrict__ edges,
-                                                      int N, const bf16_t* __restrict__ Wt,
-                                                      const uint2* __restrict__ mask, const float* __restrict__ G,
+                                                      const int32_t* __restrict__ n_off, int N,
+                                                      const bf16_t* __restrict__ Wt, const uint2* __restrict__ mask, const float* __restrict__ G,
                                                       float* S, bf16_t* __restrict__ dP, float* __restrict__ M,
                                                       float* __restrict__ part, float* __restrict__ part_e)
 {
@@ -370,6 +375,7 @@ __global__ __launch_bounds__(256, 4) void k_layer_bwd(const int32_t* __restrict_
     __shared__ float red[256];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane & 3;
     const int block = xcd_block(), r = 16 * (block * 4 + wave) + (lane >> 2), row = min(r, N - 1);
+    float* pe = part_e + (size_t)block * O_WC;
     Edges E;
     if constexpr (GATHER || LAST) E.offsets(off, row, q);
     stage_weights<K, 64>(sW, Wt);
@@ -403,7 +409,23 @@ __global__ __launch_bounds__(256, 4) void k_layer_bwd(const int32_t* __restrict_
     f[1] = to_product(f[1], lane);
     product<2>(g, sW, 1, f, lane);
     from_product(g, lane);
-    if (r < N) st_row(M + (size_t)r * HID, g, q);
+    if constexpr (LAST && !LIT) {
+        // (a row past N has dP = 0, so dX = 0)
+        int occ = 0;
+        for (int e = E.e0 + q; e < E.e1; e += 4) {
+            const int l = edges[e];
+            occ += n_off[l + 1] - n_off[l];
+        }
+        occ += __builtin_amdgcn_mov_dpp(occ, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
+        occ += __builtin_amdgcn_mov_dpp(occ, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
+#pragma unroll
+        for (int i = 0; i < 16; i++) s[i] = (float)occ * 0.03125f * g[i];
+        block_sum<true>(s, red, pe, lane, wave);
+#pragma unroll
+        for (int i = 0; i < 16; i++) g[i] *= (float)deg * 0.25f;
+        block_sum<true>(g, red, pe + O_VL, lane, wave);
+    }
+    if (r < N && (LIT || !LAST)) st_row(M + (size_t)r * HID, g, q);
     product<2>(g, sW, 0, f, lane);
     if constexpr (LIT) {
         product<2>(s, sW, 2, f, lane);
@@ -412,11 +434,11 @@ __global__ __launch_bounds__(256, 4) void k_layer_bwd(const int32_t* __restrict_
     }
     from_product(g, lane);
     if constexpr (LAST) {
-        // (a row past N has dP = 0, so dX = 0)
-        block_sum<true>(g, red, part_e + (size_t)block * 128 + 64, lane, wave);
+        block_sum<true>(g, red, pe + (LIT ? O_VL : O_VC), lane, wave);
 #pragma unroll
-        for (int i = 0; i < 16; i++) g[i] *= (float)deg * 0.25f;
-        block_sum<true>(g, red, part_e + (size_t)block * 128, lane, wave);
+        for (int i = 0; i < 16; i++) g[i] *= (float)deg * (LIT ? 0.125f : 0.25f);
+        block_sum<true>(g, red, pe + (LIT ? O_UL : O_UC), lane, wave);
+        if (LIT && threadIdx.x < 128) pe[O_UC + threadIdx.x] = 0.f;
     } else if (r < N)
         st_row(S + (size_t)r * HID, g, q);
 }
@@ -643,10 +665,6 @@ __global__ __launch_bounds__(256) void k_dense_dw(const bf16_t* __restrict__ dP,
     }
 }
 
-// This workgroup's partial gradients of the literals' embeddings u_l, v_l (parameters 0..127)
-// from dH^0 = S + 1/4 (sum of M over the clauses); 16 lanes per row, each on 4 consecutive
-// dimensions.
-__device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 __device__ __forceinline__ void fma4(float4& s, float a, const float4& x)
 {
     s.x += a * x.x;
@@ -654,44 +672,6 @@ __device__ __forceinline__ void fma4(float4& s, float a, const float4& x)
     s.z += a * x.z;
     s.w += a * x.w;
 }
-__global__ __launch_bounds__(256) void k_bwd_embed(const int32_t* __restrict__ off, const int32_t* __restrict__ edges,
-                                                   int L, const float* __restrict__ S, const float* __restrict__ M,
-                                                   float* __restrict__ part)
-{
-    __shared__ float4 red[16][32];
-    const int k16 = threadIdx.x & 15, d = 4 * k16, slot = threadIdx.x >> 4;
-    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-    float4 gu = zero, gv = zero;
-    const int block = xcd_block(), per = (L + gridDim.x - 1) / gridDim.x;
-    for (int l = block * per + slot, end = min(L, (block + 1) * per); l < end; l += 16) {
-        const int e0 = off[l], e1 = off[l + 1];
-        float4 m = zero;
-        for (int e = e0; e < e1; e += 4) {
-            const int k = e1 - e;
-            const int i0 = edges[e], i1 = edges[k > 1 ? e + 1 : e], i2 = edges[k > 2 ? e + 2 : e],
-                      i3 = edges[k > 3 ? e + 3 : e];
-            const float4 x0 = ld4(M + (size_t)i0 * HID + d), x1 = ld4(M + (size_t)i1 * HID + d);
-            const float4 x2 = ld4(M + (size_t)i2 * HID + d), x3 = ld4(M + (size_t)i3 * HID + d);
-            fma4(m, 1.f, x0);
-            if (k > 1) fma4(m, 1.f, x1);
-            if (k > 2) fma4(m, 1.f, x2);
-            if (k > 3) fma4(m, 1.f, x3);
-        }
-        float4 g = ld4(S + (size_t)l * HID + d);
-        fma4(g, 0.25f, m);
-        fma4(gu, (float)(e1 - e0) * 0.125f, g);
-        fma4(gv, 1.f, g);
-    }
-    red[slot][k16] = gu;
-    red[slot][16 + k16] = gv;
-    __syncthreads();
-    if (threadIdx.x < 32) {
-        float4 s = zero;
-        for (int i = 0; i < 16; i++) fma4(s, 1.f, red[i][threadIdx.x]);
-        *reinterpret_cast<float4*>(part + (size_t)block * O_UC + 4 * threadIdx.x) = s;
-    }
-}
-
 // Fixed-order reductions of the workgroups' partials, all of a pass's in two launches: every
 // gradient and the loss are summed this way, never with floating-point atomics, so a gradient
 // is the same bit for bit on every run.  Job: `slots` rows of `quads` float4; stage 1 splits
@@ -878,7 +858,6 @@ using namespace gpsat::gnn;
 // Workgroups of the weight-gradient products (one partial matrix each; two workgroups per CU, as
 // more of them write more partials and gain nothing) and of the embedding gradient.
 constexpr int DW_BLOCKS = 512;
-constexpr int EMBED_BLOCKS = 2048;
 constexpr int MAX_GROUPS = 32;
 
 // One pass's activations, carved from the model's arena (see gpsat_gnn_model); the second part
@@ -889,7 +868,7 @@ struct Acts {
     bf16_t *dPc = nullptr, *dPl = nullptr, *dPo = nullptr;                    // [rounds][rows][64]
     uint2 *mask_c = nullptr, *mask_l = nullptr;                               // [rounds][rows]
     float *Sl = nullptr, *Ml = nullptr, *Sc = nullptr, *Mc = nullptr, *loss = nullptr;
-    float *part_o = nullptr, *part_l = nullptr, *part_c = nullptr, *part_el = nullptr, *part_ec = nullptr;
+    float *part_o = nullptr, *part_l = nullptr, *part_c = nullptr, *part_e = nullptr;
     float *part_wl = nullptr, *part_wc = nullptr, *part_wo = nullptr, *part2 = nullptr;
 };
 
@@ -1020,8 +999,7 @@ size_t carve(const gpsat_gnn_graph* g, bool train, char* base, Acts& a)
     take(a.part_o, (size_t)row_blocks(V, readout_tiles((int)V)) * HEAD_PART);
     take(a.part_l, R * row_blocks(L) * HID);
     take(a.part_c, R * row_blocks(C) * HID);
-    take(a.part_el, (size_t)EMBED_BLOCKS * 2 * HID);
-    take(a.part_ec, (size_t)row_blocks(C) * 2 * HID);
+    take(a.part_e, ((size_t)row_blocks(L) + row_blocks(C)) * O_WC);   // literals' workgroups, then clauses'
     take(a.part_wl, (size_t)dw_blocks(R * L) * 64 * 192);
     take(a.part_wc, (size_t)dw_blocks(R * C) * 64 * 128);
     take(a.part_wo, (size_t)dw_blocks(V) * 64 * 128);
@@ -1087,10 +1065,12 @@ void layer_bwd(gpsat_gnn_model* m, gpsat_gnn_graph* g, const Acts& a, int t)
     const int N = LIT ? g->L : g->C;
     if (N == 0) return;
     hipLaunchKernelGGL((k_layer_bwd<LIT, SELF, GATHER, LAST>), dim3(row_blocks(N)), dim3(256), 0, g->st,
-                       LIT ? g->l_off : g->c_off, LIT ? g->l_edges : g->c_edges, N, LIT ? m->Wlt : m->Wct,
+                       LIT ? g->l_off : g->c_off, LIT ? g->l_edges : g->c_edges, LIT ? g->c_off : g->l_off, N,
+                       LIT ? m->Wlt : m->Wct,
                        (LIT ? a.mask_l : a.mask_c) + (size_t)t * N, LIT ? a.Mc : a.Ml, LIT ? a.Sl : a.Sc,
                        (LIT ? a.dPl : a.dPc) + (size_t)t * N * HID, LIT ? a.Ml : a.Mc,
-                       (LIT ? a.part_l : a.part_c) + (size_t)t * row_blocks(N) * HID, a.part_ec);
+                       (LIT ? a.part_l : a.part_c) + (size_t)t * row_blocks(N) * HID,
+                       a.part_e + (LIT ? 0 : (size_t)row_blocks(g->L) * O_WC));
 }
 
 // Backward pass from the readout's gradients to m->grad (every element written) and the loss.
@@ -1101,10 +1081,14 @@ hipError_t backward_pass(gpsat_gnn_model* m, gpsat_gnn_graph* g, const Acts& a)
     const int sl = L ? row_blocks(L) : 0, sc = C ? row_blocks(C) : 0;
     for (int t = R - 1; t >= 0; t--) {
         const bool top = t == R - 1;
-        if (top)
+        if (top && t)
             layer_bwd<true, true, false, false>(m, g, a, t);
-        else
+        else if (top)
+            layer_bwd<true, true, false, true>(m, g, a, t);
+        else if (t)
             layer_bwd<true, true, true, false>(m, g, a, t);
+        else
+            layer_bwd<true, true, true, true>(m, g, a, t);
         if (top && t)
             layer_bwd<false, false, true, false>(m, g, a, t);
         else if (top)
@@ -1118,7 +1102,6 @@ hipError_t backward_pass(gpsat_gnn_model* m, gpsat_gnn_graph* g, const Acts& a)
     hipLaunchKernelGGL((k_dense_dw<192>), dim3(bl), dim3(256), 0, st, a.dPl, a.Xl, a.part_wl, (int64_t)R * L);
     hipLaunchKernelGGL((k_dense_dw<128>), dim3(bc), dim3(256), 0, st, a.dPc, a.Xc, a.part_wc, (int64_t)R * C);
     hipLaunchKernelGGL((k_dense_dw<128>), dim3(bo), dim3(256), 0, st, a.dPo, a.Z, a.part_wo, (int64_t)V);
-    hipLaunchKernelGGL(k_bwd_embed, dim3(EMBED_BLOCKS), dim3(256), 0, st, g->l_off, g->l_edges, L, a.Sl, a.Mc, a.part_el);
     RedJobs jobs{};
     int nb1 = 0, nb2 = 0;
     float* part2 = a.part2;
@@ -1132,8 +1115,7 @@ hipError_t backward_pass(gpsat_gnn_model* m, gpsat_gnn_graph* g, const Acts& a)
     job(a.part_o, V ? row_blocks(V, readout_tiles(V)) : 0, HEAD_PART, m->grad + O_BO, HEAD_GRADS, a.loss);
     job(a.part_l, R * sl, HID, m->grad + O_BL, HID);
     job(a.part_c, R * sc, HID, m->grad + O_BC, HID);
-    job(a.part_el, EMBED_BLOCKS, 2 * HID, m->grad + O_UL, 2 * HID);
-    job(a.part_ec, sc, 2 * HID, m->grad + O_UC, 2 * HID);
+    job(a.part_e, sl + sc, O_WC, m->grad, O_WC);
     job(a.part_wl, bl, 64 * 192, m->grad + O_WL, 64 * 192);
     job(a.part_wc, bc, 64 * 128, m->grad + O_WC, 64 * 128);
     job(a.part_wo, bo, 64 * 128, m->grad + O_WO, 64 * 128);
