@@ -16,7 +16,7 @@
 // Each half round is one kernel per direction (gather, product and elementwise work on rows
 // held in registers), as memory traffic and its latency bound the network, not arithmetic: the 172
 // GFLOP of a training pass over 512 x (n=300, m=1278) would take 0.15 ms at half of the MFMA
-// peak, moving its rows of ~4.6 GB about 1 ms.  The pass takes 1.94 ms, where separate gather, product,
+// peak, moving its rows of ~4.6 GB about 1 ms.  The pass takes 1.78 ms, where separate gather, product,
 // mask and reduction kernels moved ~9 GB in 3.70 ms; a layer's kernel runs at 3-4.3 TB/s of
 // compulsory bytes.
 #include <hip/hip_runtime.h>
@@ -255,6 +255,11 @@ __device__ __forceinline__ void block_sum(const float (&x)[16], float* red, floa
     }
 }
 
+// Wavefronts of a layer's workgroup, which share the staged weights: 8 (instead of 4: the
+// clauses' layer 132 -> 126 us, its backward 157 -> 142), but 4 where the first round's backward
+// sums rows over the workgroup at several barriers (121 us; 8: 141).
+constexpr int LAYER_WAVES = 8, LAST_WAVES = 4;
+
 // One half round, whole: H' = relu([H | scale * sum of neighbours | (LIT) H of l ^ 1] W^T + b),
 // 16 rows per wavefront, in place (a row is read and written by its own wavefront only, and the
 // two rows of a variable share one).
@@ -264,7 +269,7 @@ __device__ __forceinline__ void block_sum(const float (&x)[16], float* red, floa
 //          occurrences it would be rounded differently)
 //   TRAIN  X = bf16([H | messages]) and the sign mask of H' are kept for the backward pass
 template <bool LIT, bool FIRST, bool TRAIN>
-__global__ __launch_bounds__(256, 4) void k_layer(const int32_t* __restrict__ off, const int32_t* __restrict__ edges,
+__global__ __launch_bounds__(64 * LAYER_WAVES, 4) void k_layer(const int32_t* __restrict__ off, const int32_t* __restrict__ edges,
                                                   const int32_t* __restrict__ n_off, int N, const float* __restrict__ th,
                                                   const bf16_t* __restrict__ W, const float* __restrict__ bias,
                                                   const float* __restrict__ Hn, float* H, bf16_t* __restrict__ X,
@@ -273,7 +278,7 @@ __global__ __launch_bounds__(256, 4) void k_layer(const int32_t* __restrict__ of
     constexpr int K = LIT ? 192 : 128, KS = K / 32;
     __shared__ __align__(16) bf16_t sW[64 * (K + 8)];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane & 3;
-    const int r = 16 * (xcd_block() * 4 + wave) + (lane >> 2), row = min(r, N - 1);
+    const int r = 16 * (xcd_block() * LAYER_WAVES + wave) + (lane >> 2), row = min(r, N - 1);
     Edges E;
     E.offsets(off, row, q);
     stage_weights<64, K>(sW, W);
@@ -364,17 +369,17 @@ __global__ __launch_bounds__(256, 4) void k_layer(const int32_t* __restrict__ of
 // again took 88 us, and the rows' stores 50, of 1.94 ms.
 // part: the workgroup's bias sums, 64 floats; part_e: those for u_l, v_l, u_c, v_c, 256.
 template <bool LIT, bool SELF, bool GATHER, bool LAST>
-__global__ __launch_bounds__(256, 4) void k_layer_bwd(const int32_t* __restrict__ off, const int32_t* __restrict__ edges,
+__global__ __launch_bounds__(64 * (LAST ? LAST_WAVES : LAYER_WAVES), 4) void k_layer_bwd(const int32_t* __restrict__ off, const int32_t* __restrict__ edges,
                                                       const int32_t* __restrict__ n_off, int N,
                                                       const bf16_t* __restrict__ Wt, const uint2* __restrict__ mask, const float* __restrict__ G,
                                                       float* S, bf16_t* __restrict__ dP, float* __restrict__ M,
                                                       float* __restrict__ part, float* __restrict__ part_e)
 {
-    constexpr int K = LIT ? 192 : 128;
+    constexpr int K = LIT ? 192 : 128, NW = LAST ? LAST_WAVES : LAYER_WAVES;
     __shared__ __align__(16) bf16_t sW[K * (64 + 8)];
-    __shared__ float red[256];
+    __shared__ float red[64 * NW];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane & 3;
-    const int block = xcd_block(), r = 16 * (block * 4 + wave) + (lane >> 2), row = min(r, N - 1);
+    const int block = xcd_block(), r = 16 * (block * NW + wave) + (lane >> 2), row = min(r, N - 1);
     float* pe = part_e + (size_t)block * O_WC;
     Edges E;
     if constexpr (GATHER || LAST) E.offsets(off, row, q);
@@ -960,9 +965,10 @@ struct gpsat_gnn_graph {
 
 namespace {
 
-// Workgroups that cover N rows, 16 per wavefront and `tiles` of those one after another: a
-// multiple of 8, see xcd_block.
-int row_blocks(int64_t N, int tiles = 1) { return (int)(((N + 64 * tiles - 1) / (64 * tiles) + 7) / 8 * 8); }
+// Workgroups that cover N rows, 16 * tiles each: a multiple of 8, see xcd_block.
+int row_blocks(int64_t N, int tiles) { return (int)(((N + 16 * tiles - 1) / (16 * tiles) + 7) / 8 * 8); }
+// Bias partials of a layer over N rows: the first round's workgroups, then the other rounds'.
+size_t bias_slot(int64_t N, int t) { return t ? row_blocks(N, LAST_WAVES) + (size_t)(t - 1) * row_blocks(N, LAYER_WAVES) : 0; }
 // The readout's wavefronts take several tiles in turn where there are enough to fill the GPU:
 // both forms of W_o are staged per workgroup.
 int readout_tiles(int V) { return std::max(1, std::min(4, V / (16 * 2048))); }
@@ -996,10 +1002,10 @@ size_t carve(const gpsat_gnn_graph* g, bool train, char* base, Acts& a)
     take(a.Sc, C * HID);
     take(a.Mc, C * HID);
     take(a.loss, HEAD_PART - HEAD_GRADS);   // (the rest of a readout partial's row)
-    take(a.part_o, (size_t)row_blocks(V, readout_tiles((int)V)) * HEAD_PART);
-    take(a.part_l, R * row_blocks(L) * HID);
-    take(a.part_c, R * row_blocks(C) * HID);
-    take(a.part_e, ((size_t)row_blocks(L) + row_blocks(C)) * O_WC);   // literals' workgroups, then clauses'
+    take(a.part_o, (size_t)row_blocks(V, 4 * readout_tiles((int)V)) * HEAD_PART);
+    take(a.part_l, bias_slot(L, (int)R) * HID);
+    take(a.part_c, bias_slot(C, (int)R) * HID);
+    take(a.part_e, ((size_t)row_blocks(L, LAST_WAVES) + row_blocks(C, LAST_WAVES)) * O_WC);   // literals' workgroups, then clauses'
     take(a.part_wl, (size_t)dw_blocks(R * L) * 64 * 192);
     take(a.part_wc, (size_t)dw_blocks(R * C) * 64 * 128);
     take(a.part_wo, (size_t)dw_blocks(V) * 64 * 128);
@@ -1030,8 +1036,8 @@ void layer(gpsat_gnn_model* m, gpsat_gnn_graph* g, const Acts& a, int t)
 {
     const int N = LIT ? g->L : g->C;
     if (N == 0) return;
-    hipLaunchKernelGGL((k_layer<LIT, FIRST, TRAIN>), dim3(row_blocks(N)), dim3(256), 0, g->st, LIT ? g->l_off : g->c_off,
-                       LIT ? g->l_edges : g->c_edges, LIT ? g->c_off : g->l_off, N, m->th,
+    hipLaunchKernelGGL((k_layer<LIT, FIRST, TRAIN>), dim3(row_blocks(N, LAYER_WAVES)), dim3(64 * LAYER_WAVES), 0, g->st,
+                       LIT ? g->l_off : g->c_off, LIT ? g->l_edges : g->c_edges, LIT ? g->c_off : g->l_off, N, m->th,
                        LIT ? m->Wl : m->Wc, m->th + (LIT ? O_BL : O_BC), LIT ? a.Hc : a.Hl, LIT ? a.Hl : a.Hc,
                        TRAIN ? (LIT ? a.Xl : a.Xc) + (size_t)t * N * 128 : nullptr,
                        TRAIN ? (LIT ? a.mask_l : a.mask_c) + (size_t)t * N : nullptr);
@@ -1054,7 +1060,7 @@ hipError_t forward_pass(gpsat_gnn_model* m, gpsat_gnn_graph* g, const Acts& a, f
     }
     const int tiles = readout_tiles(g->V);
     if (g->V)
-        hipLaunchKernelGGL((k_readout<TRAIN>), dim3(row_blocks(g->V, tiles)), dim3(256), 0, g->st, g->V, tiles, a.Hl, m->Wo, m->Wot,
+        hipLaunchKernelGGL((k_readout<TRAIN>), dim3(row_blocks(g->V, 4 * tiles)), dim3(256), 0, g->st, g->V, tiles, a.Hl, m->Wo, m->Wot,
                            m->Wy, m->th, g->Y, g->target, g->phase, g->mask, alpha, a.Z, a.dPo, a.Sl, a.part_o);
     return hipGetLastError();
 }
@@ -1064,13 +1070,14 @@ void layer_bwd(gpsat_gnn_model* m, gpsat_gnn_graph* g, const Acts& a, int t)
 {
     const int N = LIT ? g->L : g->C;
     if (N == 0) return;
-    hipLaunchKernelGGL((k_layer_bwd<LIT, SELF, GATHER, LAST>), dim3(row_blocks(N)), dim3(256), 0, g->st,
+    constexpr int NW = LAST ? LAST_WAVES : LAYER_WAVES;
+    hipLaunchKernelGGL((k_layer_bwd<LIT, SELF, GATHER, LAST>), dim3(row_blocks(N, NW)), dim3(64 * NW), 0, g->st,
                        LIT ? g->l_off : g->c_off, LIT ? g->l_edges : g->c_edges, LIT ? g->c_off : g->l_off, N,
                        LIT ? m->Wlt : m->Wct,
                        (LIT ? a.mask_l : a.mask_c) + (size_t)t * N, LIT ? a.Mc : a.Ml, LIT ? a.Sl : a.Sc,
                        (LIT ? a.dPl : a.dPc) + (size_t)t * N * HID, LIT ? a.Ml : a.Mc,
-                       (LIT ? a.part_l : a.part_c) + (size_t)t * row_blocks(N) * HID,
-                       a.part_e + (LIT ? 0 : (size_t)row_blocks(g->L) * O_WC));
+                       (LIT ? a.part_l : a.part_c) + bias_slot(N, t) * HID,
+                       a.part_e + (LIT ? 0 : (size_t)row_blocks(g->L, LAST_WAVES) * O_WC));
 }
 
 // Backward pass from the readout's gradients to m->grad (every element written) and the loss.
@@ -1078,7 +1085,6 @@ hipError_t backward_pass(gpsat_gnn_model* m, gpsat_gnn_graph* g, const Acts& a)
 {
     hipStream_t st = g->st;
     const int R = g->R, L = g->L, C = g->C, V = g->V;
-    const int sl = L ? row_blocks(L) : 0, sc = C ? row_blocks(C) : 0;
     for (int t = R - 1; t >= 0; t--) {
         const bool top = t == R - 1;
         if (top && t)
@@ -1112,10 +1118,10 @@ hipError_t backward_pass(gpsat_gnn_model* m, gpsat_gnn_graph* g, const Acts& a)
         nb1 += width / 64 * gr;
         nb2 += (width + 255) / 256;
     };
-    job(a.part_o, V ? row_blocks(V, readout_tiles(V)) : 0, HEAD_PART, m->grad + O_BO, HEAD_GRADS, a.loss);
-    job(a.part_l, R * sl, HID, m->grad + O_BL, HID);
-    job(a.part_c, R * sc, HID, m->grad + O_BC, HID);
-    job(a.part_e, sl + sc, O_WC, m->grad, O_WC);
+    job(a.part_o, V ? row_blocks(V, 4 * readout_tiles(V)) : 0, HEAD_PART, m->grad + O_BO, HEAD_GRADS, a.loss);
+    job(a.part_l, (int)bias_slot(L, R), HID, m->grad + O_BL, HID);
+    job(a.part_c, (int)bias_slot(C, R), HID, m->grad + O_BC, HID);
+    job(a.part_e, row_blocks(L, LAST_WAVES) + row_blocks(C, LAST_WAVES), O_WC, m->grad, O_WC);
     job(a.part_wl, bl, 64 * 192, m->grad + O_WL, 64 * 192);
     job(a.part_wc, bc, 64 * 128, m->grad + O_WC, 64 * 128);
     job(a.part_wo, bo, 64 * 128, m->grad + O_WO, 64 * 128);
