@@ -16,7 +16,7 @@
 // Each half round is one kernel per direction (gather, product and elementwise work on rows
 // held in registers), as memory traffic and its latency bound the network, not arithmetic: the 172
 // GFLOP of a training pass over 512 x (n=300, m=1278) would take 0.15 ms at half of the MFMA
-// peak, moving its rows of ~4.6 GB about 1 ms.  The pass takes 1.78 ms, where separate gather, product,
+// peak, moving its rows of ~4.6 GB about 1 ms.  The pass takes 1.75 ms, where separate gather, product,
 // mask and reduction kernels moved ~9 GB in 3.70 ms; a layer's kernel runs at 3-4.3 TB/s of
 // compulsory bytes.
 #include <hip/hip_runtime.h>
@@ -91,25 +91,31 @@ __device__ __forceinline__ bf16x8 pack8(const float* x)
     for (int i = 0; i < 8; i++) v[i] = (__bf16)x[i];
     return v;
 }
-// this lane's 16 values of a 64-wide FP32 row: the columns in(i), or out(i)
-template <bool OUT = false>
+// this lane's 16 values of a 64-wide FP32 row: the columns in(i), or out(i).  NT: past the caches,
+// for rows that are next touched after more than they hold.
+typedef float v4f __attribute__((ext_vector_type(4)));
+template <bool OUT = false, bool NT = false>
 __device__ __forceinline__ void ld_row(float (&x)[16], const float* row, int q)
 {
-    const float4* p = reinterpret_cast<const float4*>(row) + (OUT ? q : 2 * q);
+    const v4f* p = reinterpret_cast<const v4f*>(row) + (OUT ? q : 2 * q);
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        const float4 v = p[OUT ? 4 * k : 8 * (k >> 1) + (k & 1)];
-        x[4 * k] = v.x;
-        x[4 * k + 1] = v.y;
-        x[4 * k + 2] = v.z;
-        x[4 * k + 3] = v.w;
+        const v4f* a = p + (OUT ? 4 * k : 8 * (k >> 1) + (k & 1));
+        const v4f v = NT ? __builtin_nontemporal_load(a) : *a;
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[4 * k + j] = v[j];
     }
 }
+template <bool NT = false>
 __device__ __forceinline__ void st_row(float* row, const float (&x)[16], int q)   // columns out(i)
 {
-    float4* p = reinterpret_cast<float4*>(row + 4 * q);
+    v4f* p = reinterpret_cast<v4f*>(row + 4 * q);
 #pragma unroll
-    for (int k = 0; k < 4; k++) p[4 * k] = make_float4(x[4 * k], x[4 * k + 1], x[4 * k + 2], x[4 * k + 3]);
+    for (int k = 0; k < 4; k++) {
+        const v4f v = {x[4 * k], x[4 * k + 1], x[4 * k + 2], x[4 * k + 3]};
+        if (NT) __builtin_nontemporal_store(v, p + 4 * k);
+        else p[4 * k] = v;
+    }
 }
 // the same values of the neighbouring row (l ^ 1: the other polarity of the variable)
 __device__ __forceinline__ bf16x8 flip8(bf16x8 v)
@@ -361,6 +367,7 @@ __global__ __launch_bounds__(64 * LAYER_WAVES, 4) void k_layer(const int32_t* __
 // (kept in BF16 for the weight gradient; its FP32 sum is the bias gradient) and dX = dP W: the
 // columns of this row's own H go to S in place (LIT: plus those the other polarity's row has for
 // it, exchanged between neighbouring lanes), the message columns to M.
+// NT (see layer_bwd): S is read once a round, a round after it was written, and passes the caches.
 // In the first round (LAST) what remains is the gradient of the embeddings, and dX is summed
 // here instead of stored: H_l^0 = occ(l)/8 u_l + v_l, so the own columns of a literal enter the
 // gradients of (u_l, v_l) with weights (occ(l)/8, 1), those of a clause (u_c, v_c) with
@@ -368,7 +375,7 @@ __global__ __launch_bounds__(64 * LAYER_WAVES, 4) void k_layer(const int32_t* __
 // (u_l, v_l) with (sum of occ(l)/8, len) / 4 -- a kernel that gathered them to the literals
 // again took 88 us, and the rows' stores 50, of 1.94 ms.
 // part: the workgroup's bias sums, 64 floats; part_e: those for u_l, v_l, u_c, v_c, 256.
-template <bool LIT, bool SELF, bool GATHER, bool LAST>
+template <bool LIT, bool SELF, bool GATHER, bool LAST, bool NT>
 __global__ __launch_bounds__(64 * (LAST ? LAST_WAVES : LAYER_WAVES), 4) void k_layer_bwd(const int32_t* __restrict__ off, const int32_t* __restrict__ edges,
                                                       const int32_t* __restrict__ n_off, int N,
                                                       const bf16_t* __restrict__ Wt, const uint2* __restrict__ mask, const float* __restrict__ G,
@@ -390,7 +397,7 @@ __global__ __launch_bounds__(64 * (LAST ? LAST_WAVES : LAYER_WAVES), 4) void k_l
     const uint32_t m = (m2.x >> 8 * q & 0xFF) | (m2.y >> 8 * q & 0xFF) << 8;
     float g[16], s[16];
     if constexpr (SELF)
-        ld_row(g, S + (size_t)row * HID, q);
+        ld_row<false, GATHER && NT>(g, S + (size_t)row * HID, q);   // (without GATHER S was just written)
     else {
 #pragma unroll
         for (int i = 0; i < 16; i++) g[i] = 0.f;
@@ -445,7 +452,7 @@ __global__ __launch_bounds__(64 * (LAST ? LAST_WAVES : LAYER_WAVES), 4) void k_l
         block_sum<true>(g, red, pe + (LIT ? O_UL : O_UC), lane, wave);
         if (LIT && threadIdx.x < 128) pe[O_UC + threadIdx.x] = 0.f;
     } else if (r < N)
-        st_row(S + (size_t)r * HID, g, q);
+        st_row<NT>(S + (size_t)r * HID, g, q);
 }
 
 // Readout of 16 variables per wavefront and tile: R = relu([H_{2v+1} | H_{2v}] W_o^T + b_o),
@@ -1071,13 +1078,22 @@ void layer_bwd(gpsat_gnn_model* m, gpsat_gnn_graph* g, const Acts& a, int t)
     const int N = LIT ? g->L : g->C;
     if (N == 0) return;
     constexpr int NW = LAST ? LAST_WAVES : LAYER_WAVES;
-    hipLaunchKernelGGL((k_layer_bwd<LIT, SELF, GATHER, LAST>), dim3(row_blocks(N, NW)), dim3(64 * NW), 0, g->st,
-                       LIT ? g->l_off : g->c_off, LIT ? g->l_edges : g->c_edges, LIT ? g->c_off : g->l_off, N,
-                       LIT ? m->Wlt : m->Wct,
-                       (LIT ? a.mask_l : a.mask_c) + (size_t)t * N, LIT ? a.Mc : a.Ml, LIT ? a.Sl : a.Sc,
-                       (LIT ? a.dPl : a.dPc) + (size_t)t * N * HID, LIT ? a.Ml : a.Mc,
-                       (LIT ? a.part_l : a.part_c) + bias_slot(N, t) * HID,
-                       a.part_e + (LIT ? 0 : (size_t)row_blocks(g->L, LAST_WAVES) * O_WC));
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(row_blocks(N, NW)), dim3(64 * NW), 0, g->st,
+                           LIT ? g->l_off : g->c_off, LIT ? g->l_edges : g->c_edges, LIT ? g->c_off : g->l_off, N,
+                           LIT ? m->Wlt : m->Wct,
+                           (LIT ? a.mask_l : a.mask_c) + (size_t)t * N, LIT ? a.Mc : a.Ml, LIT ? a.Sl : a.Sc,
+                           (LIT ? a.dPl : a.dPc) + (size_t)t * N * HID, LIT ? a.Ml : a.Mc,
+                           (LIT ? a.part_l : a.part_c) + bias_slot(N, t) * HID,
+                           a.part_e + (LIT ? 0 : (size_t)row_blocks(g->L, LAST_WAVES) * O_WC));
+    };
+    // Rows' gradients beyond the 256 MB last-level cache are kept out of it, which leaves it to the
+    // gathered ones (961,536 rows: the pass 1.78 -> 1.75 ms); smaller ones stay (235,000 rows: 519
+    // us, past the caches 529).
+    if ((int64_t)(g->L + (int64_t)g->C) * 2 * HID * 4 > (int64_t)256 << 20)
+        launch(k_layer_bwd<LIT, SELF, GATHER, LAST, true>);
+    else
+        launch(k_layer_bwd<LIT, SELF, GATHER, LAST, false>);
 }
 
 // Backward pass from the readout's gradients to m->grad (every element written) and the loss.

@@ -91,3 +91,32 @@ def test_graph_built_on_device_and_host(m, lo, hi):
             got.append(g.forward(Lr.GnnModel(theta))[:V])
             g.close()
     np.testing.assert_array_equal(got[0], got[1])
+
+
+def test_gradient_of_many_copies():
+    """A batch whose gradient rows exceed the last-level cache (576,000 rows of 512 bytes; they
+    pass the caches), as 512 copies of one formula: the loss is a mean over variables, and 512 a
+    power of two, so every row's gradient is the single formula's scaled exactly and only the
+    order of the FP32 sums differs (each a sum of the same terms, 2^-24 per addition over about
+    40 levels and runs, with some cancellation: 1e-4 of the block's norm)."""
+    print("[gnn shapes] 512 copies", flush=True)
+    rng = np.random.default_rng(5)
+    f = formula(rng, 180, 765, 3, 3)
+    theta = R.init_params(17)
+    lab = rng.random(180), (rng.random(180) < 0.5).astype(float), (rng.random(180) < 0.6).astype(float)
+    out = []
+    for k in (1, 512):
+        with G.GpuBatch(Batch.from_formulas([f] * k)) as gb:
+            g = Lr.GnnGraph(gb)
+            g.labels(*(np.tile(x, k) for x in lab))
+            out.append(g.loss_grad(Lr.GnnModel(theta)))
+            g.close()
+    (l1, g1, y1), (lk, gk, yk) = out
+    np.testing.assert_array_equal(np.tile(y1, (512, 1)), yk)
+    assert abs(l1 - lk) <= 1e-5 * abs(l1)
+    o = 0
+    for name, shp in R.PARAM_SHAPES:
+        k = int(np.prod(shp))
+        a, r = gk[o:o + k], g1[o:o + k]
+        o += k
+        assert np.linalg.norm(a - r) <= 1e-4 * max(np.linalg.norm(r), 1e-12), name
