@@ -63,8 +63,7 @@ __device__ __forceinline__ float from_bf16(bf16_t h) { return __uint_as_float((u
 // Memory is read and written in another lane order with the same columns: lane 4r + q, so that
 // four neighbouring lanes share a row and a float4 access of theirs falls in one 128-byte line
 // (with the product's own lane order every lane of a quad is on another row, and the address
-// unit takes four times as long: it bounded the clause layer at 168 us where 134 MB were read
-// and 332 MB written).  Registers change order through ds_bpermute, rows in BF16 on the way in
+// unit takes four times as long: the clause layer took 168 us instead of 146).  Registers change order through ds_bpermute, rows in BF16 on the way in
 // and results in FP32 on the way out (to_product, from_product).  So a layer is gather -> BF16
 // -> MFMA -> ReLU -> store without a trip through memory.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
