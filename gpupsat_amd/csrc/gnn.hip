@@ -10,7 +10,7 @@
 // Y_v = (branching score, phase logit).  The three 64-wide products run on MFMA
 // (v_mfma_f32_16x16x32_bf16): BF16 weights and BF16 inputs, FP32 accumulation.
 // Aggregations, biases, the 2-output head, the loss and Adam are FP32.  Gradients and the
-// loss are summed from per-wavefront (or per-workgroup) partials in a fixed order, never
+// loss are summed from per-workgroup partials in a fixed order, never
 // with floating-point atomics, so they are reproducible bit for bit.
 //
 // Each half round is one kernel per direction (gather, product and elementwise work on rows
@@ -63,11 +63,11 @@ __device__ __forceinline__ float from_bf16(bf16_t h) { return __uint_as_float((u
 // Memory is read and written in another lane order with the same columns: lane 4r + q, so that
 // four neighbouring lanes share a row and a float4 access of theirs falls in one 128-byte line
 // (with the product's own lane order every lane of a quad is on another row, and the address
-// unit takes four times as long: the clause layer took 168 us instead of 146).  Registers change order through ds_bpermute, rows in BF16 on the way in
-// and results in FP32 on the way out (to_product, from_product).  So a layer is gather -> BF16
-// -> MFMA -> ReLU -> store without a trip through memory.
+// unit takes four times as long: the clause layer took 168 us instead of 146).  Registers change
+// order through ds_bpermute, rows in BF16 on the way in and results in FP32 on the way out
+// (to_product, from_product).  So a layer is gather -> BF16 -> MFMA -> ReLU -> store without a
+// trip through memory.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ bf16x8 ld8(const bf16_t* p) { return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p)); }
 // (rows kept for the backward pass or the weight gradient: read again only after far more than
