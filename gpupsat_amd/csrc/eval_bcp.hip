@@ -958,6 +958,7 @@ __global__ __launch_bounds__(256) void k_eval_bcp3(const InstMeta* __restrict__ 
 // is cleared before this pass's barrier, after every wave has read it two barriers earlier),
 // and 192 count totals.
 constexpr int kPkAhead = 4;
+constexpr int kPkDirect = 12;
 
 __host__ __device__ constexpr int pk_lds_words(int W) { return 128 * W + 8 + 8 + 192; }
 
@@ -1180,8 +1181,12 @@ __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int
     // ends where the table ends; a batch of 8 NW words is read from it before any of the batch's
     // slots are written, and those end below the stage's later words (128 * 8NW(b + 1) <= 63W +
     // 65 * 8NW(b + 1) while W > 8NW(b + 1)).
-    RowWalk walk(tid, nthreads, W);
-    {
+    // Rows of at most kPkDirect words are read by their lanes, 2 or 3 loads each: there the copy's
+    // two barriers cost more than it saves (colourings of n = 120 x 3,300: staged 27.6 us, read
+    // directly 26.4; mixed k-SAT of n <= 190 x 999: 18.0, 17.9).
+    const bool direct = W <= kPkDirect;
+    if (!direct) {
+        RowWalk walk(tid, nthreads, W);
         uint32_t* stage = tab + 63 * W;
         const int nw = A * W;
         for (int ub = 0; ub < nw; ub += 8 * nthreads) {
@@ -1209,10 +1214,12 @@ __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             const int j = jb + wv + u * NW;
-            r[u] = (j < W && lane < A) ? tab[63 * W + 65 * j + lane] : 0u;
-            in_pop += __builtin_popcount(r[u]);
+            r[u] = 0u;
+            if (j < W && lane < A) r[u] = direct ? src[lane * W + j] : tab[63 * W + 65 * j + lane];
         }
-        __syncthreads();
+        if (!direct) __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 8; u++) in_pop += __builtin_popcount(r[u]);
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             const int j = jb + wv + u * NW;

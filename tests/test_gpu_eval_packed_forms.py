@@ -64,11 +64,11 @@ def test_colorings(orc, n_nodes):
                         np.testing.assert_array_equal(g, w)
 
 
-@pytest.mark.parametrize("n", [1, 16, 17, 127, 128, 129, 496, 511, 512, 513, 1024, 2016])
+@pytest.mark.parametrize("n", [1, 16, 17, 127, 128, 129, 192, 193, 496, 511, 512, 513, 1024, 2016])
 def test_row_lengths(orc, n):
     """Rows copied in and out a word at a time over all wavefronts: rows of 1 word, of the words
-    one batch of transposes takes (8, 16, 24 or 32, by the wavefronts) and one more, of the most
-    a table holds; beside an instance without variables."""
+    one batch of transposes takes (8, 16, 24 or 32, by the wavefronts) and one more, of the 12
+    that are read without a copy and one more, of the most a table holds; beside an instance without variables."""
     print("[packed forms] rows", n, flush=True)
     rng = np.random.default_rng(n)
     k = min(n, 4)
