@@ -110,7 +110,7 @@ int solve_plan(const DeviceBatch& d, const gpsat_solve_opts& o, int32_t n_jobs, 
     p.cus = prop.multiProcessorCount;
     const size_t lds_cu = prop.maxSharedMemoryPerMultiProcessor ? prop.maxSharedMemoryPerMultiProcessor : 65536;
     const size_t lds_block_max = prop.sharedMemPerBlock ? prop.sharedMemPerBlock : 65536;
-    const bool ids16 = o.clause_mem != 4 && solve_ids16(d.max_n, d.max_m, max_L, a.o);
+    const bool ids16 = o.clause_mem != 4 && solve_ids16(d.max_n, d.max_m, max_L, d.max_len, a.o);
     a.lay = solve_layout(d.max_n, d.max_m, max_L, d.all3 && ids16, ids16 ? 2 : 4, a.o);
     const size_t state_b = (size_t)a.lay.state_bytes;
     const size_t lds_hyb = state_b + (size_t)a.lay.watch_bytes, lds_all = lds_hyb + (size_t)a.lay.arena_bytes;

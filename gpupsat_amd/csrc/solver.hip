@@ -1588,10 +1588,11 @@ SolveLayout solve_layout(int32_t max_n, int32_t max_m, int64_t max_L, bool all3,
 }
 
 // 16-bit ids hold every literal (with a mark bit), clause id (with a none value), clause start in
-// units of 4 literals, clause length and list length of these sizes.
-bool solve_ids16(int32_t max_n, int32_t max_m, int64_t max_L, const SolveOptsDev& o)
+// units of 4 literals, clause length (max_len: the longest; literals may repeat, so n does not
+// bound it) and list length of these sizes.
+bool solve_ids16(int32_t max_n, int32_t max_m, int64_t max_L, int64_t max_len, const SolveOptsDev& o)
 {
-    return max_n < 16000 && (int64_t)max_m + o.learnt_cap < 65000 && max_L + 3 * (int64_t)max_m < 4 * 65000 &&
+    return max_n < 16000 && max_len <= UINT16_MAX && (int64_t)max_m + o.learnt_cap < 65000 && max_L + 3 * (int64_t)max_m < 4 * 65000 &&
            max_L < 65000 * 4 && (int64_t)o.larena_cap + 7 * (int64_t)o.learnt_cap < 8 * 65000 && o.watch_slack < 65000;
 }
 

@@ -122,7 +122,7 @@ int64_t solve_ref_ws_ints(int32_t n, int32_t m, int32_t ecap);
 hipError_t launch_solve_ref(const RefArgs& a, hipStream_t st);
 
 SolveLayout solve_layout(int32_t max_n, int32_t max_m, int64_t max_L, bool all3, int id_bytes, const SolveOptsDev& o);
-bool solve_ids16(int32_t max_n, int32_t max_m, int64_t max_L, const SolveOptsDev& o);
+bool solve_ids16(int32_t max_n, int32_t max_m, int64_t max_L, int64_t max_len, const SolveOptsDev& o);
 
 // Launch plan of one solve (solve_plan in capi_solve.cpp): mode 1 all job state in LDS,
 // 2 the clause part in HBM, 3 the watch structures in LDS and the learned literals in
