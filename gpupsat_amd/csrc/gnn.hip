@@ -767,8 +767,8 @@ __global__ void k_quantize(const float* __restrict__ th, bf16_t* __restrict__ Wc
 // from matching their codes bit by bit with ballots, so the order is that of a serial pass.
 // Built on the host this took 1.3 ms, and its copies 0.35 ms, of the 2.4 ms of an inference on
 // 256 x (n=300, m=1278).
-// clause_of: scratch, one int per edge.  Limits (see graph_on_device): the counters fit 64 KB of
-// LDS, and no clause is so long that one thread listing it is what takes the time.
+// clause_of: scratch, one int per edge.  Limits (see gnn_graph_on_device): the counters fit 64 KB
+// of LDS, and no clause is so long that one thread listing it is what takes the time.
 constexpr int GRAPH_WAVES = 4;
 __global__ __launch_bounds__(64 * GRAPH_WAVES) void k_graph(const InstMeta* __restrict__ meta, const int32_t* __restrict__ lits,
                                                             const int32_t* __restrict__ coff,
@@ -1145,15 +1145,6 @@ hipError_t backward_pass(gpsat_gnn_model* m, gpsat_gnn_graph* g, const Acts& a)
     return hipGetLastError();
 }
 
-// k_graph takes a batch whose instances' counters fit the LDS a workgroup may ask for (n <= 1,984:
-// 63.5 KB and the scan's 1 KB) and whose longest clause and largest instance one thread and one
-// wavefront get through in well under the host's time for the batch (64 literals; 65,536 edges:
-// 256 steps of 64 for each wavefront, ~0.1 ms).  Others are built on the host.
-bool graph_on_device(const DeviceBatch& d)
-{
-    return d.n_inst > 0 && d.max_n <= 1984 && d.max_len <= 64 && d.max_lits <= 65536;
-}
-
 hipError_t build_on_device(gpsat_gnn_graph* g, const DeviceBatch& d, const std::vector<int32_t>& var_base)
 {
     hipError_t e = hipMemcpyAsync(g->var_base, var_base.data(), 4 * (size_t)d.n_inst, hipMemcpyHostToDevice, g->st);
@@ -1280,7 +1271,7 @@ int gpsat_gnn_graph_create(gpsat_batch* b, int32_t rounds, gpsat_gnn_graph** out
     g->C = (int32_t)d.n_clauses;
     g->E = d.n_lits;
     hipError_t e = g->alloc(d.n_inst);
-    if (e == hipSuccess) e = graph_on_device(d) ? build_on_device(g, d, var_base) : build_on_host(g, d, var_base);
+    if (e == hipSuccess) e = gnn_graph_on_device(d, g->dev) ? build_on_device(g, d, var_base) : build_on_host(g, d, var_base);
     if (e != hipSuccess) {
         set_error(std::string("gnn graph: ") + hipGetErrorString(e));
         delete g;

@@ -105,6 +105,17 @@ EvalKernel eval_kernel(const DeviceBatch& b);
 // Words of HBM mask-table slices a general eval/BCP launch on this batch needs (0: none).
 size_t eval_bcp_gtab_words(const DeviceBatch& b);
 
+// Whether the branching network's incidence graph of batch d is built on the GPU (k_graph) for a
+// graph on device dev.  k_graph reads the batch's arrays, so only on the batch's own device; it
+// takes a batch whose instances' counters fit the LDS a workgroup may ask for (n <= 1,984: 63.5 KB
+// and the scan's 1 KB) and whose longest clause and largest instance one thread and one wavefront
+// get through in well under the host's time for the batch (64 literals; 65,536 edges: 256 steps of
+// 64 for each wavefront, ~0.1 ms).  Others are built on the host.
+inline bool gnn_graph_on_device(const DeviceBatch& d, int dev)
+{
+    return dev == d.device && d.n_inst > 0 && d.max_n <= 1984 && d.max_len <= 64 && d.max_lits <= 65536;
+}
+
 hipError_t launch_copy(const void* src, void* dst, int64_t bytes, hipStream_t st);
 
 hipError_t launch_preprocess(const DeviceBatch& b, int32_t* dlits, int32_t* dlen, int32_t* out_lits, int32_t* out_coff,

@@ -1,0 +1,37 @@
+"""Host rules that choose a path, compiled from the library's headers (no GPU needed)."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+import gpupsat_amd as G
+
+ROOT = os.path.dirname(G._HERE)
+
+
+def run_rules(tmp_path, body):
+    """Compile `body` (statements that print) against the internal headers, host pass only."""
+    hipcc = next((c for c in ("/opt/rocm/bin/hipcc", shutil.which("hipcc")) if c and os.path.exists(c)), None)
+    if hipcc is None:
+        pytest.skip("no hipcc")
+    src, exe = tmp_path / "rules.cpp", tmp_path / "rules"
+    src.write_text('#include <stdio.h>\n#include "gpsat_internal.hpp"\n#include "solver.hpp"\n'
+                   "using namespace gpsat;\nint main()\n{\n" + body + "\n}\n")
+    subprocess.run([hipcc, "-x", "hip", "--offload-arch=gfx950", "--offload-host-only", "-std=c++17", "-O1",
+                    "-I" + os.path.join(ROOT, "include"), "-I" + os.path.join(G._HERE, "csrc"), str(src), "-o", str(exe),
+                    "-L" + G._HERE, "-lgpsat", "-Wl,-rpath," + G._HERE], check=True, capture_output=True, text=True)
+    return subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split()
+
+
+def test_gnn_graph_is_built_where_its_batch_is(tmp_path):
+    """A graph on another device than its batch is built from the host's copies."""
+    got = run_rules(tmp_path, """
+    DeviceBatch d;
+    d.n_inst = 4; d.max_n = 100; d.max_len = 3; d.max_lits = 1278; d.n_lits = 4 * 1278;
+    for (int batch : {0, 1})
+        for (int dev : {0, 1}) {
+            d.device = batch;
+            printf("%d ", (int)gnn_graph_on_device(d, dev));
+        }""")
+    assert got == ["1", "0", "0", "1"]
