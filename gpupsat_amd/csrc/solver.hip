@@ -99,7 +99,9 @@ template <> struct Hdr<uint16_t> {
     static __device__ __forceinline__ void set_l0(type* h) { h->y &= 0xffffu; }
 };
 template <> struct Hdr<uint32_t> {
-    typedef uint4 type;
+    struct type {
+        uint32_t x, y, z;
+    };
     static __device__ __forceinline__ int32_t no(const type& h) { return (int32_t)h.y; }
     static __device__ __forceinline__ int32_t nl(const type& h) { return (int32_t)h.z; }
     static __device__ __forceinline__ int32_t add_o(type* h) { return (int32_t)atomicAdd(&h->y, 1u); }
@@ -124,7 +126,12 @@ template <> struct Hdr<uint32_t> {
 // ran.  So:
 //  * 16-bit ids, so that what a step reads is one record: a literal's header (list start and
 //    both lengths), a clause's record (its watches and literals), a variable's level and
-//    reason; the per-job state shrinks enough to hold the watch structures in LDS.
+//    reason; the per-job state shrinks enough to hold the watch structures in LDS.  With 32-bit
+//    ids (kShared: formulas whose watch structures are in HBM at any size) a wavefront keeps a
+//    clause's two watches only and reads its literals from the batch's arrays, which all
+//    wavefronts share: 20 bytes per 3-literal clause instead of the 52 of records and literals of
+//    its own, with which 8,192 wavefronts had room for 0.42 M clauses instead of 0.7 M, and 1,024
+//    cubes of 66,000 clauses over 2,000 variables took 73.7 ms instead of 60.2.
 //  * both watch lists of a literal are walked in one pass of the wavefront, one entry per lane,
 //    and the next literal's header and entries are fetched while the current one is processed
 //    (a queued literal's negation is false, so nothing moves a watch to its lists meanwhile).
@@ -137,6 +144,7 @@ struct Search {
     typedef typename Vec<I>::x4 I4;
     typedef Hdr<I> H;
     typedef typename H::type HT;
+    static constexpr bool kShared = sizeof(I) == 4;
     static constexpr I kNone = (I)~(I)0;
     static constexpr I kDrop = (I)((I)1 << (8 * sizeof(I) - 1));   // a literal dropped by minimization
 
@@ -159,6 +167,7 @@ struct Search {
     I* Wo;               // original-clause watch lists (capacity = occurrences)
     I4* rec;             // [m] ALL3: the three literals in order and the unwatched one; else the
                          // two watches, first literal / 4 in olits, length
+    I2* wrec;            // [m] in its place (kShared): the two watches
     I* Wl;               // learned-clause watch lists, slack slots per literal (index of the clause)
     I4* lrec;            // [learnt_cap] the two watches (kNone: detached), first literal / 8 in larena, length
     I* llbd;             // [learnt_cap]
@@ -166,6 +175,8 @@ struct Search {
     uint8_t* lused;      // [learnt_cap] used by an analysis since the last reduction
     I* olits;            // original literals (not ALL3), each clause filled up to a multiple of 4
                          // with the always-false literal
+    const I* lits;       // kShared: the instance's literals and clause offsets in the batch
+    const int32_t* coff;
     I* larena;           // learned literals, likewise to a multiple of 8
     int32_t slack, learnt_cap, larena_cap;
     // search state (uniform)
@@ -213,6 +224,7 @@ struct Search {
         phase = (int8_t*)(s + L.phase);
         mark = (uint8_t*)(s + L.mark);
         rec = (I4*)(w + L.rec);
+        wrec = (I2*)(w + L.rec);
         lrec = (I4*)(w + L.lrec);
         Wo = (I*)(w + L.wo);
         Wl = (I*)(w + L.wl);
@@ -273,9 +285,23 @@ struct Search {
         }
     }
 
-    // The first literal of a clause (its literals at q, filled up to a multiple of W with false
-    // ones) that is neither `other` nor false, kNone if none: W literals per round trip.
-    template <int W>
+    // The literals k .. k+3 of a clause of len literals at q; past its end, the false literals it
+    // is filled up with (FILLED), or its last literal again.
+    template <bool FILLED>
+    static __device__ __forceinline__ I4 four(const I* q, int32_t k, int32_t len)
+    {
+        if constexpr (FILLED) return *(const I4*)(q + k);
+        I4 y;
+        y.x = q[k];
+        y.y = q[min(k + 1, len - 1)];
+        y.z = q[min(k + 2, len - 1)];
+        y.w = q[min(k + 3, len - 1)];
+        return y;
+    }
+
+    // The first literal of a clause (its literals at q) that is neither `other` nor false, kNone
+    // if none: W literals per round trip.
+    template <int W, bool FILLED>
     __device__ __forceinline__ uint32_t find_watch(const I* q, int32_t len, uint32_t other) const
     {
         uint32_t rep = kNone;
@@ -283,7 +309,7 @@ struct Search {
             uint32_t x[W], v[W];
 #pragma unroll
             for (int t = 0; t < W; t += 4) {
-                const I4 y = *(const I4*)(q + k + t);
+                const I4 y = four<FILLED>(q, FILLED ? k + t : min(k + t, len - 1), len);
                 x[t] = y.x;
                 x[t + 1] = y.y;
                 x[t + 2] = y.z;
@@ -295,6 +321,38 @@ struct Search {
             for (int t = W - 1; t >= 0; t--) rep = min(v[t], x[t] ^ other) != 0u ? x[t] : rep;
         }
         return rep;
+    }
+
+    // Original clause e's record; its watches only (x and y) with kShared.
+    __device__ __forceinline__ I4 record(uint32_t e) const
+    {
+        if constexpr (!kShared) return rec[e];
+        const I2 w = wrec[e];
+        I4 r = {};
+        r.x = w.x;
+        r.y = w.y;
+        return r;
+    }
+
+    __device__ __forceinline__ void set_watches(uint32_t e, uint32_t x, uint32_t y)
+    {
+        I2 w;
+        w.x = (I)x;
+        w.y = (I)y;
+        if constexpr (kShared) wrec[e] = w;
+        else *(I2*)&rec[e] = w;
+    }
+
+    // Where the literals of original clause c with record r are (not ALL3).
+    __device__ __forceinline__ const I* original_lits(uint32_t c, I4 r, int32_t& len) const
+    {
+        if constexpr (kShared) {
+            const int32_t b = coff[c];
+            len = coff[c + 1] - b;
+            return lits + b;
+        }
+        len = (int32_t)r.w;
+        return olits + 4 * (uint32_t)r.z;
     }
 
     // One step of an original-clause list of the false literal fl (start ws), 64 entries from i0,
@@ -315,7 +373,11 @@ struct Search {
             other = (uint32_t)r.x + r.y - fl;
             open = in && confl < 0 && value(other) != 2;
             rep = kNone;
-            if (open && r.w > 2) rep = find_watch<4>(olits + 4 * (uint32_t)r.z, r.w, other);
+            if (open) {
+                int32_t len;
+                const I* q = original_lits(e, r, len);
+                if (len > 2) rep = find_watch<4, !kShared>(q, len, other);
+            }
             move = rep != (uint32_t)kNone;
         }
         const bool no = open && !move && value(other) == 0, unit = open && !move && !no;
@@ -327,10 +389,7 @@ struct Search {
             if (ALL3) {
                 rec[e].w = (I)fl;
             } else {
-                I2 w;
-                w.x = (I)other;
-                w.y = (I)rep;
-                *(I2*)&rec[e] = w;
+                set_watches(e, other, rep);
             }
         }
         const uint64_t km = ballot(in) & ~mm;
@@ -371,7 +430,7 @@ struct Search {
                 }
             }
         } else if (open) {
-            rep = find_watch<8>(larena + 8 * (uint32_t)r.z, r.w, other);
+            rep = find_watch<8, true>(larena + 8 * (uint32_t)r.z, r.w, other);
         }
         const bool move = rep != (uint32_t)kNone;
         const bool no = open && !move && vo == 0, unit = open && !move && vo != 0;
@@ -421,7 +480,7 @@ struct Search {
             int32_t keep = 0;
             for (int32_t i0 = 0; i0 < co; i0 += kWave) {
                 const uint32_t e = Wo[ws + min(i0 + (int32_t)lane, co - 1)];
-                step_original(fl, ws, i0, keep, i0 + (int32_t)lane < co, e, rec[e], confl);
+                step_original(fl, ws, i0, keep, i0 + (int32_t)lane < co, e, record(e), confl);
             }
             keep = 0;
             for (int32_t i0 = 0; i0 < cl; i0 += kWave) {
@@ -465,7 +524,7 @@ struct Search {
                 eo = ino ? eo : 0u;
                 el = inl ? el : 0u;
                 uint32_t fln = vec(trail[qhead]) ^ 1u;   // the next one, if one is queued
-                const I4 ro = rec[eo], rl = lrec[el];
+                const I4 ro = record(eo), rl = lrec[el];
                 HT hn = hdr[fln];
                 uint32_t lbn = fln * (uint32_t)slack;
                 uint32_t other, rep, vo, vq = 0;
@@ -572,6 +631,11 @@ struct Search {
     __device__ __forceinline__ const I* clause_lits(int32_t c, int32_t& len) const
     {
         if (c < m) {
+            if constexpr (kShared) {
+                const int32_t b = uni(coff[c]);
+                len = uni(coff[c + 1]) - b;
+                return lits + b;
+            }
             const I4 r = rec[c];
             len = uni((int32_t)r.w);
             return olits + 4 * uni((int32_t)r.z);
@@ -589,14 +653,23 @@ struct Search {
             const I4 x = rec[r];
             return min(min((uint32_t)vi[x.x >> 1].w, (uint32_t)vi[x.y >> 1].w), (uint32_t)vi[x.z >> 1].w) != 0u;
         }
+        if (kShared && r < m) {
+            int32_t len;
+            const I* q = original_lits(r, I4{}, len);
+            return all_in_clause<false>(q, len);
+        }
         const I4 x = r < m ? rec[r] : lrec[r - m];
-        const I* lits = r < m ? olits + 4 * (int32_t)x.z : larena + 8 * (int32_t)x.z;
-        const int32_t len = x.w;
+        return all_in_clause<true>(r < m ? olits + 4 * (int32_t)x.z : larena + 8 * (int32_t)x.z, x.w);
+    }
+
+    template <bool FILLED>
+    __device__ __forceinline__ bool all_in_clause(const I* q, int32_t len) const
+    {
         uint32_t all = 1;
         for (int32_t k = 0; k < len && all; k += 4) {
-            const I4 q = *(const I4*)(lits + k);
-            const int32_t a = q.x >> 1, b = k + 1 < len ? q.y >> 1 : a, c = k + 2 < len ? q.z >> 1 : a,
-                          d = k + 3 < len ? q.w >> 1 : a;
+            const I4 y = four<FILLED>(q, k, len);
+            const int32_t a = y.x >> 1, b = k + 1 < len ? y.y >> 1 : a, c = k + 2 < len ? y.z >> 1 : a,
+                          d = k + 3 < len ? y.w >> 1 : a;
             all = min(min((uint32_t)vi[a].w, (uint32_t)vi[b].w), min((uint32_t)vi[c].w, (uint32_t)vi[d].w));
         }
         return all != 0u;
@@ -1026,6 +1099,8 @@ struct Search {
         m = uni(mi.m);
         const int32_t* lits = a.lits + mi.lit_base;
         const int32_t* coff = a.coff + mi.coff_base;
+        this->lits = (const I*)lits;
+        this->coff = coff;
         const int32_t n2 = 2 * n;
         const int64_t vb = a.var_base[ins];
         slack = o.watch_slack;
@@ -1081,7 +1156,7 @@ struct Search {
                 len = full;
             }
             int32_t start = 0;
-            if (!ALL3) {
+            if (!ALL3 && !kShared) {
                 const int32_t quads = (full + 3) >> 2;
                 const int32_t s = wave_inclusive_scan(quads);
                 start = top + s - quads;
@@ -1105,18 +1180,22 @@ struct Search {
                 } else {
                     for (int32_t k = 0; k < full; k++) {
                         const int32_t q = lits[b + k];
-                        olits[4 * start + k] = (I)q;
+                        if (!kShared) olits[4 * start + k] = (I)q;
                         if (l1 < 0 && q != l0) l1 = q;
                         if (full <= 8)
                             for (int32_t j = 0; j < k; j++) twice |= (lits[b + j] >> 1) == (q >> 1);
                     }
-                    for (int32_t k = full; k & 3; k++) olits[4 * start + k] = (I)n2;
-                    I4 r;
-                    r.x = (I)l0;
-                    r.y = (I)l1;
-                    r.z = (I)start;
-                    r.w = (I)full;
-                    rec[c] = r;
+                    if (kShared) {
+                        set_watches(c, l0, l1);
+                    } else {
+                        for (int32_t k = full; k & 3; k++) olits[4 * start + k] = (I)n2;
+                        I4 r;
+                        r.x = (I)l0;
+                        r.y = (I)l1;
+                        r.z = (I)start;
+                        r.w = (I)full;
+                        rec[c] = r;
+                    }
                 }
                 if (l1 >= 0) {
                     len = 2;
@@ -1150,9 +1229,13 @@ struct Search {
             }
         }
         if (m == 0) {
-            I4 none;
-            none.x = none.y = none.z = none.w = 0;
-            rec[0] = none;
+            if (kShared) {
+                set_watches(0, 0, 0);
+            } else {
+                I4 none;
+                none.x = none.y = none.z = none.w = 0;
+                rec[0] = none;
+            }
         }
         dups = ballot(twice) != 0;
         shortl = ballot(longl) == 0;
@@ -1561,7 +1644,7 @@ SolveLayout solve_layout(int32_t max_n, int32_t max_m, int64_t max_L, bool all3,
     };
     L.id_bytes = id_bytes;
     L.lv = take(2 * n + 1);   // at the region's start: its address needs no addition
-    L.hdr = take(2 * n * (id_bytes == 2 ? 8 : 16));
+    L.hdr = take(2 * n * (id_bytes == 2 ? 8 : 12));
     L.vi = take(n * 4 * I);
     L.act = take(n * 4);
     L.lstamp = take((n + 2) * 4);
@@ -1573,14 +1656,14 @@ SolveLayout solve_layout(int32_t max_n, int32_t max_m, int64_t max_L, bool all3,
     L.state_bytes = at;
     at = 0;
     // a list is read by all 64 lanes, and clause 0 also where there is none
-    L.rec = take((int64_t)(max_m + 1) * 4 * I);
+    L.rec = take((int64_t)(max_m + 1) * (id_bytes == 2 ? 4 : 2) * I);
     L.lrec = take((int64_t)o.learnt_cap * 4 * I);
     L.wo = take((max_L + 64) * I);
     L.wl = take((2 * n * o.watch_slack + 64) * I);
     L.llbd = take(o.learnt_cap * I);
     L.remap = take(o.learnt_cap * I);
     L.lused = take(o.learnt_cap);
-    L.olits = take(all3 ? 0 : (max_L + 3 * (int64_t)max_m) * I);
+    L.olits = take(all3 || id_bytes == 4 ? 0 : (max_L + 3 * (int64_t)max_m) * I);
     L.watch_bytes = at;
     L.arena_bytes = ((int64_t)o.larena_cap + 7 * (int64_t)o.learnt_cap) * I;
     L.arena_bytes = (L.arena_bytes + 15) & ~(int64_t)15;

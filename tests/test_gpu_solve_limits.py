@@ -5,6 +5,7 @@ import pytest
 
 import gpupsat_amd as G
 from gpupsat_amd.formula import Batch, Formula
+from test_gpu_solve_paths import _formulas
 
 pytestmark = pytest.mark.gpu
 
@@ -22,3 +23,24 @@ def test_clause_length_beyond_16_bits(length):
             r = gb.solve(G.SolveOpts.default(clause_mem=mem))
             assert r["status"].tolist() == [G.SAT, G.UNSAT]
             assert r["verified"].tolist() == [1, 0]
+
+
+@pytest.mark.parametrize("kind", ["chain", "hub3", "repeat3", "mixed"])
+def test_32_bit_ids_run_the_same_search(kind):
+    """The search with 32-bit ids (a cap of 66,000 learned clauses asks for them; its clauses'
+    literals are the batch's, not the wavefront's) against the one with 16-bit ids: neither fills
+    its cap, so models and counters are equal.  With the whole state in HBM (placement 4) only the
+    verdicts are: lanes that move a watch to the same literal in one step append to its list in
+    the order that their atomics reach the cache, which is not the lanes' order as in LDS, and the
+    order of a list decides which of several conflicts is met first."""
+    batch = Batch.from_formulas(_formulas(kind))
+    ref = None
+    with G.GpuBatch(batch) as gb:
+        for cap, mem in ((20000, 1), (20000, 2), (66000, 2), (66000, 4)):
+            print("[solve limits]", kind, "learnt_cap", cap, "clause_mem", mem, flush=True)
+            r = gb.solve(G.SolveOpts.default(clause_mem=mem, phase_init=1, learnt_cap=cap, larena_cap=300000,
+                                             max_conflicts=4000), want_bumps=True)
+            got = r["status"], r["model_rows"], r["job_stats"][:, :7], r["var_bumps"]
+            ref = ref or got
+            for x, y in list(zip(got, ref))[: 1 if mem == 4 else 4]:
+                np.testing.assert_array_equal(x, y)
