@@ -111,7 +111,7 @@ int solve_plan(const DeviceBatch& d, const gpsat_solve_opts& o, int32_t n_jobs, 
     const size_t lds_cu = prop.maxSharedMemoryPerMultiProcessor ? prop.maxSharedMemoryPerMultiProcessor : 65536;
     const size_t lds_block_max = prop.sharedMemPerBlock ? prop.sharedMemPerBlock : 65536;
     const bool ids16 = o.clause_mem != 4 && solve_ids16(d.max_n, d.max_m, max_L, d.max_len, a.o);
-    a.lay = solve_layout(d.max_n, d.max_m, max_L, d.all3 && ids16, ids16 ? 2 : 4, a.o);
+    a.lay = solve_layout(d.max_n, d.max_m, max_L, d.all3, ids16 ? 2 : 4, a.o);
     const size_t state_b = (size_t)a.lay.state_bytes;
     const size_t lds_hyb = state_b + (size_t)a.lay.watch_bytes, lds_all = lds_hyb + (size_t)a.lay.arena_bytes;
     int mode;
@@ -148,7 +148,7 @@ int solve_plan(const DeviceBatch& d, const gpsat_solve_opts& o, int32_t n_jobs, 
         }
         if (!few_jobs && lds_all <= lds_block_max && estimate(1, lds_all, 1.0, 0.0, 3.2) < best) mode = 1;
     }
-    if (mode == 4) a.lay = solve_layout(d.max_n, d.max_m, max_L, false, 4, a.o);
+    if (mode == 4) a.lay = solve_layout(d.max_n, d.max_m, max_L, d.all3, 4, a.o);
     const int64_t slice = a.lay.arena_bytes + (mode == 2 || mode == 4 ? a.lay.watch_bytes : 0) +
                           (mode == 4 ? a.lay.state_bytes : 0);
     a.ws_ints_per_wave = (slice / 4 + 63) & ~(int64_t)63;

@@ -128,8 +128,8 @@ template <> struct Hdr<uint32_t> {
 //    both lengths), a clause's record (its watches and literals), a variable's level and
 //    reason; the per-job state shrinks enough to hold the watch structures in LDS.  With 32-bit
 //    ids (kShared: formulas whose watch structures are in HBM at any size) a wavefront keeps a
-//    clause's two watches only and reads its literals from the batch's arrays, which all
-//    wavefronts share: 20 bytes per 3-literal clause instead of the 52 of records and literals of
+//    clause's two watches (or one unwatched literal of three) only and reads its literals from the
+//    batch's arrays, which all wavefronts share: 16 to 20 bytes per 3-literal clause instead of the 52 of records and literals of
 //    its own, with which 8,192 wavefronts had room for 0.42 M clauses instead of 0.7 M, and 1,024
 //    cubes of 66,000 clauses over 2,000 variables took 73.7 ms instead of 60.2.
 //  * both watch lists of a literal are walked in one pass of the wavefront, one entry per lane,
@@ -167,7 +167,8 @@ struct Search {
     I* Wo;               // original-clause watch lists (capacity = occurrences)
     I4* rec;             // [m] ALL3: the three literals in order and the unwatched one; else the
                          // two watches, first literal / 4 in olits, length
-    I2* wrec;            // [m] in its place (kShared): the two watches
+    I2* wrec;            // [m] in its place with kShared: the two watches, or
+    I* urec;             // [m] (ALL3) the unwatched literal
     I* Wl;               // learned-clause watch lists, slack slots per literal (index of the clause)
     I4* lrec;            // [learnt_cap] the two watches (kNone: detached), first literal / 8 in larena, length
     I* llbd;             // [learnt_cap]
@@ -225,6 +226,7 @@ struct Search {
         mark = (uint8_t*)(s + L.mark);
         rec = (I4*)(w + L.rec);
         wrec = (I2*)(w + L.rec);
+        urec = (I*)(w + L.rec);
         lrec = (I4*)(w + L.lrec);
         Wo = (I*)(w + L.wo);
         Wl = (I*)(w + L.wl);
@@ -323,15 +325,29 @@ struct Search {
         return rep;
     }
 
-    // Original clause e's record; its watches only (x and y) with kShared.
+    // Original clause e's record; its watches only (x and y) with kShared and not ALL3.
     __device__ __forceinline__ I4 record(uint32_t e) const
     {
         if constexpr (!kShared) return rec[e];
-        const I2 w = wrec[e];
         I4 r = {};
-        r.x = w.x;
-        r.y = w.y;
+        if constexpr (ALL3) {
+            const I* q = lits + 3 * e;
+            r.x = q[0];
+            r.y = q[1];
+            r.z = q[2];
+            r.w = urec[e];
+        } else {
+            const I2 w = wrec[e];
+            r.x = w.x;
+            r.y = w.y;
+        }
         return r;
+    }
+
+    __device__ __forceinline__ void set_unwatched(uint32_t e, uint32_t u)
+    {
+        if constexpr (kShared) urec[e] = (I)u;
+        else rec[e].w = (I)u;
     }
 
     __device__ __forceinline__ void set_watches(uint32_t e, uint32_t x, uint32_t y)
@@ -387,7 +403,7 @@ struct Search {
             H::sub_o(&hdr[fl]);
             Wo[at] = (I)e;
             if (ALL3) {
-                rec[e].w = (I)fl;
+                set_unwatched(e, fl);
             } else {
                 set_watches(e, other, rep);
             }
@@ -501,6 +517,13 @@ struct Search {
         return x;
     }
 
+    // This lane's entry of a list of k <= 64 (lanes past it: any).  Lists in HBM are read no
+    // further than they go.
+    static __device__ __forceinline__ uint32_t entry(const I* list, int32_t k)
+    {
+        return list[kShared ? min((int32_t)lane_id(), max(k - 1, 0)) : (int32_t)lane_id()];
+    }
+
     __device__ __forceinline__ int32_t propagate()
     {
         if (!shortl) return propagate_long();
@@ -515,7 +538,7 @@ struct Search {
             HT h = hdr[fl];
             uint32_t lb = fl * (uint32_t)slack;
             bool fetched;
-            uint32_t eo = Wo[h.x + lane], el = Wl[lb + lane];
+            uint32_t eo = entry(Wo + h.x, H::no(h)), el = entry(Wl + lb, H::nl(h));
             for (;;) {
                 qhead++;
                 props++;
@@ -539,7 +562,7 @@ struct Search {
                 vo = value(other);
                 const uint32_t lother = learned_other(rl, fl);
                 uint32_t vl = value(lother);
-                uint32_t eon = Wo[hn.x + lane], eln = Wl[lbn + lane];
+                uint32_t eon = entry(Wo + hn.x, H::no(hn)), eln = entry(Wl + lbn, H::nl(hn));
                 vo = ino ? vo : 2u;
                 vl = inl ? vl : 2u;
                 // (decisions are single compares: a ballot of one goes straight to scalar
@@ -552,7 +575,7 @@ struct Search {
                             const uint32_t at = (uint32_t)hdr[rep].x + H::add_o(&hdr[rep]);
                             H::sub_o(&hdr[fl]);
                             Wo[at] = (I)eo;
-                            rec[eo].w = (I)fl;
+                            set_unwatched(eo, fl);
                         } else if (ino) {
                             Wo[ws + lane - prefix_count(mm)] = (I)eo;
                         }
@@ -582,8 +605,8 @@ struct Search {
                                 fln = vec(trail[qhead]) ^ 1u;
                                 hn = hdr[fln];
                                 lbn = fln * (uint32_t)slack;
-                                eon = Wo[hn.x + lane];
-                                eln = Wl[lbn + lane];
+                                eon = entry(Wo + hn.x, H::no(hn));
+                                eln = entry(Wl + lbn, H::nl(hn));
                                 queued = tsize;
                             }
                         }
@@ -650,7 +673,7 @@ struct Search {
     __device__ __forceinline__ bool implied(int32_t r) const
     {
         if (ALL3 && r < m) {
-            const I4 x = rec[r];
+            const I4 x = record(r);
             return min(min((uint32_t)vi[x.x >> 1].w, (uint32_t)vi[x.y >> 1].w), (uint32_t)vi[x.z >> 1].w) != 0u;
         }
         if (kShared && r < m) {
@@ -716,7 +739,7 @@ struct Search {
         int32_t nl = 1, c = confl, j = 0;
         do {
             if (ALL3 && c < m) {
-                const I4 r = rec[c];
+                const I4 r = record(c);
                 const int32_t q = lane == 0 ? r.x : lane == 1 ? r.y : r.z;
                 const I4 x = vi[q >> 1];
                 const uint32_t ra = end - (uint32_t)vi[r.x >> 1].z, rb = end - (uint32_t)vi[r.y >> 1].z,
@@ -779,7 +802,7 @@ struct Search {
             int32_t len = 3;
             const I* cl = nullptr;
             I4 r3 = {};
-            if (ALL3 && c < m) r3 = rec[c];
+            if (ALL3 && c < m) r3 = record(c);
             else cl = clause_lits(c, len);
             if (c >= m && lane == 0) lused[c - m] = 1;
             for (int32_t k0 = 0; k0 < len; k0 += kWave) {
@@ -1099,7 +1122,8 @@ struct Search {
         m = uni(mi.m);
         const int32_t* lits = a.lits + mi.lit_base;
         const int32_t* coff = a.coff + mi.coff_base;
-        this->lits = (const I*)lits;
+        // (without clauses the lanes that have no list entry read their own first record instead)
+        this->lits = m ? (const I*)lits : (const I*)urec;
         this->coff = coff;
         const int32_t n2 = 2 * n;
         const int64_t vb = a.var_base[ins];
@@ -1171,12 +1195,16 @@ struct Search {
                     if (y != l0) l1 = y;
                     else if (z != l0) l1 = z;
                     twice |= (y >> 1) == (l0 >> 1) || (z >> 1) == (l0 >> 1) || (y >> 1) == (z >> 1);
-                    I4 r;
-                    r.x = (I)l0;
-                    r.y = (I)y;
-                    r.z = (I)z;
-                    r.w = (I)rest;
-                    rec[c] = r;
+                    if (kShared) {
+                        set_unwatched(c, rest);
+                    } else {
+                        I4 r;
+                        r.x = (I)l0;
+                        r.y = (I)y;
+                        r.z = (I)z;
+                        r.w = (I)rest;
+                        rec[c] = r;
+                    }
                 } else {
                     for (int32_t k = 0; k < full; k++) {
                         const int32_t q = lits[b + k];
@@ -1229,7 +1257,9 @@ struct Search {
             }
         }
         if (m == 0) {
-            if (kShared) {
+            if (kShared && ALL3) {
+                set_unwatched(0, 0);
+            } else if (kShared) {
                 set_watches(0, 0, 0);
             } else {
                 I4 none;
@@ -1656,7 +1686,7 @@ SolveLayout solve_layout(int32_t max_n, int32_t max_m, int64_t max_L, bool all3,
     L.state_bytes = at;
     at = 0;
     // a list is read by all 64 lanes, and clause 0 also where there is none
-    L.rec = take((int64_t)(max_m + 1) * (id_bytes == 2 ? 4 : 2) * I);
+    L.rec = take((int64_t)(max_m + 1) * (id_bytes == 2 ? 4 : all3 ? 1 : 2) * I);
     L.lrec = take((int64_t)o.learnt_cap * 4 * I);
     L.wo = take((max_L + 64) * I);
     L.wl = take((2 * n * o.watch_slack + 64) * I);
@@ -1695,8 +1725,12 @@ hipError_t launch_solve(const SolveArgs& a, int clause_mem, int waves, size_t ld
     const dim3 grid(waves / wpb), block(kWave * wpb);
     const size_t lds = lds_bytes * wpb;
     const bool ids16 = a.lay.id_bytes == 2;
-    if (clause_mem == 4)
+    if (clause_mem == 4 && a.all3)
+        hipLaunchKernelGGL((k_solve<4, uint32_t, true>), grid, block, 0, st, a);
+    else if (clause_mem == 4)
         hipLaunchKernelGGL((k_solve<4, uint32_t, false>), grid, block, 0, st, a);
+    else if (!ids16 && a.all3)
+        hipLaunchKernelGGL((k_solve<2, uint32_t, true>), grid, block, lds, st, a);
     else if (!ids16)
         hipLaunchKernelGGL((k_solve<2, uint32_t, false>), grid, block, lds, st, a);
     else if (a.all3)

@@ -39,9 +39,10 @@ def test_gnn_graph_is_built_where_its_batch_is(tmp_path):
 
 def test_large_formulas_keep_their_memory_per_wavefront(tmp_path):
     """Bytes of a wavefront's state with 32-bit ids: 63 a variable, two watch list entries of 4
-    for each learned-clause slot of its literals, 4 a literal and 8 a clause, 53 a learned clause
-    besides the literals it may hold, and at most 1 KB of rounding (each of 19 arrays to 16
-    bytes, 64 entries read past two of them)."""
+    for each learned-clause slot of its literals, 4 a literal and 8 a clause (4 where all have
+    three literals: the one that is not watched), 53 a learned clause besides the
+    literals it may hold, and at most 1 KB of rounding (each of 19 arrays to 16 bytes, 64 entries
+    read past two of them)."""
     got = run_rules(tmp_path, """
     SolveOptsDev o{};
     for (int all3 : {0, 1})
@@ -50,7 +51,7 @@ def test_large_formulas_keep_their_memory_per_wavefront(tmp_path):
                 o.learnt_cap = 256; o.larena_cap = 32 * 256 + n; o.watch_slack = 8;
                 const long L = 3l * m + (all3 ? 0 : 12345);
                 const SolveLayout lay = solve_layout(n, m, L, all3, 4, o);
-                const long most = 63l * n + 2l * n * 8 * 4 + 4 * L + 8l * m + 53l * o.learnt_cap + 4l * o.larena_cap + 1024;
+                const long most = 63l * n + 2l * n * 8 * 4 + 4 * L + (all3 ? 4l : 8l) * m + 53l * o.learnt_cap + 4l * o.larena_cap + 1024;
                 printf("%d ", (int)(lay.state_bytes + lay.watch_bytes + lay.arena_bytes <= most));
             }""")
     assert got == ["1"] * 12
