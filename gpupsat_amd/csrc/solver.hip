@@ -1085,13 +1085,30 @@ struct Search {
     {
         uint32_t best = 0;
         int32_t bv = 0;
-        for (int32_t v = lane_id(); v < n; v += kWave) {
-            if (lv[2 * v] == 1) {
-                // non-negative floats order as integers
-                const uint32_t key = mode == 1 ? (uint32_t)v + 1u : (__float_as_uint(act[v]) | 0x80000000u);
-                if (key > best) {
-                    best = key;
-                    bv = v;
+        // With the state in HBM a trip takes about 0.6 us, so eight variables of each lane are read
+        // at once, assigned or not (n = 20,000, 1,024 wavefronts: a decision 0.19 ms one by one, 0.05
+        // eight at a time).
+        constexpr int kAtOnce = kMode == 4 ? 8 : 1;
+        for (int32_t v0 = lane_id(); v0 < n; v0 += kAtOnce * kWave) {
+            uint32_t val[kAtOnce];
+            float score[kAtOnce];
+#pragma unroll
+            for (int u = 0; u < kAtOnce; u++) {
+                const int32_t v = min(v0 + u * kWave, n - 1);
+                val[u] = lv[2 * v];
+                if (kMode == 4) score[u] = act[v];
+            }
+#pragma unroll
+            for (int u = 0; u < kAtOnce; u++) {
+                const int32_t v = v0 + u * kWave;
+                if (val[u] == 1 && v < n) {
+                    // non-negative floats order as integers
+                    const float a = kMode == 4 ? score[u] : act[v];
+                    const uint32_t key = mode == 1 ? (uint32_t)v + 1u : (__float_as_uint(a) | 0x80000000u);
+                    if (key > best) {
+                        best = key;
+                        bv = v;
+                    }
                 }
             }
         }

@@ -44,3 +44,25 @@ def test_32_bit_ids_run_the_same_search(kind):
             ref = ref or got
             for x, y in list(zip(got, ref))[: 1 if mem == 4 else 4]:
                 np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("decision", [0, 1])
+def test_branching_variable_with_the_state_in_hbm(decision):
+    """The next variable to branch on, found eight at a time per lane (512 a step) where the
+    state is in HBM: the same as in LDS, ties included.  Clauses of two literals that share no
+    variable: the model shows which of the two was decided first, and no watch list holds two
+    clauses (with two, their order could differ, as above)."""
+    rng = np.random.default_rng(3)
+    fs = [Formula.from_clauses(n, [[2 * int(x) + 1 for x in v] for v in rng.permutation(n)[: n // 2 * 2].reshape(-1, 2)])
+          for n in (1, 63, 64, 65, 511, 512, 513, 575, 576, 577, 1100)]
+    batch = Batch.from_formulas(fs)
+    act = rng.integers(0, 4, int(batch.n_vars.sum())).astype(np.float32)
+    got = []
+    with G.GpuBatch(batch) as gb:
+        for mem in (2, 4):
+            print("[solve limits] branching, decision", decision, "clause_mem", mem, flush=True)
+            r = gb.solve(G.SolveOpts.default(clause_mem=mem, decision=decision, max_conflicts=1000), act_init=act)
+            assert r["info"]["clause_mem"] == mem
+            got.append((r["status"], r["model_rows"], r["job_stats"][:, :7]))
+    for x, y in zip(*got):
+        np.testing.assert_array_equal(x, y)
