@@ -180,7 +180,14 @@ inline int solve_core(gpsat_batch* b, const gpsat_solve_opts& o, const int32_t* 
             }
             set_waves(plan, fit);
         }
-        HIP_OR(mem.alloc(d_ws, (size_t)plan.waves * a.ws_ints_per_wave));
+        hipError_t we = mem.alloc(d_ws, (size_t)plan.waves * a.ws_ints_per_wave);
+        // a large formula's slices may not all fit the GPU: then the jobs share fewer wavefronts
+        while (!Mem::kNoAlloc && we == hipErrorOutOfMemory && plan.waves > plan.wpb) {
+            (void)hipGetLastError();
+            set_waves(plan, plan.waves / 2 / plan.wpb * plan.wpb);
+            we = mem.alloc(d_ws, (size_t)plan.waves * a.ws_ints_per_wave);
+        }
+        HIP_OR(we);
     }
     a.chunk = plan.chunk;
     const int waves = plan.waves;

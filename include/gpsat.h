@@ -197,7 +197,8 @@ typedef struct gpsat_solve_opts {
     int32_t phase_init;      /* initial phase without a hint: 0 false, 1 true */
     double max_ms;           /* per-job wall-clock budget in ms (<= 0: none), exceeded -> UNDEF */
     int32_t waves;           /* persistent wavefronts (0: automatic, up to 16 per CU, 32 with the
-                                clause part in HBM, as LDS allows) */
+                                clause part in HBM, as LDS allows); fewer if their state does not
+                                fit the GPU's memory */
     int32_t clause_mem;      /* clause part of the job state: 0 automatic, 1 LDS, 2 HBM, 3 the watch
                                 lists and clause records in LDS, the learned clauses' literals in
                                 HBM, 4 the whole job state in HBM.  Automatic: with at most 4 jobs

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import gpupsat_amd as G
+from gpupsat_amd import workloads as W
 from gpupsat_amd.formula import Batch, Formula
 from test_gpu_solve_paths import _formulas
 
@@ -66,3 +67,14 @@ def test_branching_variable_with_the_state_in_hbm(decision):
             got.append((r["status"], r["model_rows"], r["job_stats"][:, :7]))
     for x, y in zip(*got):
         np.testing.assert_array_equal(x, y)
+
+
+def test_workspace_larger_than_the_gpu(orc):
+    """64 jobs with room for 1.9e9 learned literals each (7.6 GB a wavefront, 486 GB in all) share
+    as many wavefronts as there is memory for."""
+    print("[solve limits] 7.6 GB a wavefront", flush=True)
+    batch = W.random_3sat_batch(64, 20, 85, seed=4)
+    with G.GpuBatch(batch) as gb:
+        r = gb.solve(G.SolveOpts.default(larena_cap=1900000000))
+    assert 1 <= r["info"]["waves"] <= 32
+    assert r["status"].tolist() == [orc.solve_cdcl(batch.instance(i))[0] for i in range(64)]
