@@ -169,6 +169,20 @@ inline int solve_core(gpsat_batch* b, const gpsat_solve_opts& o, const int32_t* 
     if (var_bumps) HIP_OR(mem.alloc(d_bumps, (size_t)var_base[N]));
     if (act_init) HIP_OR(mem.alloc(d_act, (size_t)var_base[N]));
     if (phase_init) HIP_OR(mem.alloc(d_phase, (size_t)var_base[N]));
+    if (Mem::kNoAlloc && plan.mode != 1 && o.clause_mem == 0) {
+        // where a fixed region has room for few slices, or none, the automatic placement is the LDS
+        // if the state fits it, as long as that runs more wavefronts
+        gpsat_solve_opts in_lds = o;
+        in_lds.clause_mem = 1;
+        SolveArgs la{};
+        SolvePlan lp{};
+        const size_t fit = mem.remaining() / (4 * (size_t)a.ws_ints_per_wave);
+        if (fit < (size_t)plan.waves && solve_plan(d, in_lds, n_jobs, la, lp) == GPSAT_OK && lp.mode == 1 &&
+            (size_t)lp.waves > fit) {
+            a = la;
+            plan = lp;
+        }
+    }
     if (plan.mode != 1) {
         // the workspace slices come last: a fixed region holds as many as are left room for
         const size_t slice = 4 * (size_t)a.ws_ints_per_wave;

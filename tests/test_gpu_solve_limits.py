@@ -7,6 +7,7 @@ import gpupsat_amd as G
 from gpupsat_amd import workloads as W
 from gpupsat_amd.formula import Batch, Formula
 from test_gpu_solve_paths import _formulas
+from test_zz_no_alloc import _call
 
 pytestmark = pytest.mark.gpu
 
@@ -78,3 +79,28 @@ def test_workspace_larger_than_the_gpu(orc):
         r = gb.solve(G.SolveOpts.default(larena_cap=1900000000))
     assert 1 <= r["info"]["waves"] <= 32
     assert r["status"].tolist() == [orc.solve_cdcl(batch.instance(i))[0] for i in range(64)]
+
+
+def test_noalloc_with_the_scratch_region_full():
+    """4,000 jobs whose cubes (their literals repeated) leave 8 KB of the 64 MiB scratch region,
+    less than one wavefront's learned literals: the job state goes to LDS, which needs none."""
+    f = W.random_3sat_batch(1, 10, 20, seed=5).instance(0)
+    batch = Batch.from_formulas([f, W.pigeonhole_formula(4, 3)])
+    J, N = 4000, 2
+    up = lambda n: (n + 255) // 256 * 256                                 # noqa: E731
+    words = 2
+    table = [16 * J, 4, 8, 8 * N, 4 * N, 4 * N, 4 * N, 4 * N, 8 * (N + 1), 8 * len(G.JOB_STAT_FIELDS) * J, 4 * words, 12 * N]
+    total = ((64 << 20) - sum(up(x) for x in table) - 8192) // 256 * 256 // 4
+    per = np.full(J, total // J)
+    per[: total - per.sum()] += 1
+    ji = np.repeat(np.arange(2, dtype=np.int32), J // 2)
+    co = np.concatenate([[0], np.cumsum(per)]).astype(np.int32)
+    assert co[-1] == total
+    cl = (np.repeat(np.arange(J), per) % 2 + 2 * np.repeat(np.arange(J) // 2 % 10, per)).astype(np.int32)
+    with G.GpuBatch(batch) as gb:
+        assert gb.row_words(1) == words
+        print("[solve limits] scratch region full", flush=True)
+        rc, status, *_, info = _call("gpsat_solve_noalloc", gb, G.SolveOpts.default(), jobs=(ji, co, cl))
+        assert rc == 0, G.lib().gpsat_last_error()
+    assert status.tolist() == [G.SAT, G.UNSAT]
+    assert info.clause_mem == 1 and info.workspace_bytes == 0
