@@ -109,11 +109,15 @@ size_t eval_bcp_gtab_words(const DeviceBatch& b);
 // graph on device dev.  k_graph reads the batch's arrays, so only on the batch's own device; it
 // takes a batch whose instances' counters fit the LDS a workgroup may ask for (n <= 1,984: 63.5 KB
 // and the scan's 1 KB) and whose longest clause and largest instance one thread and one wavefront
-// get through in well under the host's time for the batch (64 literals; 65,536 edges: 256 steps of
-// 64 for each wavefront, ~0.1 ms).  Others are built on the host.
+// get through: 64 literals, 65,536 edges.  Where the device is the faster one: k_graph gives an
+// instance one workgroup, so a call takes 48 us + 4.4 ns per edge of the largest instance, where the
+// host takes 92 us + 1.45 ns per edge of the whole batch and more beyond its caches (us, device and
+// host: one instance of 8,000 edges 83 and 110, of 16,000 118 and 108, of 32,000 190 and 127, of
+// 65,000 333 and 175; three of 32,000 191 and 207; 16 of 1,000 60 and 160).
 inline bool gnn_graph_on_device(const DeviceBatch& d, int dev)
 {
-    return dev == d.device && d.n_inst > 0 && d.max_n <= 1984 && d.max_len <= 64 && d.max_lits <= 65536;
+    return dev == d.device && d.n_inst > 0 && d.max_n <= 1984 && d.max_len <= 64 && d.max_lits <= 65536 &&
+           3 * d.max_lits <= d.n_lits + 25000;
 }
 
 hipError_t launch_copy(const void* src, void* dst, int64_t bytes, hipStream_t st);

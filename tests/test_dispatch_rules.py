@@ -55,3 +55,19 @@ def test_large_formulas_keep_their_memory_per_wavefront(tmp_path):
                 printf("%d ", (int)(lay.state_bytes + lay.watch_bytes + lay.arena_bytes <= most));
             }""")
     assert got == ["1"] * 12
+
+
+def test_gnn_graph_of_one_large_instance_is_built_on_the_host(tmp_path):
+    """(edges of each instance, instances) on either side of the line, and the kernel's limits:
+    variables, clause length, edges."""
+    got = run_rules(tmp_path, """
+    struct { long lits; int inst, n, len; } c[] = {
+        {300, 1, 100, 3}, {8000, 1, 600, 3}, {12500, 1, 900, 3}, {12501, 1, 900, 3}, {32000, 1, 1900, 3}, {32000, 2, 1900, 3},
+        {32000, 3, 1900, 3}, {65000, 2, 1900, 3}, {65536, 3, 1984, 64}, {65537, 3, 1984, 64}, {65536, 3, 1985, 64},
+        {65536, 3, 1984, 65}};
+    for (auto& x : c) {
+        DeviceBatch d;
+        d.n_inst = x.inst; d.max_n = x.n; d.max_len = x.len; d.max_lits = x.lits; d.n_lits = x.lits * x.inst;
+        printf("%d ", (int)gnn_graph_on_device(d, d.device));
+    }""")
+    assert got == list("111000101000")
