@@ -288,20 +288,6 @@ static void packk_instance(const int32_t* lits, const int64_t* coff, int32_t m, 
     }
 }
 
-// The wide form: four 16-bit slots, in clause order (no placement pass, which would cost the
-// caller about 1 us a clause).
-static void packk_wide_instance(const int32_t* lits, const int64_t* coff, int32_t m, int32_t W, uint32_t* out)
-{
-    const uint32_t fl = 32u * (uint32_t)W + 1u;
-    for (int32_t c = 0; c < m; c++) {
-        uint32_t code[kPkkWideMaxLen] = {fl, fl, fl, fl};
-        const int len = (int)(coff[c + 1] - coff[c]);
-        for (int k = 0; k < len; k++) code[k] = (uint32_t)lits[coff[c] + k];
-        out[2 * c] = code[0] | code[1] << 16;
-        out[2 * c + 1] = code[2] | code[3] << 16;
-    }
-}
-
 int gpsat_batch_create(const int32_t* lits, const int64_t* clause_off, const int64_t* inst_clause_off,
                        const int32_t* n_vars, int32_t n_inst, gpsat_batch** out)
 {
@@ -324,6 +310,7 @@ int gpsat_batch_create(const int32_t* lits, const int64_t* clause_off, const int
     d.n_clauses = M;
     d.n_lits = L;
     d.h_meta.resize(n_inst);
+    d.h_coff.reserve(M + n_inst + (size_t)n_inst * (sizeof(InstMeta) / 4 + 2) + 8);   // (see the upload)
     d.h_coff.resize(M + n_inst);
     d.h_lits.assign(lits ? lits + l0 : nullptr, lits ? lits + l0 + L : nullptr);
     int64_t wbase = 0;
@@ -406,18 +393,15 @@ int gpsat_batch_create(const int32_t* lits, const int64_t* clause_off, const int
     const char* pf3 = getenv("GPSAT_PKK_FOR_FAST3");
     const bool use_pkk = (packk || packw) && (!d.fast3 || (pf3 && atoi(pf3) != 0)) && n_inst > 0 && M > 0;
     d.pkk_wide = use_pkk && !packk;
-    if (use_pkk) {
+    if (use_pkk && !d.pkk_wide) {
         h_pkk.resize(2 * M);
         const int32_t T = (int32_t)std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
         const int32_t nt = std::min(T, 1 + n_inst / 16);
         const auto work = [&](int32_t t) {
             for (int32_t i = t; i < n_inst; i += nt) {
                 const int64_t cb = inst_clause_off[i];
-                const int32_t m = d.h_meta[i].m, W = words_per_row(d.h_meta[i].n);
-                if (d.pkk_wide)
-                    packk_wide_instance(lits, clause_off + cb, m, W, h_pkk.data() + 2 * (cb - c0));
-                else
-                    packk_instance(lits, clause_off + cb, m, W, std::max<int>(3, h_klen[i]), h_pkk.data() + 2 * (cb - c0));
+                packk_instance(lits, clause_off + cb, d.h_meta[i].m, words_per_row(d.h_meta[i].n),
+                               std::max<int>(3, h_klen[i]), h_pkk.data() + 2 * (cb - c0));
             }
         };
         std::vector<std::thread> pool;
@@ -427,26 +411,34 @@ int gpsat_batch_create(const int32_t* lits, const int64_t* clause_off, const int
     }
     hipError_t e = hipGetDevice(&d.device);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&d.stream, hipStreamNonBlocking);
-    if (e == hipSuccess && n_inst) e = hipMalloc(&d.meta, sizeof(InstMeta) * n_inst);
-    if (e == hipSuccess && L) e = hipMalloc(&d.lits, sizeof(int32_t) * L);
-    if (e == hipSuccess && n_inst) e = hipMalloc(&d.coff, sizeof(int32_t) * (M + n_inst));
-    if (e == hipSuccess && n_inst) e = hipMemcpy(d.meta, d.h_meta.data(), sizeof(InstMeta) * n_inst, hipMemcpyHostToDevice);
-    if (e == hipSuccess && L) e = hipMemcpy(d.lits, d.h_lits.data(), sizeof(int32_t) * L, hipMemcpyHostToDevice);
-    if (e == hipSuccess && n_inst)
-        e = hipMemcpy(d.coff, d.h_coff.data(), sizeof(int32_t) * (M + n_inst), hipMemcpyHostToDevice);
-    if (e == hipSuccess && d.fast3) e = hipMalloc(&d.pk3, sizeof(uint32_t) * M);
-    if (e == hipSuccess && d.fast3) e = hipMemcpy(d.pk3, h_pk3.data(), sizeof(uint32_t) * M, hipMemcpyHostToDevice);
-    if (e == hipSuccess && use_pkk) e = hipMalloc(&d.pkk, sizeof(uint32_t) * 2 * M);
-    if (e == hipSuccess && use_pkk) e = hipMemcpy(d.pkk, h_pkk.data(), sizeof(uint32_t) * 2 * M, hipMemcpyHostToDevice);
-    if (e == hipSuccess && use_pkk) e = hipMalloc(&d.klen, n_inst);
-    if (e == hipSuccess && use_pkk) e = hipMemcpy(d.klen, h_klen.data(), n_inst, hipMemcpyHostToDevice);
-    if (e == hipSuccess && use_pkk) {
-        std::vector<int32_t> order(n_inst);
-        for (int32_t i = 0; i < n_inst; i++) order[i] = i;
+    const auto up = [&](auto*& p, const auto& src, size_t n) {
+        if (e == hipSuccess && n) e = hipMalloc(&p, sizeof(*p) * n);
+        if (e == hipSuccess && n) e = hipMemcpy(p, src.data(), sizeof(*p) * n, hipMemcpyHostToDevice);
+    };
+    // behind the offsets, in the same upload (one costs ~20 us): the instances' metadata and, for
+    // the packed kernel, the instances by decreasing cost and their longest clauses
+    const size_t at_meta = (M + n_inst + 3) / 4 * 4, at_order = at_meta + sizeof(InstMeta) / 4 * n_inst,
+                 at_klen = at_order + (use_pkk ? n_inst : 0);
+    d.h_coff.resize(n_inst ? at_klen + (use_pkk ? (n_inst + 3) / 4 : 0) : 0);
+    if (n_inst) memcpy(d.h_coff.data() + at_meta, d.h_meta.data(), sizeof(InstMeta) * n_inst);
+    if (use_pkk) {
         const auto cost = [&](int32_t i) { return (int64_t)d.h_meta[i].m * std::max<int64_t>(3, h_klen[i]); };
-        std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t c) { return cost(a) > cost(c); });
-        e = hipMalloc(&d.korder, sizeof(int32_t) * n_inst);
-        if (e == hipSuccess) e = hipMemcpy(d.korder, order.data(), sizeof(int32_t) * n_inst, hipMemcpyHostToDevice);
+        const auto order = d.h_coff.begin() + at_order;
+        for (int32_t i = 0; i < n_inst; i++) order[i] = i;
+        std::stable_sort(order, order + n_inst, [&](int32_t a, int32_t c) { return cost(a) > cost(c); });
+        memcpy(d.h_coff.data() + at_klen, h_klen.data(), n_inst);
+    }
+    up(d.coff, d.h_coff, d.h_coff.size());
+    if (e == hipSuccess && n_inst) d.meta = (InstMeta*)(d.coff + at_meta);
+    if (e == hipSuccess && use_pkk) d.korder = d.coff + at_order;
+    if (e == hipSuccess && use_pkk) d.klen = (uint8_t*)(d.coff + at_klen);
+    up(d.lits, d.h_lits, L);
+    up(d.pk3, h_pk3, h_pk3.size());
+    up(d.pkk, h_pkk, h_pkk.size());
+    if (e == hipSuccess && d.pkk_wide) {
+        e = hipMalloc(&d.pkk, sizeof(uint32_t) * 2 * M);
+        if (e == hipSuccess) e = launch_pack_wide(d, nullptr);
+        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     }
     if (e != hipSuccess) {
         set_error(std::string("batch upload: ") + hipGetErrorString(e));
@@ -462,13 +454,10 @@ int gpsat_batch_destroy(gpsat_batch* b)
     if (!b) return GPSAT_OK;
     DeviceBatch& d = b->d;
     if (d.stream) (void)hipStreamSynchronize(d.stream);
-    (void)hipFree(d.meta);
-    (void)hipFree(d.lits);
     (void)hipFree(d.coff);
+    (void)hipFree(d.lits);
     (void)hipFree(d.pk3);
     (void)hipFree(d.pkk);
-    (void)hipFree(d.klen);
-    (void)hipFree(d.korder);
     (void)hipFree(d.gtab);
     if (d.stream) (void)hipStreamDestroy(d.stream);
     delete b;

@@ -22,7 +22,7 @@ struct DeviceBatch {
     int64_t total_words = 0;      // sum of W_i (rows buffer holds A * total_words words)
     bool fast3 = false;           // every instance fits the register-resident 3-literal kernel
     bool all3 = false;            // every clause of every instance has exactly 3 literals
-    InstMeta* meta = nullptr;     // device [n_inst]
+    InstMeta* meta = nullptr;     // device [n_inst] (with klen and korder, behind coff in its memory)
     int32_t* lits = nullptr;      // device [n_lits]
     int32_t* coff = nullptr;      // device [n_clauses + n_inst], per-instance relative offsets
     // device [n_clauses] when fast3: clause c's three literal codes in bits 0-9, 10-19 and
@@ -98,6 +98,8 @@ size_t eval_bcp_lds_bytes(int max_n);
 hipError_t launch_eval_bcp(const DeviceBatch& b, const uint32_t* rows, int A, int32_t* counts, uint32_t* out_rows,
                            int32_t* conflict, int32_t* props, int32_t* passes, bool do_eval, bool do_bcp,
                            hipStream_t st, uint32_t* gtab_ext = nullptr);
+// The packed kernel's wide words of a batch (d.pkk), from its literals on the device.
+hipError_t launch_pack_wide(const DeviceBatch& d, hipStream_t st);
 // The kernel an eval/BCP launch on this batch runs under the current tuning (the kinds of
 // gpsat_batch_eval_kernel).
 enum EvalKernel { EK_FAST3 = 0, EK_PACKED = 1, EK_CSR = 2, EK_CSR_HBM = 3 };
