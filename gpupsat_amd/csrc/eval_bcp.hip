@@ -1184,7 +1184,9 @@ __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int
     // Rows of at most kPkDirect words are read by their lanes, 2 or 3 loads each: there the copy's
     // two barriers cost more than it saves (colourings of n = 120 x 3,300: staged 27.6 us, read
     // directly 26.4; mixed k-SAT of n <= 190 x 999: 18.0, 17.9).
-    const bool direct = W <= kPkDirect;
+    // So are all rows where they are only evaluated: nothing is written back, and the copy and its
+    // barriers cost 3-SAT of n = 300 x 3,000 2.6 us of 15.4.
+    const bool direct = !DO_BCP || W <= kPkDirect;
     if (!direct) {
         RowWalk walk(tid, nthreads, W);
         uint32_t* stage = tab + 63 * W;
@@ -1214,8 +1216,8 @@ __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             const int j = jb + wv + u * NW;
-            r[u] = 0u;
-            if (j < W && lane < A) r[u] = direct ? src[lane * W + j] : tab[63 * W + 65 * j + lane];
+            if (direct) r[u] = (j < W && lane < A) ? src[lane * W + j] : 0u;
+            else r[u] = (j < W && lane < A) ? tab[63 * W + 65 * j + lane] : 0u;
         }
         if (!direct) __syncthreads();
 #pragma unroll
