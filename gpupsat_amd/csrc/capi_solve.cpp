@@ -162,19 +162,16 @@ int solve_plan(const DeviceBatch& d, const gpsat_solve_opts& o, int32_t n_jobs, 
         const int per_cu = (int)std::max<size_t>(1, std::min<size_t>(most, per_cu_lds));
         waves = prop.multiProcessorCount * per_cu;
     }
-    p.wpb = solve_waves_per_block(p.lds_bytes);
     p.req_chunk = o.chunk;
     p.n_jobs = n_jobs;
     set_waves(p, waves);
     return GPSAT_OK;
 }
 
-// Persistent wavefronts (at most one per job, whole workgroups: surplus wavefronts find
-// the queue empty and exit) and the chunk that goes with them.
+// Persistent wavefronts (at most one per job) and the chunk that goes with them.
 void set_waves(SolvePlan& p, int waves)
 {
-    waves = std::max(1, std::min(waves, std::max(p.n_jobs, 1)));
-    p.waves = (waves + p.wpb - 1) / p.wpb * p.wpb;
+    p.waves = std::max(1, std::min(waves, std::max(p.n_jobs, 1)));
     // chunks of consecutive jobs let cubes of one instance reuse its watch lists; a few
     // chunks per wavefront keep the queue balanced
     p.chunk = (int32_t)std::max<int64_t>(1, std::min<int64_t>(64, (int64_t)p.n_jobs / ((int64_t)p.waves * 4)));

@@ -1415,7 +1415,7 @@ __device__ __forceinline__ void eval_bcpk_body(const InstMeta& mi, int inst, int
                 fz |= __hip_atomic_load(sh_fz, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 uint32_t chg = 0;
                 const auto imply = [&](const PkGroup32<K, WIDE>& gr) {
-                        uint32_t T, N0, N1;
+                    uint32_t T, N0, N1;
                     pk_status32(gr, T, N0, N1);
                     const uint32_t newconf = andn2(N0, T, fz);
                     const uint32_t U = andn2(N1, T, fz);

@@ -867,7 +867,7 @@ using namespace gpsat;
 using namespace gpsat::gnn;
 
 // Workgroups of the weight-gradient products (one partial matrix each; two workgroups per CU, as
-// more of them write more partials and gain nothing) and of the embedding gradient.
+// more of them write more partials and gain nothing).
 constexpr int DW_BLOCKS = 512;
 constexpr int MAX_GROUPS = 32;
 

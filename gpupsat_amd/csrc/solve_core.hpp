@@ -187,8 +187,8 @@ inline int solve_core(gpsat_batch* b, const gpsat_solve_opts& o, const int32_t* 
         // the workspace slices come last: a fixed region holds as many as are left room for
         const size_t slice = 4 * (size_t)a.ws_ints_per_wave;
         if ((size_t)plan.waves * slice > mem.remaining()) {
-            const int fit = (int)(mem.remaining() / slice) / plan.wpb * plan.wpb;
-            if (fit < plan.wpb) {
+            const int fit = (int)(mem.remaining() / slice);
+            if (fit < 1) {
                 set_error("gpsat_solve_noalloc: the solver workspace does not fit the scratch region");
                 return GPSAT_ERR_CAPACITY;
             }
@@ -196,9 +196,9 @@ inline int solve_core(gpsat_batch* b, const gpsat_solve_opts& o, const int32_t* 
         }
         hipError_t we = mem.alloc(d_ws, (size_t)plan.waves * a.ws_ints_per_wave);
         // a large formula's slices may not all fit the GPU: then the jobs share fewer wavefronts
-        while (!Mem::kNoAlloc && we == hipErrorOutOfMemory && plan.waves > plan.wpb) {
+        while (!Mem::kNoAlloc && we == hipErrorOutOfMemory && plan.waves > 1) {
             (void)hipGetLastError();
-            set_waves(plan, plan.waves / 2 / plan.wpb * plan.wpb);
+            set_waves(plan, plan.waves / 2);
             we = mem.alloc(d_ws, (size_t)plan.waves * a.ws_ints_per_wave);
         }
         HIP_OR(we);

@@ -199,9 +199,12 @@ struct Search {
     int64_t conflicts, decisions, props, learned, restarts;
     int32_t levelmax;
 
-    // Orders this wavefront's accesses across its lanes.  LDS requests of one wavefront are
-    // served in order, so with the state in LDS only the compiler has to be held; state in this
-    // wavefront's HBM slice also waits for its outstanding memory operations.
+    // Orders this wavefront's accesses across its lanes.  What one wavefront issues to an address,
+    // loads, stores and atomics, takes effect there in the order it was issued, in LDS as in its HBM
+    // slice (all go through one CU's path to memory; the wavefront scope of the memory model needs
+    // no wait either), and no other wavefront touches the slice during a job.  So only the compiler
+    // has to be held.  msync also waits for what is outstanding: the steps that rewrite whole arrays
+    // (set-up, reductions, a new learned clause) use it, where it is not measurable; none needs it.
     static __device__ __forceinline__ void lsync() { wave_sync(); }
     static __device__ __forceinline__ void msync()
     {
@@ -1285,6 +1288,8 @@ struct Search {
             }
         }
         dups = ballot(twice) != 0;
+        // (a list longer than a wavefront or a watch_slack above 64 makes the instance take
+        // propagate_long: 2,000 x n=120 at a slack of 100 137 ms, at 16 76)
         shortl = ballot(longl) == 0;
         if (!ALL3)
             for (int32_t v = lane; v < n + 2; v += kWave) lstamp[v] = 0;
@@ -1502,17 +1507,12 @@ struct Search {
 // literals in HBM; 4 everything in the HBM slice (formulas whose per-var state does not fit a
 // workgroup's LDS).
 template <int kMode, class I, bool ALL3>
-__global__ __launch_bounds__(kSolveWavesPerBlock * kWave) __attribute__((amdgpu_waves_per_eu(solve_waves_per_eu(kMode), solve_waves_per_eu(kMode))))
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(solve_waves_per_eu(kMode), solve_waves_per_eu(kMode))))
 void k_solve(SolveArgs a)
 {
-    extern __shared__ __align__(16) char smem_all[];
+    extern __shared__ __align__(16) char smem[];
     const int lane = lane_id();
-    // the wavefronts of a workgroup are independent (separate jobs, private LDS regions,
-    // wave-level ordering only)
-    const int wslot = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-    const int64_t gwave = (int64_t)blockIdx.x * (blockDim.x / kWave) + wslot;
-    char* smem = smem_all + (uint32_t)wslot * (uint32_t)a.lds_per_wave;
-    char* slice = (char*)(a.ws + gwave * a.ws_ints_per_wave);
+    char* slice = (char*)(a.ws + (int64_t)blockIdx.x * a.ws_ints_per_wave);
     Search<kMode, I, ALL3> J;
     if (kMode == 4) J.carve(slice, slice + a.lay.state_bytes, slice + a.lay.state_bytes + a.lay.watch_bytes, a);
     else if (kMode == 2) J.carve(smem, slice, slice + a.lay.watch_bytes, a);
@@ -1736,11 +1736,9 @@ static void launch_mode(const SolveArgs& a, int mode, dim3 grid, dim3 block, siz
 
 hipError_t launch_solve(const SolveArgs& a, int clause_mem, int waves, size_t lds_bytes, hipStream_t st)
 {
-    // waves is a multiple of the wavefronts per workgroup (solve_waves_per_block)
-    const int wpb = solve_waves_per_block(lds_bytes);
-    if (waves % wpb != 0 || (size_t)a.lds_per_wave != lds_bytes) return hipErrorInvalidValue;
-    const dim3 grid(waves / wpb), block(kWave * wpb);
-    const size_t lds = lds_bytes * wpb;
+    if ((size_t)a.lds_per_wave != lds_bytes) return hipErrorInvalidValue;
+    const dim3 grid(waves), block(kWave);   // a workgroup per wavefront
+    const size_t lds = lds_bytes;
     const bool ids16 = a.lay.id_bytes == 2;
     if (clause_mem == 4 && a.all3)
         hipLaunchKernelGGL((k_solve<4, uint32_t, true>), grid, block, 0, st, a);
@@ -1755,13 +1753,6 @@ hipError_t launch_solve(const SolveArgs& a, int clause_mem, int waves, size_t ld
     else
         launch_mode<false>(a, clause_mem, grid, block, lds, st);
     return hipGetLastError();
-}
-
-int solve_waves_per_block(size_t lds_bytes)
-{
-    int wpb = kSolveWavesPerBlock;
-    while (wpb > 1 && (size_t)wpb * lds_bytes > 64 * 1024) wpb >>= 1;
-    return wpb;
 }
 
 }  // namespace gpsat

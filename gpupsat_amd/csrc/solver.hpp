@@ -9,9 +9,8 @@ namespace gpsat {
 
 // Solver options (the strategy surfaces of the reference's compile-time Configs.cuh,
 // chosen at run time here).
-// k_solve launch shape: independent wavefronts per workgroup, and the wavefronts per SIMD
-// the register allocation is held to (8 -> at most 64 VGPRs per lane, 4 -> 128)
-constexpr int kSolveWavesPerBlock = 1;
+// k_solve launch shape (a workgroup is one wavefront): the wavefronts per SIMD the register
+// allocation is held to (8 -> at most 64 VGPRs per lane, 4 -> 128)
 constexpr int solve_waves_per_eu(int mode) { return mode == 1 || mode == 3 ? 4 : 8; }
 
 struct SolveOptsDev {
@@ -131,7 +130,6 @@ struct SolvePlan {
     int mode;
     int waves;
     int chunk;
-    int wpb;             // wavefronts per workgroup
     int req_chunk;       // the caller's chunk (0: automatic)
     int32_t n_jobs;
     int cus;
@@ -141,7 +139,6 @@ struct SolvePlan {
 hipError_t launch_epoch_begin(const SolveArgs& a, hipStream_t st);
 hipError_t launch_epoch_end(const SolveArgs& a, int32_t* remaining, hipStream_t st);
 hipError_t launch_solve(const SolveArgs& a, int clause_mem, int waves, size_t lds_bytes, hipStream_t st);
-int solve_waves_per_block(size_t lds_bytes);
 
 }  // namespace gpsat
 

@@ -203,7 +203,9 @@ typedef struct gpsat_solve_opts {
                                 lists and clause records in LDS, the learned clauses' literals in
                                 HBM, 4 the whole job state in HBM.  Automatic: with at most 4 jobs
                                 per CU, LDS, else split, else HBM, whichever fits first; with more,
-                                whichever is estimated to finish the jobs first */
+                                whichever is estimated to finish the jobs first.  1 and 3 become 2
+                                where they do not fit, or where clause ids (original and learned)
+                                need more than 16 bits; gpsat_solve_info says what ran */
     int32_t verify;          /* 1: re-check every SAT model with the clause-evaluation kernel */
     int32_t chunk;           /* jobs per queue grab (0: automatic); cubes of one instance in one
                                 chunk reuse its watch lists on the wavefront */

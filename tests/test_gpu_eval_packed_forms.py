@@ -1,6 +1,6 @@
-"""The packed evaluation kernel's forms: wide slots (n above 496), and the sweeps over clauses
-of at most two literals, at the sizes where the rule changes form and at the edges of their
-64-clause groups -- equal to the oracle and to the CSR kernel."""
+"""The packed evaluation kernel's forms: wide slots (n above 496) and 10-bit ones, at the sizes
+where the rule changes form, at the edges of their 64-clause groups and at the lengths where rows
+are read another way -- equal to the oracle and to the CSR kernel."""
 import numpy as np
 import pytest
 

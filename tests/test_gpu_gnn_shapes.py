@@ -1,5 +1,5 @@
-"""The branching network's layers at the edges of their tiles (16 rows a wavefront, 64 a
-workgroup, neighbours read in fours) and for every form of the first and last round, against
+"""The branching network's layers at the edges of their tiles (16 rows a wavefront, 128 or, in the
+first round backward, 64 a workgroup, neighbours read in fours) and for every form of the first and last round, against
 the CPU FP64 oracle with the same BF16 rounding points."""
 import numpy as np
 import pytest
