@@ -129,9 +129,10 @@ template <> struct Hdr<uint32_t> {
 //    reason; the per-job state shrinks enough to hold the watch structures in LDS.  With 32-bit
 //    ids (kShared: formulas whose watch structures are in HBM at any size) a wavefront keeps a
 //    clause's two watches (or one unwatched literal of three) only and reads its literals from the
-//    batch's arrays, which all wavefronts share: 16 to 20 bytes per 3-literal clause instead of the 52 of records and literals of
-//    its own, with which 8,192 wavefronts had room for 0.42 M clauses instead of 0.7 M, and 1,024
-//    cubes of 66,000 clauses over 2,000 variables took 73.7 ms instead of 60.2.
+//    batch's arrays, which all wavefronts share: 16 bytes per 3-literal clause (20 in a mixed
+//    formula) instead of the 52 of records and literals of its own, with which 8,192 wavefronts
+//    had room for 0.42 M clauses instead of 0.7 M, and 1,024 cubes of 66,000 clauses over 2,000
+//    variables took 73.7 ms instead of 46.6.
 //  * both watch lists of a literal are walked in one pass of the wavefront, one entry per lane,
 //    and the next literal's header and entries are fetched while the current one is processed
 //    (a queued literal's negation is false, so nothing moves a watch to its lists meanwhile).

@@ -273,7 +273,8 @@ int gpsat_solve(gpsat_batch *b, const gpsat_solve_opts *o, const int32_t *job_in
  * solver workspace, the model check's counts) is carved from one static device region of
  * GPSAT_NOALLOC_SCRATCH_MIB MiB per GPU, which the library holds until the process ends; no
  * hipMalloc, hipFree or pinned allocation is made.  When the clause part of the job state
- * sits in HBM, fewer persistent wavefronts are launched if their slices would not fit.  A call
+ * sits in HBM, fewer persistent wavefronts are launched if their slices would not fit; the
+ * automatic placement keeps all of it in LDS if that runs more.  A call
  * whose buffers exceed the region returns GPSAT_ERR_CAPACITY before anything runs; restart
  * epochs (epoch_conflicts > 0) and the learned-clause dump return GPSAT_ERR_ARG.  Every call
  * on a GPU shares that GPU's region: calls that overlap on one GPU race. */
